@@ -232,6 +232,12 @@ int picard_timing_kernel_clock(picard_ctx *ctx, double *jacobi_ms, int64_t *jaco
  * the last picard_timing_enable, and the number of solves timed.  No
  * reference counterpart (the reference calls no timer). */
 int picard_timing_solve(picard_ctx *ctx, double *solve_ms, int64_t *solves);
+/* By default the FP32-split form (and the FP64 form with
+ * PICARD_DEPOSIT_FIXED_POINT) takes the field solve to a few iterates before
+ * its stop in closed form, in FP64, and sweeps from there; the iterate and the
+ * sweep count are those of sweeping all the way, to FP64 rounding.  On a
+ * context on which one of the next two functions was called the split form
+ * sweeps all the way, as they say. */
 /* FP32-split solve: `inner` FP32 sweeps per FP64 refinement step, 2..512
  * (default 512); other values return PICARD_ERR_ARG.  No reference
  * counterpart; the solution agrees with the FP64 form's to the split form's

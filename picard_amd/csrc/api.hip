@@ -127,6 +127,7 @@ void release(picard_ctx *c) {
   dfree(c->C);
   dfree(c->D);
   bcpot_fft_release(c);
+  spec_release(c);
   dfree(c->haser_off);
   dfree(c->F);
   dfree(c->Fraw);
@@ -227,11 +228,11 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   PICARD_TRY(dalloc(&c->D, DN));
   // the Jacobi iterates and b start one element into their allocations, so
   // that node pairs (i, i+1) with i even are 16-byte aligned when nx is even
-  if (!c->split)
-    for (int q = 0; q < 3; ++q) {
-      PICARD_TRY(dalloc(&c->jb_mem[q], g.G + 2));
-      c->jb[q] = c->jb_mem[q] + 1;
-    }
+  for (int q = 0; q < 3; ++q) {
+    PICARD_TRY(dalloc(&c->jb_mem[q], g.G + 2));
+    c->jb[q] = c->jb_mem[q] + 1;
+  }
+  if (spec_eligible(c)) PICARD_TRY(spec_create(c));
   PICARD_TRY(dalloc(&c->b_mem, g.G + 2));
   c->b = c->b_mem + 1;
   PICARD_TRY(dalloc(&c->consts, 16));
@@ -649,6 +650,7 @@ int picard_split_solver(picard_ctx *c, int32_t inner) {
     return PICARD_ERR_ARG;
   }
   c->mx_inner = inner;
+  c->mx_forced = true;
   return PICARD_OK;
 }
 
@@ -661,6 +663,7 @@ int picard_split_sweeps_per_launch(picard_ctx *c, int32_t sweeps) {
   }
   c->mx_pairs = sweeps >= 2;
   c->mx_triples = sweeps == 3;
+  c->mx_forced = true;
   return PICARD_OK;
 }
 

@@ -554,7 +554,8 @@ __global__ void __launch_bounds__(256) k_charge_yfirst(GridDims g, const double 
 // interior at the wrapped position, and iterate 0 keeps whatever halo U came
 // in with; flow faces keep their input values throughout.
 //
-// Pass p computes U_p = J(U_{p-1}) and, for p >= 2, the residual r_{p-1} of
+// Pass p computes U_p = J(U_{p-1}) and, for p > p0 (the first pass of the
+// solve, or of its part after the eigenbasis step), the residual r_{p-1} of
 // U_{p-1}, which the reference evaluates with the halo of U_{p-2} ("stale"
 // halo: CalcEpotential.f90:83-92 runs before the exchange of :100-239).  The
 // last block to finish a pass reduces the block sums in a fixed order and
@@ -634,7 +635,7 @@ __global__ void __launch_bounds__(kStencilT, 8) k_jacobi_pass(PassGeo pg, Jacobi
                                                      double *b2, const double *__restrict__ b,
                                                      const double *__restrict__ Pin,
                                                      double *__restrict__ Pout, JacobiState *st,
-                                                     int32_t p, unsigned long long *ks) {
+                                                     int32_t p, int32_t p0, unsigned long long *ks) {
   __shared__ double sh[kStencilT / 64];
   __shared__ int decide;
   kstamp_begin(ks);
@@ -644,7 +645,7 @@ __global__ void __launch_bounds__(kStencilT, 8) k_jacobi_pass(PassGeo pg, Jacobi
   // iteration ss = p-1 on the residual of U_{p-2} (partials of launch p-1)
   StopSlot cur = prev;
   if (!prev.done) {
-    if (p >= 3) {
+    if (p >= p0 + 2) {
       const double S = sum_partials(Pin, (int)gridDim.x, sh);
       if (t0 == 0) decide = (p - 1 <= st->maxit && sqrt(S) <= st->thresh) ? 1 : 0;
       __syncthreads();
@@ -667,7 +668,7 @@ __global__ void __launch_bounds__(kStencilT, 8) k_jacobi_pass(PassGeo pg, Jacobi
   const int r = p % 3;
   const double *curb = r == 1 ? b0 : (r == 2 ? b1 : b2);           // U_{p-1} in bufs[(p-1)%3]
   double *out = r == 0 ? b0 : (r == 1 ? b1 : b2);                  // U_p in bufs[p%3]
-  const double *old = p >= 2 ? (r == 2 ? b0 : (r == 0 ? b1 : b2)) : nullptr;   // U_{p-2}
+  const double *old = p > p0 ? (r == 2 ? b0 : (r == 0 ? b1 : b2)) : nullptr;   // U_{p-2}
   const bool wrap_cur = (p - 1) >= 1;              // halo of U_{p-1} = wrapped interior
   const bool wrap_old = (p - 2) >= 1;
   const bool px = pg.px, py = pg.py, pz = pg.pz;
@@ -709,7 +710,7 @@ __global__ void __launch_bounds__(kStencilT, 8) k_jacobi_pass(PassGeo pg, Jacobi
       const double bc = b[c];
       // CalcEpotential.f90:74-80
       out[c] = jc.ax * (ue + uw) + jc.ay * (un + us) + jc.az * (ut + ub) - jc.af * bc;
-      if (p >= 2) {
+      if (p > p0) {
         // residual of U_{p-1} with the halo of U_{p-2}: periodic guard
         // neighbours come from `old` (wrapped, or the stored input halo at p-2 = 0)
         double re = ue, rw = uw, rn = un, rs = us, rt = ut, rb = ub;
@@ -766,7 +767,7 @@ __global__ void __launch_bounds__(kStencilT, 4) k_jacobi_pass2(PassGeo pg, Jacob
                                                        const double *__restrict__ b,
                                                        const double *__restrict__ Pin,
                                                        double *__restrict__ Pout, JacobiState *st,
-                                                       int32_t p, unsigned long long *ks) {
+                                                       int32_t p, int32_t p0, unsigned long long *ks) {
   __shared__ double sh[kStencilT / 64];
   __shared__ int decide;
   kstamp_begin(ks);
@@ -774,7 +775,7 @@ __global__ void __launch_bounds__(kStencilT, 4) k_jacobi_pass2(PassGeo pg, Jacob
   const int t0 = lin_tid();
   StopSlot cur = prev;
   if (!prev.done) {
-    if (p >= 3) {
+    if (p >= p0 + 2) {
       const double S = sum_partials(Pin, (int)gridDim.x, sh);
       if (t0 == 0) decide = (p - 1 <= st->maxit && sqrt(S) <= st->thresh) ? 1 : 0;
       __syncthreads();
@@ -797,10 +798,10 @@ __global__ void __launch_bounds__(kStencilT, 4) k_jacobi_pass2(PassGeo pg, Jacob
   const int r = p % 3;
   const double *curb = r == 1 ? b0 : (r == 2 ? b1 : b2);           // U_{p-1} in bufs[(p-1)%3]
   double *out = r == 0 ? b0 : (r == 1 ? b1 : b2);                  // U_p in bufs[p%3]
-  const double *old = p >= 2 ? (r == 2 ? b0 : (r == 0 ? b1 : b2)) : nullptr;   // U_{p-2}
+  const double *old = p > p0 ? (r == 2 ? b0 : (r == 0 ? b1 : b2)) : nullptr;   // U_{p-2}
   const bool wrap_cur = (p - 1) >= 1;              // halo of U_{p-1} = wrapped interior
   const bool wrap_old = (p - 2) >= 1;
-  const bool res = p >= 2;
+  const bool res = p > p0;
   const bool py = pg.py, pz = pg.pz;
   const uint32_t X = pg.X, XY = pg.XY;
   const int nx = pg.nx, ny = pg.ny, nz = pg.nz;
@@ -1272,12 +1273,16 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
   init.pass = 1;
   init.maxit = maxit;
   init.last = 2 * (int64_t)maxit + 1;
-  PICARD_HIP(hipMemcpyAsync(c->js, &init, sizeof(JacobiState), hipMemcpyHostToDevice, c->stream));
-  for (int q = 0; q < 3; ++q)
-    PICARD_HIP(hipMemcpyAsync(c->jb[q], c->U, sizeof(double) * g.G, hipMemcpyDeviceToDevice,
-                              c->stream));
+  const int64_t last = init.last;
   const int nbn = grid_blocks(g.G, kT);
-  PICARD_TRY(launch_bnorm(c, maxerr));
+  // b, |b| and the buffers of iterate 0
+  auto begin = [&]() -> int {
+    PICARD_HIP(hipMemcpyAsync(c->js, &init, sizeof(JacobiState), hipMemcpyHostToDevice, c->stream));
+    for (int q = 0; q < 3; ++q)
+      PICARD_HIP(hipMemcpyAsync(c->jb[q], c->U, sizeof(double) * g.G, hipMemcpyDeviceToDevice,
+                                c->stream));
+    return launch_bnorm(c, maxerr);
+  };
 
   // even nx: two cells per lane, tiles of 128 x 4 cells
   const bool two = g.nx % 2 == 0;
@@ -1325,70 +1330,101 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
   pg.XY = (uint32_t)g.X * (uint32_t)g.Y;
   pg.px = !g.flow[0]; pg.py = !g.flow[1]; pg.pz = !g.flow[2];
   pg.ntx = ts.ntx; pg.TP = ts.TP; pg.W = ts.W;
-  const int64_t last = init.last;
   double *P[2] = {c->s.partials, c->s.partials + c->s.partials_len};
-  int64_t p = 1;                  // next pass (launch number)
-  // first batch from the previous solve's count (cold starts are alike from
-  // step to step), then short batches: few no-op passes after convergence
-  int64_t batch = c->last_sweeps > 64 ? (c->last_sweeps * 15) / 16 : 32;
-  const int64_t kMaxBatch = int64_t(1) << 16;
-  if (batch > kMaxBatch) batch = kMaxBatch;
+  auto pass = [&](int64_t p, int64_t first, hipEvent_t e0, hipEvent_t e1, unsigned long long *ks) {
+    const double *pin = P[(p - 1) & 1];
+    if (two && g.flow[0])
+      hipExtLaunchKernelGGL(k_jacobi_pass2<false>, dim3(ts.B), dim3(ts.bx, ts.by), 0, c->stream,
+                            e0, e1, 0, pg, jc, c->jb[0], c->jb[1], c->jb[2],
+                            (const double *)c->b, pin, P[p & 1], c->js, (int32_t)p,
+                            (int32_t)first, ks);
+    else if (two)
+      hipExtLaunchKernelGGL(k_jacobi_pass2<true>, dim3(ts.B), dim3(ts.bx, ts.by), 0, c->stream,
+                            e0, e1, 0, pg, jc, c->jb[0], c->jb[1], c->jb[2],
+                            (const double *)c->b, pin, P[p & 1], c->js, (int32_t)p,
+                            (int32_t)first, ks);
+    else
+      hipExtLaunchKernelGGL(k_jacobi_pass, dim3(ts.B), dim3(ts.bx, ts.by), 0, c->stream,
+                            e0, e1, 0, pg, jc, c->jb[0], c->jb[1], c->jb[2],
+                            (const double *)c->b, pin, P[p & 1], c->js, (int32_t)p,
+                            (int32_t)first, ks);
+  };
   StopSlot fin{};
-  for (;;) {
-    const int64_t todo = (last + 1 - (p - 1)) < batch ? (last + 1 - (p - 1)) : batch;
-    // timing: one pass in kTimeEvery, with dispatch-packet events around it
-    // and the kernel's own clock stamps (events around every pass would slow
-    // the timed solve itself)
-    int64_t timed = (todo + kTimeEvery / 2 - 1) / kTimeEvery;         // passes q = 8, 24, ...
-    if (timed > picard_ctx::kStamps) timed = picard_ctx::kStamps;
-    if (c->timing) {
-      while ((int64_t)c->tev.size() < 2 * timed) {
-        hipEvent_t e;
-        PICARD_HIP(hipEventCreate(&e));
-        c->tev.push_back(e);
+  // passes p, p + 1, ... to the end of the solve, the first of the sweeps being `first`
+  auto sweep = [&](int64_t p, int64_t first, int64_t batch) -> int {
+    for (;;) {
+      const int64_t todo = (last + 1 - (p - 1)) < batch ? (last + 1 - (p - 1)) : batch;
+      // timing: one pass in kTimeEvery, with dispatch-packet events around it
+      // and the kernel's own clock stamps (events around every pass would slow
+      // the timed solve itself)
+      int64_t timed = (todo + kTimeEvery / 2 - 1) / kTimeEvery;         // passes q = 8, 24, ...
+      if (timed > picard_ctx::kStamps) timed = picard_ctx::kStamps;
+      if (c->timing) {
+        while ((int64_t)c->tev.size() < 2 * timed) {
+          hipEvent_t e;
+          PICARD_HIP(hipEventCreate(&e));
+          c->tev.push_back(e);
+        }
+        PICARD_TRY(kstamp_reset(c, (int)timed));
       }
-      PICARD_TRY(kstamp_reset(c, (int)timed));
-    }
-    for (int64_t q = 0; q < todo; ++q, ++p) {
-      const bool stamp = c->timing && q % kTimeEvery == kTimeEvery / 2 && q / kTimeEvery < timed;
-      unsigned long long *ks = stamp ? c->kst + picard_ctx::kStampWords * (q / kTimeEvery) : nullptr;
-      hipEvent_t e0 = stamp ? c->tev[2 * (q / kTimeEvery)] : nullptr;
-      hipEvent_t e1 = stamp ? c->tev[2 * (q / kTimeEvery) + 1] : nullptr;
-      const double *pin = P[(p - 1) & 1];
-      if (two && g.flow[0])
-        hipExtLaunchKernelGGL(k_jacobi_pass2<false>, dim3(ts.B), dim3(ts.bx, ts.by), 0, c->stream,
-                              e0, e1, 0, pg, jc, c->jb[0], c->jb[1], c->jb[2],
-                              (const double *)c->b, pin, P[p & 1], c->js, (int32_t)p, ks);
-      else if (two)
-        hipExtLaunchKernelGGL(k_jacobi_pass2<true>, dim3(ts.B), dim3(ts.bx, ts.by), 0, c->stream,
-                              e0, e1, 0, pg, jc, c->jb[0], c->jb[1], c->jb[2],
-                              (const double *)c->b, pin, P[p & 1], c->js, (int32_t)p, ks);
-      else
-        hipExtLaunchKernelGGL(k_jacobi_pass, dim3(ts.B), dim3(ts.bx, ts.by), 0, c->stream,
-                              e0, e1, 0, pg, jc, c->jb[0], c->jb[1], c->jb[2],
-                              (const double *)c->b, pin, P[p & 1], c->js, (int32_t)p, ks);
-    }
-    PICARD_HIP(hipGetLastError());
-    PICARD_HIP(hipMemcpyAsync(c->js_host, c->js, sizeof(JacobiState), hipMemcpyDeviceToHost,
-                              c->stream));
-    PICARD_HIP(hipStreamSynchronize(c->stream));
-    if (c->timing) {
-      for (int64_t q = 0; q < timed; ++q) {
-        float ms = 0.0f;
-        PICARD_HIP(hipEventElapsedTime(&ms, c->tev[2 * q], c->tev[2 * q + 1]));
-        c->t_ms += ms;
+      for (int64_t q = 0; q < todo; ++q, ++p) {
+        const bool stamp = c->timing && q % kTimeEvery == kTimeEvery / 2 && q / kTimeEvery < timed;
+        unsigned long long *ks = stamp ? c->kst + picard_ctx::kStampWords * (q / kTimeEvery) : nullptr;
+        hipEvent_t e0 = stamp ? c->tev[2 * (q / kTimeEvery)] : nullptr;
+        hipEvent_t e1 = stamp ? c->tev[2 * (q / kTimeEvery) + 1] : nullptr;
+        pass(p, first, e0, e1, ks);
       }
-      c->t_launches += timed;
-      c->t_sweeps += timed;
-      PICARD_TRY(kstamp_collect(c, (int)timed));
+      PICARD_HIP(hipGetLastError());
+      PICARD_HIP(hipMemcpyAsync(c->js_host, c->js, sizeof(JacobiState), hipMemcpyDeviceToHost,
+                                c->stream));
+      PICARD_HIP(hipStreamSynchronize(c->stream));
+      if (c->timing) {
+        for (int64_t q = 0; q < timed; ++q) {
+          float ms = 0.0f;
+          PICARD_HIP(hipEventElapsedTime(&ms, c->tev[2 * q], c->tev[2 * q + 1]));
+          c->t_ms += ms;
+        }
+        c->t_launches += timed;
+        c->t_sweeps += timed;
+        PICARD_TRY(kstamp_collect(c, (int)timed));
+      }
+      fin = c->js_host->slot[(p - 1) & 1];
+      if (fin.done) return PICARD_OK;
+      if (p > last + 1) {
+        set_error("CalcEpotential: pass accounting out of step");
+        return PICARD_ERR_STATE;
+      }
+      batch = 64;
     }
-    fin = c->js_host->slot[(p - 1) & 1];
-    if (fin.done) break;
-    if (p > last + 1) {
-      set_error("CalcEpotential: pass accounting out of step");
-      return PICARD_ERR_STATE;
+  };
+  bool done = false, few = false;
+  if (spec_eligible(c) && last > 64) {
+    // the eigenbasis step to a few iterates before the stop, then the sweeps
+    // with the stop test; a solve that passes one of the first two tests may
+    // have been taken past its stop and starts again with a wider margin
+    for (int margin = 4; !done && margin <= 1024; margin *= 16) {
+      PICARD_TRY(begin());
+      // the order-free form's first sweep reads the halo U came in with
+      const int64_t base = c->order_free ? 1 : 0;
+      if (base) pass(1, 1, nullptr, nullptr, nullptr);
+      int64_t to = -1;
+      PICARD_TRY(spec_step(c, base ? c->jb[1] : c->U, base, margin, &to));
+      if (to < 0) {
+        if (c->split) return kNoSpecStep;
+        few = to == -1;
+        break;
+      }
+      PICARD_TRY(sweep(to + 1, to + 1, margin + 5));
+      done = fin.result == last || fin.result > to + 2;
     }
-    batch = 64;
+  }
+  if (!done) {
+    PICARD_TRY(begin());
+    // first batch from the previous solve's count (cold starts are alike from
+    // step to step), then short batches: few no-op passes after convergence
+    const int64_t kMaxBatch = int64_t(1) << 16;
+    const int64_t batch = !few && c->last_sweeps > 64 ? (c->last_sweeps * 15) / 16 : 32;
+    PICARD_TRY(sweep(1, 1, batch < kMaxBatch ? batch : kMaxBatch));
   }
   c->last_sweeps = fin.result;
   k_jacobi_finish<<<nbn, kT, 0, c->stream>>>(g, c->jb[0], c->jb[1], c->jb[2], c->U, fin.result);

@@ -108,6 +108,8 @@ struct DeviceScratch {
   int64_t partials_len = 0;
 };
 
+struct SpecState;                  // spectral.hip
+
 }  // namespace picard
 
 struct picard_ctx {
@@ -132,6 +134,7 @@ struct picard_ctx {
   float *r32 = nullptr, *e32[2] = {nullptr, nullptr};
   float *eo32[4] = {nullptr, nullptr, nullptr, nullptr};
   int mx_inner = 512;        // split: FP32 sweeps per FP64 refinement
+  bool mx_forced = false;    // split: the caller chose how to sweep, so the solve sweeps all the way
   bool mx_pairs = true;      // split: two sweeps per launch where the grid allows
   bool mx_triples = false;   // split: three sweeps per launch where the grid allows
   int pair_wmax = 0;         // split: resident blocks per XCD of the two-sweep kernel
@@ -165,6 +168,14 @@ struct picard_ctx {
   double2 *fft_work = nullptr;   // transformed charge planes + two face accumulators
   int64_t fft_work_len = 0;
   bool fft_ready = false;
+
+  // split and order-free FP64 forms: the solve's eigenbasis step (spectral.hip)
+  double *spec_buf[3] = {nullptr, nullptr, nullptr};   // padded interior arrays
+  double *spec_fwd[3] = {nullptr, nullptr, nullptr};   // per axis: basis, its transpose,
+  double *spec_inv[3] = {nullptr, nullptr, nullptr};
+  double *spec_eig[3] = {nullptr, nullptr, nullptr};   // and eigenvalue parts
+  double spec_lnmax = 0.0;                             // largest ln|lambda|
+  picard::SpecState *spec_st = nullptr, *spec_host = nullptr;
 
   // number fluxes of ParticlesGridifyAll (allocated on first use)
   double *F = nullptr;                 // F(species, 3, node)
@@ -245,9 +256,18 @@ int launch_bnorm(picard_ctx *c, double maxerr);
 int launch_gridify(picard_ctx *c, bool flux = false);
 int launch_calc_distance(picard_ctx *c);
 int launch_bc_potentials(picard_ctx *c);
+// kNoSpecStep (split form only): no eigenbasis step was taken and U is as it
+// was; the caller solves by its own sweeps
+constexpr int kNoSpecStep = 1000;
 int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t *sweeps);
 int launch_calc_efield(picard_ctx *c);
 int launch_bc_fields(picard_ctx *c);
+
+// ---- spectral.hip ----
+bool spec_eligible(const picard_ctx *c);
+int spec_create(picard_ctx *c);
+void spec_release(picard_ctx *c);
+int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, int64_t *to);
 
 // ---- diag.hip ----
 int diagnostics(picard_ctx *c, const double *mass, picard_diag *out);

@@ -1,0 +1,464 @@
+// spectral.hip -- the Jacobi solve's long middle in closed form, for the forms
+// that are not held to the reference's rounding (FP32-split, and FP64 with the
+// order-free deposit).
+//
+// CalcEpotential.f90:58-92 is a linear iteration: with r_b the residual of
+// iterate b, U_p = U_b - af sum_{i < p-b} J^i r_b and r_p = J^{p-b} r_b.  J is
+// diagonal in the product of the axes' eigenbases (spectral.h), so one transform of r_b gives
+// every later iterate and the norm of its residual.  The solve transforms r_b,
+// finds the iterate the stop rule will pick, goes to a few iterates before it
+// in one step and leaves the rest, with the stop test itself, to the sweeps
+// (grid.hip): the iterate returned and its count are those of sweeping all the way, to FP64
+// rounding.
+//
+// The stop rule's residual takes the previous iterate's values across periodic
+// boundaries (CalcEpotential.f90:83-92), which makes it J0 r_{p-1}: one Jacobi
+// step of the plain residual with zeros beyond every boundary.  Its norm is
+// not a sum over eigenvectors, so the search finds the crossing of the plain
+// norm first, evaluates the rule's own norm there in space, and corrects by
+// the slope.
+//
+// Cost: nine axis transforms of 2 n operations a cell, whatever the number of
+// sweeps (about 3 n^2 to 1e-6).  Measured, whole solve with its last sweeps
+// against sweeping: 16^3 0.29 ms (FP32 sweeps 7.3), 64^3 0.5 ms (FP64 sweeps 280),
+// 128^3 to 1e-10 1.7 ms (FP32 sweeps 620), 160^3 2.5 ms (FP32 sweeps 880).
+// Against the FP64 form that sweeps all the way U differs by 2e-15 to 3e-13
+// (the FP32 sweeps differed by 5e-7 to 5e-6) and the sweep counts are equal.
+#include <cmath>
+
+#include "picard_internal.h"
+#include "reduce.h"
+#include "spectral.h"
+
+namespace picard {
+
+constexpr int kSpecCand = 8;        // stop candidates per pass over the spectrum
+constexpr int kSpecPasses = 3;
+
+// Device state of one search.  `skip`: no step is taken (0: go on).
+struct SpecState {
+  double q[kSpecCand];              // candidates, in sweeps after the base iterate
+  double lo, hi, flo, fhi;          // bracket of the plain norm's crossing, and the norms^2 there
+  double T, f0;                     // threshold^2, the base residual's norm^2
+  double q1, slope;                 // crossing, and d ln(norm^2) / d sweep there
+  double steps;                     // sweeps the step covers
+  int64_t to;                       // iterate the step ends on
+  int32_t skip;
+  uint32_t arrive;
+};
+
+namespace {
+
+constexpr int kT = 256;
+enum { kSpecGo = 0, kSpecFew = 1, kSpecBad = 2 };
+// fewer sweeps than this are not worth the step (about 30 launches)
+constexpr int kSpecFewest = 32;
+
+// Compact padded FP64 layout of the transforms: x fastest, rows of PX.
+struct SpecGeo {
+  int nx, ny, nz, PX;
+  int64_t X, XY;                    // node strides of the guard layout
+  int px, py, pz;
+  int64_t len;                      // PX ny nz
+  double ax, ay, az, af, dx2, dy2, dz2;
+  const double *eig[3];             // per axis: 4 a sin^2 (n values), then 4 a cos^2
+};
+
+__global__ void __launch_bounds__(kT) k_spec_basis(int n, int flow, double *fwd, double *inv) {
+  const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
+  const int np = spec_cols(n);
+  if (t >= spec_mat_len(n)) return;
+  const int r = (int)(t / np), c = (int)(t % np);
+  const bool in = r < n && c < n;
+  fwd[t] = in ? spec_basis(n, flow != 0, r, c) : 0.0;
+  inv[t] = in ? spec_basis(n, flow != 0, c, r) : 0.0;
+}
+
+__global__ void __launch_bounds__(kT) k_spec_eig(int n, int flow, double a, double *eig) {
+  const int k = (int)blockIdx.x * kT + (int)threadIdx.x;
+  if (k >= n) return;
+  const double h = spec_half_angle(n, flow != 0, k);
+  const double s = sinpi(h), c = cospi(h);
+  eig[k] = 4.0 * a * s * s;
+  eig[n + k] = 4.0 * a * c * c;
+}
+
+// Ends a reduction: true in the block that finishes last, after every
+// block's partials are visible.
+__device__ __forceinline__ bool last_block(uint32_t *arrive) {
+  __shared__ bool last;
+  if (threadIdx.x == 0) {
+    __threadfence();
+    last = atomicAdd(arrive, 1u) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (last) __threadfence();
+  return last;
+}
+
+// r = b - A u of the base iterate with periodic images of u itself, into the
+// compact layout (padding zero), and its norm; the last block sets up the search.
+__global__ void __launch_bounds__(kT) k_spec_residual(SpecGeo g, const double *__restrict__ u,
+                                                      const double *__restrict__ b,
+                                                      double *__restrict__ out,
+                                                      double *__restrict__ partials,
+                                                      const JacobiState *js, SpecState *st,
+                                                      int64_t base, double lnmax) {
+  __shared__ double sh[kT / 64];
+  double acc = 0.0;
+  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < g.len; t += (int64_t)gridDim.x * kT) {
+    const uint32_t row = (uint32_t)(t / g.PX), x = (uint32_t)(t % g.PX);
+    const uint32_t y = row % (uint32_t)g.ny, z = row / (uint32_t)g.ny;
+    double r = 0.0;
+    if ((int)x < g.nx) {
+      const int64_t c = (x + 1) + g.X * (int64_t)(y + 1) + g.XY * (int64_t)(z + 1);
+      const int64_t e = g.px && (int)x == g.nx - 1 ? c - (g.nx - 1) : c + 1;
+      const int64_t w = g.px && x == 0 ? c + (g.nx - 1) : c - 1;
+      const int64_t n = g.py && (int)y == g.ny - 1 ? c - (g.ny - 1) * g.X : c + g.X;
+      const int64_t s = g.py && y == 0 ? c + (g.ny - 1) * g.X : c - g.X;
+      const int64_t tp = g.pz && (int)z == g.nz - 1 ? c - (g.nz - 1) * g.XY : c + g.XY;
+      const int64_t bt = g.pz && z == 0 ? c + (g.nz - 1) * g.XY : c - g.XY;
+      const double u2 = 2.0 * u[c];
+      r = b[c] - ((u[e] + u[w] - u2) / g.dx2 + (u[n] + u[s] - u2) / g.dy2 +
+                  (u[tp] + u[bt] - u2) / g.dz2);
+    }
+    out[t] = r;
+    acc += r * r;
+  }
+  const double s = block_sum(acc, sh);
+  if (threadIdx.x == 0) partials[blockIdx.x] = s;
+  if (!last_block(&st->arrive)) return;
+  const double f0 = final_sum(partials, gridDim.x, sh);
+  if (threadIdx.x) return;
+  st->arrive = 0;
+  st->f0 = f0;
+  const double T = js->thresh * js->thresh;
+  st->T = T;
+  st->to = -1;
+  const double span = (double)(js->last - base);
+  // an infinite or NaN residual is left to the sweeps, as is a solve that has stopped
+  st->skip = !(f0 < 1.0e300) || !(T < 1.0e300) ? kSpecBad : (js->slot[base & 1].done || f0 <= T ? kSpecFew : kSpecGo);
+  // no mode decays slower than the slowest one
+  double hi = span;
+  if (T > 0.0 && lnmax < 0.0) hi = fmin(span, ceil(log(T / f0) / (2.0 * lnmax)) + 1.0);
+  st->lo = 0.0;
+  st->flo = f0;
+  st->hi = hi;
+  st->fhi = -1.0;
+  for (int i = 0; i < kSpecCand; ++i) st->q[i] = fmax(1.0, floor(ldexp(hi, -i)));
+}
+
+// sum w lambda^(2 q) over the spectrum for the pass's candidates, descending
+// (pass 0: halvings of the bound) or ascending in q (later passes: a division
+// of the bracket); the last block narrows the bracket and, after the last pass,
+// interpolates ln(norm^2) in it.  Bound: one read of the spectrum and the
+// exponentials (eight per mode that has not decayed away).
+__global__ void __launch_bounds__(kT) k_spec_search(SpecGeo g, const double *__restrict__ R,
+                                                    double *__restrict__ partials, SpecState *st,
+                                                    int pass) {
+  __shared__ double sh[kT / 64];
+  __shared__ double tot[kSpecCand];
+  if (st->skip) return;
+  double q2[kSpecCand], qmin = 1.0e300;
+#pragma unroll
+  for (int i = 0; i < kSpecCand; ++i) {
+    q2[i] = 2.0 * st->q[i];
+    qmin = fmin(qmin, q2[i]);
+  }
+  double acc[kSpecCand];
+#pragma unroll
+  for (int i = 0; i < kSpecCand; ++i) acc[i] = 0.0;
+  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < g.len; t += (int64_t)gridDim.x * kT) {
+    const uint32_t row = (uint32_t)(t / g.PX), x = (uint32_t)(t % g.PX);
+    if ((int)x >= g.nx) continue;
+    const uint32_t y = row % (uint32_t)g.ny, z = row / (uint32_t)g.ny;
+    bool neg;
+    const double ln = spec_ln(g.eig[0][x] + g.eig[1][y] + g.eig[2][z],
+                              g.eig[0][g.nx + x] + g.eig[1][g.ny + y] + g.eig[2][g.nz + z], &neg);
+    if (qmin * ln < -700.0) continue;                // below the smallest double at every candidate
+    const double w = R[t] * R[t];
+#pragma unroll
+    for (int i = 0; i < kSpecCand; ++i) acc[i] += w * exp(q2[i] * ln);
+  }
+#pragma unroll
+  for (int i = 0; i < kSpecCand; ++i) {
+    const double s = block_sum(acc[i], sh);
+    if (threadIdx.x == 0) partials[(int64_t)i * gridDim.x + blockIdx.x] = s;
+    __syncthreads();
+  }
+  if (!last_block(&st->arrive)) return;
+  for (int i = 0; i < kSpecCand; ++i) {
+    const double s = final_sum(partials + (int64_t)i * gridDim.x, gridDim.x, sh);
+    if (threadIdx.x == 0) tot[i] = s;
+    __syncthreads();
+  }
+  if (threadIdx.x) return;
+  st->arrive = 0;
+  double lo = st->lo, hi = st->hi, flo = st->flo, fhi = st->fhi;
+  for (int i = 0; i < kSpecCand; ++i) {
+    const double q = st->q[i];
+    if (tot[i] > st->T) {
+      if (q > lo) lo = q, flo = tot[i];
+    } else if (q < hi || fhi < 0.0) {
+      hi = q, fhi = tot[i];
+    }
+  }
+  st->lo = lo;
+  st->hi = hi;
+  st->flo = flo;
+  st->fhi = fhi;
+  if (pass + 1 < kSpecPasses) {
+    for (int i = 0; i < kSpecCand; ++i)
+      st->q[i] = fmax(1.0, floor(lo + (hi - lo) * (double)(i + 1) / (double)(kSpecCand + 1)));
+    return;
+  }
+  double q1 = hi, slope = 0.0;
+  if (fhi >= 0.0 && hi > lo) {
+    const double a = log(flo), c = log(fmax(fhi, 1.0e-300));
+    slope = (c - a) / (hi - lo);
+    if (st->T > 0.0 && slope < 0.0) q1 = fmin(hi, fmax(lo, lo + (log(st->T) - a) / slope));
+  }
+  st->q1 = fmax(1.0, ceil(q1));
+  st->slope = slope;
+}
+
+// The spectrum of r_{q1-1} (what = 0) or of the step's change of U, -af times
+// the sum of its sweeps' residuals (what = 1).
+__global__ void __launch_bounds__(kT) k_spec_scale(SpecGeo g, const double *__restrict__ R,
+                                                   double *__restrict__ out, const SpecState *st,
+                                                   int what) {
+  if (st->skip) return;
+  const double q = what ? st->steps : st->q1 - 1.0;
+  const bool odd = fmod(q, 2.0) != 0.0;
+  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < g.len; t += (int64_t)gridDim.x * kT) {
+    const uint32_t row = (uint32_t)(t / g.PX), x = (uint32_t)(t % g.PX);
+    const uint32_t y = row % (uint32_t)g.ny, z = row / (uint32_t)g.ny;
+    double v = 0.0;
+    if ((int)x < g.nx) {
+      const double s = g.eig[0][x] + g.eig[1][y] + g.eig[2][z];
+      const double c = g.eig[0][g.nx + x] + g.eig[1][g.ny + y] + g.eig[2][g.nz + z];
+      bool neg;
+      const double ln = spec_ln(s, c, &neg);
+      const double sg = neg && odd ? -1.0 : 1.0;
+      if (what == 0) {
+        v = q > 0.0 ? sg * exp(q * ln) : 1.0;
+      } else {
+        // (1 - lambda^q) / (1 - lambda)
+        v = s == 0.0 ? q : (neg ? 1.0 - sg * exp(q * ln) : -expm1(q * ln)) / s;
+        v = -g.af * v;
+      }
+      v = v * R[t];
+    }
+    out[t] = v;
+  }
+}
+
+// Norm of J0 w (w = r_{q1-1}, zeros beyond every boundary): the stop rule's
+// residual of iterate base + q1.  The last block moves the crossing by the
+// slope and fixes the iterate the step ends on, `margin` before it.
+__global__ void __launch_bounds__(kT) k_spec_rule(SpecGeo g, const double *__restrict__ w,
+                                                  double *__restrict__ partials,
+                                                  const JacobiState *js, SpecState *st, int64_t base,
+                                                  int margin) {
+  __shared__ double sh[kT / 64];
+  if (st->skip) return;
+  double acc = 0.0;
+  const int64_t P = (int64_t)g.PX * g.ny;
+  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < g.len; t += (int64_t)gridDim.x * kT) {
+    const uint32_t row = (uint32_t)(t / g.PX), x = (uint32_t)(t % g.PX);
+    if ((int)x >= g.nx) continue;
+    const uint32_t y = row % (uint32_t)g.ny, z = row / (uint32_t)g.ny;
+    const double e = (int)x + 1 < g.nx ? w[t + 1] : 0.0, ww = x > 0 ? w[t - 1] : 0.0;
+    const double n = (int)y + 1 < g.ny ? w[t + g.PX] : 0.0, s = y > 0 ? w[t - g.PX] : 0.0;
+    const double tp = (int)z + 1 < g.nz ? w[t + P] : 0.0, bt = z > 0 ? w[t - P] : 0.0;
+    const double r = g.ax * (e + ww) + g.ay * (n + s) + g.az * (tp + bt);
+    acc += r * r;
+  }
+  const double s = block_sum(acc, sh);
+  if (threadIdx.x == 0) partials[blockIdx.x] = s;
+  if (!last_block(&st->arrive)) return;
+  const double F = final_sum(partials, gridDim.x, sh);
+  if (threadIdx.x) return;
+  st->arrive = 0;
+  const int64_t last = js->last;
+  double q = st->q1;
+  if (st->fhi < 0.0) q = (double)(last - base);                  // not reached within the cap
+  else if (st->T > 0.0 && F > 0.0 && st->slope < 0.0) q = q + (log(st->T) - log(F)) / st->slope;
+  if (!(q < (double)(last - base))) q = (double)(last - base);
+  int64_t stop = base + (int64_t)ceil(q);
+  if (stop + 1 > (int64_t)js->maxit + 2) stop = last;            // the rule is not applied past maxit
+  const int64_t to = stop - margin;
+  if (to - base < kSpecFewest || to > 0x7fffff00) {
+    st->skip = kSpecFew;
+    return;
+  }
+  st->to = to;
+  st->steps = (double)(to - base);
+}
+
+// U_to = U_base + its change on interior nodes, into the sweeps' buffer of iterate `to`.
+__global__ void __launch_bounds__(kT) k_spec_apply(SpecGeo g, const double *__restrict__ du,
+                                                   const double *u, double *b0, double *b1,
+                                                   double *b2, const SpecState *st) {
+  if (st->skip) return;
+  const int r = (int)(st->to % 3);
+  double *out = r == 0 ? b0 : (r == 1 ? b1 : b2);
+  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < g.len; t += (int64_t)gridDim.x * kT) {
+    const uint32_t row = (uint32_t)(t / g.PX), x = (uint32_t)(t % g.PX);
+    if ((int)x >= g.nx) continue;
+    const uint32_t y = row % (uint32_t)g.ny, z = row / (uint32_t)g.ny;
+    const int64_t c = (x + 1) + g.X * (int64_t)(y + 1) + g.XY * (int64_t)(z + 1);
+    out[c] = u[c] + du[t];
+  }
+}
+
+// One axis of the transform over the whole array: 36 TFLOP/s FP64 at 160^3
+// (37 us), 43 at 128^3 (20 us), where a large library product reaches 73.  Axis tiles of a column tile
+// next to each other on one XCD (block b runs on XCD b % 8), so that the
+// columns are read from its L2 after the first.
+template <int AT, bool XAXIS>
+__global__ void __launch_bounds__(kSpecT) k_spec_axis(SpecTile t, int nat, int64_t nct,
+                                                      const SpecState *st) {
+  __shared__ double lds[2 * kSpecLds];
+  if (st->skip) return;
+  const int64_t i = blockIdx.x >> 3;
+  const int at = (int)(i % nat);
+  const int64_t ct = (i / nat) * 8 + (blockIdx.x & 7);
+  if (ct >= nct) return;
+  spec_tile<AT, XAXIS>(t, at * 32 * AT, ct * kSpecCols, lds);
+}
+
+template <bool XAXIS>
+void launch_axis(hipStream_t s, const SpecTile &t, const SpecState *st) {
+  const int64_t nct = (t.total + kSpecCols - 1) / kSpecCols;
+  // outputs in tiles of 64, or of 32 where that pads less
+  const bool wide = ((t.nout + 63) & ~63) == ((t.nout + 31) & ~31);
+  const int nat = wide ? (t.nout + 63) / 64 : (t.nout + 31) / 32;
+  const unsigned blocks = (unsigned)(((nct + 7) & ~int64_t(7)) * nat);
+  if (wide) k_spec_axis<2, XAXIS><<<blocks, kSpecT, 0, s>>>(t, nat, nct, st);
+  else k_spec_axis<1, XAXIS><<<blocks, kSpecT, 0, s>>>(t, nat, nct, st);
+}
+
+}  // namespace
+
+bool spec_eligible(const picard_ctx *c) {
+  const GridDims &g = c->gd;
+  return (c->order_free || (c->split && !c->mx_forced)) && g.nx <= kSpecMaxAxis &&
+         g.ny <= kSpecMaxAxis && g.nz <= kSpecMaxAxis;
+}
+
+void spec_release(picard_ctx *c) {
+  for (double *&p : c->spec_buf)
+    if (p) (void)hipFree(p), p = nullptr;
+  for (int d = 0; d < 3; ++d)
+    for (double **p : {&c->spec_fwd[d], &c->spec_inv[d], &c->spec_eig[d]})
+      if (*p) (void)hipFree(*p), *p = nullptr;
+  if (c->spec_st) (void)hipFree(c->spec_st), c->spec_st = nullptr;
+  if (c->spec_host) (void)hipHostFree(c->spec_host), c->spec_host = nullptr;
+}
+
+// The axes' bases and eigenvalues, and the transforms' buffers.
+int spec_create(picard_ctx *c) {
+  const GridDims &g = c->gd;
+  const int n[3] = {g.nx, g.ny, g.nz};
+  const double d2[3] = {g.dxyz[0] * g.dxyz[0], g.dxyz[1] * g.dxyz[1], g.dxyz[2] * g.dxyz[2]};
+  const double sum = 1.0 / d2[0] + 1.0 / d2[1] + 1.0 / d2[2];
+  const int64_t len = (int64_t)((g.nx + 15) & ~15) * g.ny * g.nz;
+  for (double *&p : c->spec_buf) PICARD_HIP(hipMalloc(&p, sizeof(double) * len));
+  c->spec_lnmax = 0.0;
+  double smin = 0.0, cmin = 0.0;
+  for (int d = 0; d < 3; ++d) {
+    PICARD_HIP(hipMalloc(&c->spec_fwd[d], sizeof(double) * spec_mat_len(n[d])));
+    PICARD_HIP(hipMalloc(&c->spec_inv[d], sizeof(double) * spec_mat_len(n[d])));
+    PICARD_HIP(hipMalloc(&c->spec_eig[d], sizeof(double) * 2 * n[d]));
+    const double a = 0.5 / (d2[d] * sum);             // ax, ay, az of CalcEpotential.f90:44-47
+    k_spec_basis<<<grid_blocks(spec_mat_len(n[d]), kT), kT, 0, c->stream>>>(n[d], g.flow[d], c->spec_fwd[d],
+                                                                            c->spec_inv[d]);
+    k_spec_eig<<<grid_blocks(n[d], kT), kT, 0, c->stream>>>(n[d], g.flow[d], a, c->spec_eig[d]);
+    PICARD_HIP(hipGetLastError());
+    // smallest sin^2 and cos^2 of the axis
+    const double pi = 3.14159265358979323846;
+    const double h = g.flow[d] ? 0.5 / (n[d] + 1) : 0.0;
+    const double k = g.flow[d] ? 0.5 / (n[d] + 1) : (n[d] % 2 ? 0.5 / n[d] : 0.0);
+    smin += 4.0 * a * std::sin(pi * h) * std::sin(pi * h);
+    cmin += 4.0 * a * std::sin(pi * k) * std::sin(pi * k);
+  }
+  c->spec_lnmax = std::log1p(-std::fmin(smin, cmin));
+  PICARD_HIP(hipMalloc(&c->spec_st, sizeof(SpecState)));
+  PICARD_HIP(hipMemsetAsync(c->spec_st, 0, sizeof(SpecState), c->stream));
+  PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->spec_host), sizeof(SpecState)));
+  return PICARD_OK;
+}
+
+// From iterate `base` (in `u`, guard layout) to an iterate at least `margin`
+// before the one the stop rule will pick, left in the sweeps' buffers jb; *to is
+// that iterate, -1 if too few sweeps are left for a step, or -2 if the
+// residual has no finite norm.
+int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, int64_t *to) {
+  const GridDims &g = c->gd;
+  hipStream_t s = c->stream;
+  SpecGeo sg;
+  sg.nx = g.nx; sg.ny = g.ny; sg.nz = g.nz;
+  sg.PX = (g.nx + 15) & ~15;
+  sg.X = g.X; sg.XY = (int64_t)g.X * g.Y;
+  sg.px = !g.flow[0]; sg.py = !g.flow[1]; sg.pz = !g.flow[2];
+  sg.len = (int64_t)sg.PX * g.ny * g.nz;
+  const double dx = g.dxyz[0], dy = g.dxyz[1], dz = g.dxyz[2];
+  const double den = 1.0 / ((dx * dy) * (dx * dy) + (dx * dz) * (dx * dz) + (dy * dz) * (dy * dz));
+  sg.ax = 0.5 * den * ((dy * dz) * (dy * dz));            // CalcEpotential.f90:44-47
+  sg.ay = 0.5 * den * ((dx * dz) * (dx * dz));
+  sg.az = 0.5 * den * ((dx * dy) * (dx * dy));
+  sg.af = 0.5 * den * ((dx * dy * dz) * (dx * dy * dz));
+  sg.dx2 = dx * dx; sg.dy2 = dy * dy; sg.dz2 = dz * dz;
+  for (int d = 0; d < 3; ++d) sg.eig[d] = c->spec_eig[d];
+  SpecState *st = c->spec_st;
+  double *B0 = c->spec_buf[0], *B1 = c->spec_buf[1], *B2 = c->spec_buf[2];
+  const int64_t P = (int64_t)sg.PX * g.ny;
+  auto axis = [&](int d, double *const *mat, const double *in, double *out) {
+    SpecTile t;
+    t.M = mat[d];
+    t.in = in;
+    t.out = out;
+    t.n = d == 0 ? g.nx : (d == 1 ? g.ny : g.nz);
+    t.np = spec_cols(t.n);
+    t.nout = d == 0 ? sg.PX : t.n;
+    t.ld = d == 2 ? P : sg.PX;
+    t.gs = d == 1 ? P : 0;
+    t.total = d == 0 ? (int64_t)g.ny * g.nz : (d == 1 ? (int64_t)sg.PX * g.nz : P);
+    t.gpr = (uint32_t)((d == 1 ? sg.PX : t.total) / 16);
+    if (d == 0) launch_axis<true>(s, t, st);
+    else launch_axis<false>(s, t, st);
+  };
+  // blocks of the passes over the array: four per CU at most, eight elements a
+  // thread at least; their partials fit the context's array (the search keeps
+  // eight sums per block)
+  int64_t nb = (sg.len + 8 * kT - 1) / (8 * kT);
+  if (nb > 1024) nb = 1024;
+  const int64_t cap = 4 * c->s.partials_len / kSpecCand;
+  if (nb > cap) nb = cap;
+  const unsigned B = (unsigned)(nb < 1 ? 1 : nb);
+  double *part = c->s.partials;
+  k_spec_residual<<<B, kT, 0, s>>>(sg, u, c->b, B0, part, c->js, st, base, c->spec_lnmax);
+  axis(0, c->spec_fwd, B0, B1);
+  axis(1, c->spec_fwd, B1, B2);
+  axis(2, c->spec_fwd, B2, B0);
+  for (int p = 0; p < kSpecPasses; ++p) k_spec_search<<<B, kT, 0, s>>>(sg, B0, part, st, p);
+  k_spec_scale<<<B, kT, 0, s>>>(sg, B0, B1, st, 0);
+  axis(0, c->spec_inv, B1, B2);
+  axis(1, c->spec_inv, B2, B1);
+  axis(2, c->spec_inv, B1, B2);
+  k_spec_rule<<<B, kT, 0, s>>>(sg, B2, part, c->js, st, base, margin);
+  k_spec_scale<<<B, kT, 0, s>>>(sg, B0, B1, st, 1);
+  axis(0, c->spec_inv, B1, B2);
+  axis(1, c->spec_inv, B2, B1);
+  axis(2, c->spec_inv, B1, B2);
+  k_spec_apply<<<B, kT, 0, s>>>(sg, B2, u, c->jb[0], c->jb[1], c->jb[2], st);
+  PICARD_HIP(hipGetLastError());
+  PICARD_HIP(hipMemcpyAsync(c->spec_host, st, sizeof(SpecState), hipMemcpyDeviceToHost, s));
+  PICARD_HIP(hipStreamSynchronize(s));
+  const SpecState *h = c->spec_host;
+  *to = h->skip == kSpecBad ? -2 : (h->skip ? -1 : h->to);
+  return PICARD_OK;
+}
+
+}  // namespace picard

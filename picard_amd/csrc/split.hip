@@ -8,8 +8,10 @@
 // ParticlesTransfer's single-domain wrap by index arithmetic.
 //
 // Deposit: int64 fixed point (2^-40 units) with integer guard folds, so the
-// densities do not depend on particle order.  Field solve: iterative
-// refinement -- FP32 Jacobi sweeps on the correction e of A e = r with an
+// densities do not depend on particle order.  Field solve: the eigenbasis step
+// and FP64 sweeps of launch_calc_epotential; where that step is not taken (an
+// axis too long, a solve of few sweeps, a residual without a finite norm, or a
+// caller that asked for sweeps) iterative refinement -- FP32 Jacobi sweeps on the correction e of A e = r with an
 // FP64 outer residual r = b - A u and FP64 update u += e; the residual norm of
 // every sweep's iterate u + e_j (= r - A e_j) is accumulated in FP64, so the
 // stop rule of CalcEpotential.f90:60-62 is applied sweep by sweep.  E is
@@ -2447,6 +2449,10 @@ OuterGeo outer_sched(picard_ctx *c) {
 }
 
 int sp_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t *sweeps) {
+  if (spec_eligible(c) && maxit > 32) {
+    const int rc = launch_calc_epotential(c, maxerr, maxit, sweeps);
+    if (rc != kNoSpecStep) return rc;
+  }
   const GridDims &g = c->gd;
   const double dx = g.dxyz[0], dy = g.dxyz[1], dz = g.dxyz[2];
   const double den = 1.0 / ((dx * dy) * (dx * dy) + (dx * dz) * (dx * dz) + (dy * dz) * (dy * dz));
