@@ -1399,22 +1399,29 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
   };
   bool done = false, few = false;
   if (spec_eligible(c) && last > 64) {
-    // the eigenbasis step to a few iterates before the stop, then the sweeps
-    // with the stop test; a solve that passes one of the first two tests may
-    // have been taken past its stop and starts again with a wider margin
+    // to a few iterates before the stop, then the sweeps with the stop test;
+    // a solve that passes one of the first two tests may have been taken past
+    // its stop and starts again with a wider margin
+    const bool exact = !c->split && !c->order_free;
     for (int margin = 4; !done && margin <= 1024; margin *= 16) {
       PICARD_TRY(begin());
-      // the order-free form's first sweep reads the halo U came in with
-      const int64_t base = c->order_free ? 1 : 0;
+      // the FP64 forms' first sweep reads the halo U came in with
+      const int64_t base = c->split ? 0 : 1;
       if (base) pass(1, 1, nullptr, nullptr, nullptr);
       int64_t to = -1;
-      PICARD_TRY(spec_step(c, base ? c->jb[1] : c->U, base, margin, &to));
+      PICARD_TRY(spec_step(c, base ? c->jb[1] : c->U, base, margin, !exact, &to));
       if (to < 0) {
         if (c->split) return kNoSpecStep;
         few = to == -1;
         break;
       }
-      PICARD_TRY(sweep(to + 1, to + 1, margin + 5));
+      const int T = jacobi_block_sweeps(g);
+      if (exact) {                // the same iterates by sweeps that leave out the test
+        const int64_t launches = (to - base) / T;
+        to = base + T * launches;
+        PICARD_TRY(launch_jacobi_block(c, base, launches));
+      }
+      PICARD_TRY(sweep(to + 1, to + 1, margin + T + 4));
       done = fin.result == last || fin.result > to + 2;
     }
   }

@@ -267,7 +267,13 @@ int launch_bc_fields(picard_ctx *c);
 bool spec_eligible(const picard_ctx *c);
 int spec_create(picard_ctx *c);
 void spec_release(picard_ctx *c);
-int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, int64_t *to);
+// apply = false: only finds the iterate
+int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, bool apply, int64_t *to);
+
+// ---- jacobi_block.hip ----
+int jacobi_block_sweeps(const GridDims &g);   // sweeps per launch
+bool jacobi_block_eligible(const GridDims &g);
+int launch_jacobi_block(picard_ctx *c, int64_t from, int64_t launches);
 
 // ---- diag.hip ----
 int diagnostics(picard_ctx *c, const double *mass, picard_diag *out);

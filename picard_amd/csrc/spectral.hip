@@ -341,10 +341,12 @@ void launch_axis(hipStream_t s, const SpecTile &t, const SpecState *st) {
 
 }  // namespace
 
+// The forms that are held to the reference's rounding use it to find their
+// stop, where the sweeps up to it can do without the stop test.
 bool spec_eligible(const picard_ctx *c) {
   const GridDims &g = c->gd;
-  return (c->order_free || (c->split && !c->mx_forced)) && g.nx <= kSpecMaxAxis &&
-         g.ny <= kSpecMaxAxis && g.nz <= kSpecMaxAxis;
+  const bool form = c->split ? !c->mx_forced : c->order_free || jacobi_block_eligible(g);
+  return form && g.nx <= kSpecMaxAxis && g.ny <= kSpecMaxAxis && g.nz <= kSpecMaxAxis;
 }
 
 void spec_release(picard_ctx *c) {
@@ -394,7 +396,7 @@ int spec_create(picard_ctx *c) {
 // before the one the stop rule will pick, left in the sweeps' buffers jb; *to is
 // that iterate, -1 if too few sweeps are left for a step, or -2 if the
 // residual has no finite norm.
-int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, int64_t *to) {
+int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, bool apply, int64_t *to) {
   const GridDims &g = c->gd;
   hipStream_t s = c->stream;
   SpecGeo sg;
@@ -448,11 +450,13 @@ int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, int64_t 
   axis(1, c->spec_inv, B2, B1);
   axis(2, c->spec_inv, B1, B2);
   k_spec_rule<<<B, kT, 0, s>>>(sg, B2, part, c->js, st, base, margin);
-  k_spec_scale<<<B, kT, 0, s>>>(sg, B0, B1, st, 1);
-  axis(0, c->spec_inv, B1, B2);
-  axis(1, c->spec_inv, B2, B1);
-  axis(2, c->spec_inv, B1, B2);
-  k_spec_apply<<<B, kT, 0, s>>>(sg, B2, u, c->jb[0], c->jb[1], c->jb[2], st);
+  if (apply) {
+    k_spec_scale<<<B, kT, 0, s>>>(sg, B0, B1, st, 1);
+    axis(0, c->spec_inv, B1, B2);
+    axis(1, c->spec_inv, B2, B1);
+    axis(2, c->spec_inv, B1, B2);
+    k_spec_apply<<<B, kT, 0, s>>>(sg, B2, u, c->jb[0], c->jb[1], c->jb[2], st);
+  }
   PICARD_HIP(hipGetLastError());
   PICARD_HIP(hipMemcpyAsync(c->spec_host, st, sizeof(SpecState), hipMemcpyDeviceToHost, s));
   PICARD_HIP(hipStreamSynchronize(s));
