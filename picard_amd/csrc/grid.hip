@@ -1211,6 +1211,9 @@ int launch_bc_potentials(picard_ctx *c) {
   const double tau = 6.2831853071795864769252867665590;
   const double eps0 = 8.854187817e-12;
   const double kfac = 1.0 / (2.0 * tau * eps0);
+  // rows of more cells: the kernels below, which share charge or distances
+  // between a block's chains
+  if (bcpot_seq_eligible(g)) return launch_bcpot_seq(c, kfac);
   const int per_block = kFaceR * kFaceWaves;
   constexpr int kLdsR = 2, kLdsWaves = 4;
   const size_t ring_bytes = sizeof(double) * 64 * (size_t)(g.nx + 1);

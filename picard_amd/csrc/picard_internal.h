@@ -275,6 +275,10 @@ int jacobi_block_sweeps(const GridDims &g);   // sweeps per launch
 bool jacobi_block_eligible(const GridDims &g);
 int launch_jacobi_block(picard_ctx *c, int64_t from, int64_t launches);
 
+// ---- bcpot_seq.hip ----
+bool bcpot_seq_eligible(const GridDims &g);
+int launch_bcpot_seq(picard_ctx *c, double kfac);
+
 // ---- diag.hip ----
 int diagnostics(picard_ctx *c, const double *mass, picard_diag *out);
 
