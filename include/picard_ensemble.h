@@ -20,8 +20,12 @@
  * sums reduce their partials in a fixed order.
  *
  * The FP32-split form: particles as int16 cell + FP32 offset with FP32
- * velocities, FP32 Jacobi sweeps on the correction with FP64 refinement every
- * `inner` sweeps, FP64 face sums (BCpotentials) and FP64 refinement residuals.
+ * velocities, FP64 face sums (BCpotentials), and the Jacobi iterate that the
+ * stop rule picks, computed in closed form in FP64 in the eigenbasis of the
+ * operator.  Simulations with an axis of more than 1024 cells, or whose residual
+ * has no finite norm, run FP32 Jacobi sweeps on the correction with FP64
+ * refinement every `inner` sweeps instead (these are the sweeps that the tile
+ * shape and the autotuner are about, and that solve_chunks counts).
  * The stop rule is CalcEpotential.f90:60-62 (relative residual maxerr, tested
  * before every update, at most 2*maxit+1 sweeps) applied to every iterate, with
  * fresh periodic images in the residual. */
@@ -107,7 +111,7 @@ typedef struct {
   int64_t pushed;           /* particles given to AdvanceVelocity, all simulations */
   int64_t max_sweeps;       /* largest Jacobi sweep count of the step */
   int64_t sum_sweeps;       /* sum of the simulations' sweep counts */
-  int64_t solve_chunks;     /* solve graph replays (64 sweeps each) */
+  int64_t solve_chunks;     /* solve graph replays (64 sweeps each), 0 when no simulation was swept */
   int64_t cell_sweeps;      /* sum over simulations of interior cells x sweeps */
   double step_ms;           /* host wall time of the step */
   double solve_ms;          /* of it, the solve (refinement passes and sweeps) */

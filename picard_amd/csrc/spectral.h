@@ -56,6 +56,10 @@ __device__ __forceinline__ double spec_ln(double s, double c, bool *neg) {
   return log1p(-fmin(*neg ? c : s, 1.0));
 }
 
+// Host: spectral.hip.
+int spec_axis_tables(hipStream_t s, int n, bool flow, double a, double *fwd, double *inv, double *eig);
+double spec_slowest(const int n[3], const int flow[3], const double a[3]);
+
 typedef double d4v __attribute__((ext_vector_type(4)));
 
 // One output tile of a basis applied along one axis.  The tile holds 32 AT

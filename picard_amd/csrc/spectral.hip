@@ -359,6 +359,27 @@ void spec_release(picard_ctx *c) {
   if (c->spec_host) (void)hipHostFree(c->spec_host), c->spec_host = nullptr;
 }
 
+// Basis, transpose and eigenvalue parts of one axis; `a` is the Jacobi weight of its neighbours.
+int spec_axis_tables(hipStream_t s, int n, bool flow, double a, double *fwd, double *inv, double *eig) {
+  k_spec_basis<<<grid_blocks(spec_mat_len(n), kT), kT, 0, s>>>(n, flow, fwd, inv);
+  k_spec_eig<<<grid_blocks(n, kT), kT, 0, s>>>(n, flow, a, eig);
+  PICARD_HIP(hipGetLastError());
+  return PICARD_OK;
+}
+
+// Largest ln|lambda| of a box from the axes' smallest 4 a sin^2 and 4 a cos^2.
+double spec_slowest(const int n[3], const int flow[3], const double a[3]) {
+  double smin = 0.0, cmin = 0.0;
+  const double pi = 3.14159265358979323846;
+  for (int d = 0; d < 3; ++d) {
+    const double h = flow[d] ? 0.5 / (n[d] + 1) : 0.0;
+    const double k = flow[d] ? 0.5 / (n[d] + 1) : (n[d] % 2 ? 0.5 / n[d] : 0.0);
+    smin += 4.0 * a[d] * std::sin(pi * h) * std::sin(pi * h);
+    cmin += 4.0 * a[d] * std::sin(pi * k) * std::sin(pi * k);
+  }
+  return std::log1p(-std::fmin(smin, cmin));
+}
+
 // The axes' bases and eigenvalues, and the transforms' buffers.
 int spec_create(picard_ctx *c) {
   const GridDims &g = c->gd;
@@ -367,25 +388,16 @@ int spec_create(picard_ctx *c) {
   const double sum = 1.0 / d2[0] + 1.0 / d2[1] + 1.0 / d2[2];
   const int64_t len = (int64_t)((g.nx + 15) & ~15) * g.ny * g.nz;
   for (double *&p : c->spec_buf) PICARD_HIP(hipMalloc(&p, sizeof(double) * len));
-  c->spec_lnmax = 0.0;
-  double smin = 0.0, cmin = 0.0;
+  double w[3];
   for (int d = 0; d < 3; ++d) {
     PICARD_HIP(hipMalloc(&c->spec_fwd[d], sizeof(double) * spec_mat_len(n[d])));
     PICARD_HIP(hipMalloc(&c->spec_inv[d], sizeof(double) * spec_mat_len(n[d])));
     PICARD_HIP(hipMalloc(&c->spec_eig[d], sizeof(double) * 2 * n[d]));
-    const double a = 0.5 / (d2[d] * sum);             // ax, ay, az of CalcEpotential.f90:44-47
-    k_spec_basis<<<grid_blocks(spec_mat_len(n[d]), kT), kT, 0, c->stream>>>(n[d], g.flow[d], c->spec_fwd[d],
-                                                                            c->spec_inv[d]);
-    k_spec_eig<<<grid_blocks(n[d], kT), kT, 0, c->stream>>>(n[d], g.flow[d], a, c->spec_eig[d]);
-    PICARD_HIP(hipGetLastError());
-    // smallest sin^2 and cos^2 of the axis
-    const double pi = 3.14159265358979323846;
-    const double h = g.flow[d] ? 0.5 / (n[d] + 1) : 0.0;
-    const double k = g.flow[d] ? 0.5 / (n[d] + 1) : (n[d] % 2 ? 0.5 / n[d] : 0.0);
-    smin += 4.0 * a * std::sin(pi * h) * std::sin(pi * h);
-    cmin += 4.0 * a * std::sin(pi * k) * std::sin(pi * k);
+    w[d] = 0.5 / (d2[d] * sum);                       // ax, ay, az of CalcEpotential.f90:44-47
+    PICARD_TRY(spec_axis_tables(c->stream, n[d], g.flow[d], w[d], c->spec_fwd[d], c->spec_inv[d],
+                                c->spec_eig[d]));
   }
-  c->spec_lnmax = std::log1p(-std::fmin(smin, cmin));
+  c->spec_lnmax = spec_slowest(n, g.flow, w);
   PICARD_HIP(hipMalloc(&c->spec_st, sizeof(SpecState)));
   PICARD_HIP(hipMemsetAsync(c->spec_st, 0, sizeof(SpecState), c->stream));
   PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->spec_host), sizeof(SpecState)));

@@ -107,6 +107,13 @@ class _Lane:
         self.tuned = False
 
 
+# An idle lane that gets a job waits this long for others, so that jobs of one
+# burst start in the same launches: a small job's step (about 1 ms) costs as many
+# launches as a full batch's.  A lane with jobs on the device admits at every
+# step and never waits.
+GATHER_S = 0.010
+
+
 class Server:
     """Continuous-batching server over one ensemble per lane (one lane unless
     `lanes` says otherwise)."""
@@ -159,6 +166,9 @@ class Server:
                 now = time.perf_counter() - t0
                 if time_limit is not None and now > time_limit:
                     break
+                if not running and pending and 0.0 <= now - pending[0].arrival < GATHER_S:
+                    time.sleep(GATHER_S - (now - pending[0].arrival))
+                    continue
                 # admit, in arrival order, every job of this lane that has
                 # arrived and fits the lane and the shared budget
                 while pending and pending[0].arrival <= now:

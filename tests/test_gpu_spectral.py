@@ -114,3 +114,67 @@ def test_zero_charge_and_repeated_solves():
         got.append((dom.calc_epotential(), dom.field(_lib.FIELD_U)))
     dom.close()
     assert got[0][0] == got[2][0] and np.array_equal(got[0][1], got[2][1])
+
+
+def _jacobi(U, b, dx, sweeps):
+    """`sweeps` sweeps with fresh periodic images in y and z, and the residual
+    norms of the last iterate and the one before it."""
+    U = U.copy()
+
+    def images():
+        U[0], U[-1] = U[-2], U[1]
+        U[:, 0], U[:, -1] = U[:, -2], U[:, 1]
+
+    def residual():
+        c = U[1:-1, 1:-1, 1:-1]
+        lap = (U[1:-1, 1:-1, 2:] + U[1:-1, 1:-1, :-2] + U[1:-1, 2:, 1:-1] + U[1:-1, :-2, 1:-1] +
+               U[2:, 1:-1, 1:-1] + U[:-2, 1:-1, 1:-1] - 6.0 * c) / dx ** 2
+        return b - lap
+
+    images()
+    norms = [0.0, float(np.linalg.norm(residual()))]
+    for _ in range(sweeps):
+        U[1:-1, 1:-1, 1:-1] -= dx ** 2 / 6.0 * residual()
+        images()
+        norms = [norms[1], float(np.linalg.norm(residual()))]
+    return U, norms
+
+
+@pytest.mark.parametrize("dims,ppc,kw", [((8, 8, 8), 3, {}), ((17, 9, 33), 2, {}), ((33, 16, 10), 2, {}),
+                                         ((16, 65, 8), 1, {}), ((65, 8, 12), 1, {}),
+                                         ((15, 12, 14), 2, dict(maxit=40)),      # to the cap
+                                         ((12, 10, 9), 2, dict(maxerr=1e-10))])
+def test_ensemble_solve_is_the_jacobi_iterate(dims, ppc, kw):
+    """Each simulation's potential is the iterate that sweeping in FP64 reaches
+    (the tolerance of this file's other solves), and its sweep count the first at which
+    the rule's norm passes, alone and beside another simulation."""
+    from picard_amd import ensemble
+    spec = ensemble.SimSpec(nx=dims[0], ny=dims[1], nz=dims[2], ppc=ppc, dx=10.0, density=5e6,
+                            kelvin=1.2e5, drift=4e5, B=(1e-9, 0.0, 4e-9), seed=sum(dims), **kw)
+    other = ensemble.SimSpec(nx=20, ny=11, nz=24, ppc=2, dx=8.0, density=8e6, kelvin=9e4, drift=5e5,
+                             B=(0.0, 2e-9, 0.0), seed=5)
+    got = []
+    for mix in ([spec], [other, spec]):
+        ens = ensemble.Ensemble.sized_for(mix, steps_room=4)
+        slot = [ens.add(s) for s in mix][-1]
+        ens.step()
+        st = ens.status(slot)
+        got.append((st.sweeps, st.noconv, ens.field(slot, _lib.FIELD_U), ens.field(slot, _lib.FIELD_C)))
+        ens.close()
+    assert got[0][0] == got[1][0] and np.array_equal(got[0][2], got[1][2])
+    sweeps, noconv, U, C = got[0]
+    d = ensemble.derive(spec)
+    b = -C[1:-1, 1:-1, 1:-1] / (d.dV * 8.854187817e-12)
+    U0 = np.zeros_like(U)
+    U0[1:-1, 1:-1, 0], U0[1:-1, 1:-1, -1] = U[1:-1, 1:-1, 0], U[1:-1, 1:-1, -1]
+    ref, (before, last) = _jacobi(U0, b, d.dxyz, sweeps)
+    T = spec.maxerr * np.linalg.norm(b)
+    i = (slice(1, -1),) * 3
+    err = np.linalg.norm(U[i] - ref[i]) / np.linalg.norm(ref[i])
+    print(f"[gpu-spectral] ensemble {dims}: {sweeps} sweeps, noconv {noconv}, {before / T:.9f} "
+          f"{last / T:.9f}, U {err:.2e}", flush=True)
+    assert err <= 1e-11
+    if kw.get("maxit"):
+        assert noconv == 1 and sweeps == 2 * kw["maxit"] + 1
+    else:
+        assert last <= T * (1 + 1e-8) and before > T * (1 - 1e-8)
