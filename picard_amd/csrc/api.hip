@@ -250,9 +250,9 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   PICARD_TRY(dalloc(&c->s.scan_tmp, c->s.scan_tmp_len));
   PICARD_TRY(dalloc(&c->s.counters, 16));
   PICARD_TRY(dalloc(&c->s.key, cap));
-  if (!c->split) PICARD_TRY(dalloc(&c->s.perm, cap));
+  PICARD_TRY(dalloc(&c->s.perm, cap));
   PICARD_TRY(dalloc(&c->s.hist, nb + 1));
-  PICARD_TRY(dalloc(&c->s.cursor, nb));
+  if (!c->split) PICARD_TRY(dalloc(&c->s.cursor, nb));
   const int64_t ncell = (int64_t)g.nx * g.ny * g.nz;
   int64_t pb = grid_blocks(g.G > ncell ? g.G : ncell, 256);
   const int64_t pb3 = interior_launch(g.nx, g.ny, g.nz).blocks();
@@ -494,7 +494,7 @@ int picard_diagnostics(picard_ctx *c, const double *mass, picard_diag *out) {
 
 int picard_advance_position(picard_ctx *c, double dt) {
   CTX_CHECK(c);
-  if (c->split) return sp_push(c, dt);
+  if (c->split) return sp_push(c, dt, c->n);
   return launch_push_x(c, 0, c->n, dt);
 }
 
@@ -691,13 +691,17 @@ int picard_step(picard_ctx *c, double dt, double maxerr, int32_t maxit, const do
   picard_step_stats st{};
   int rc = PICARD_OK;
   if (c->split) {
-    PICARD_TRY(sp_push(c, dt));                                          // picard.f90:564
-    if (nproduced > 0) PICARD_TRY(picard_particles_append(c, produced, produced_species, nproduced));
-    if (c->prod_on)                                                      // :566
-      PICARD_TRY(produce_haser(c, &c->prod_plasma, &c->prod_haser, c->prod_seed, c->steps_done + 1,
-                               dt, nullptr));
+    const int64_t npush = c->n;            // picard.f90:564: pushed by the sort below
+    if (nproduced > 0) rc = picard_particles_append(c, produced, produced_species, nproduced);
+    if (rc == PICARD_OK && c->prod_on)                                   // :566
+      rc = produce_haser(c, &c->prod_plasma, &c->prod_haser, c->prod_seed, c->steps_done + 1, dt,
+                         nullptr);
+    if (rc != PICARD_OK) {                 // a step that ends here has pushed its particles
+      PICARD_TRY(sp_push(c, dt, npush));
+      return rc;
+    }
     const int64_t before = c->n;
-    PICARD_TRY(sp_sort(c, 1));                                           // :569, :572
+    PICARD_TRY(sp_sort(c, 1, npush, dt));                                // :564, :569, :572
     st.num_local = c->n;
     st.removed = before - c->n;
     PICARD_TRY(sp_gridify(c));                                           // :577

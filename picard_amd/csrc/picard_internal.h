@@ -96,9 +96,9 @@ struct DeviceScratch {
   int32_t *counters = nullptr;     // small device counters (errors, totals)
   // deposit (reference order)
   int32_t *key = nullptr;          // per particle
-  int32_t *perm = nullptr;         // per particle
+  int32_t *perm = nullptr;         // per particle (split form: rank within its key)
   int32_t *hist = nullptr;         // S*K + 1
-  int32_t *cursor = nullptr;       // S*K
+  int32_t *cursor = nullptr;       // S*K (FP64 forms)
   // staging for uploads/downloads (AoS)
   double *stage = nullptr;
   int32_t *stage_sp = nullptr;
@@ -294,8 +294,9 @@ int produce_haser(picard_ctx *c, const picard_plasma *pl, const picard_haser *hs
                   int64_t step, double dt, int64_t *produced);
 
 // ---- split.hip ----
-int sp_push(picard_ctx *c, double dt);
-int sp_sort(picard_ctx *c, int wrap);
+int sp_push(picard_ctx *c, double dt, int64_t n);
+// npush > 0: the first npush particles are pushed by dt first
+int sp_sort(picard_ctx *c, int wrap, int64_t npush = 0, double dt = 0.0);
 int sp_gridify(picard_ctx *c, bool flux = false);
 // allocates the flux arrays (F, and Fraw or Ffix) on first use
 int ensure_flux(picard_ctx *c);

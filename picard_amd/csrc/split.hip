@@ -53,18 +53,26 @@ __device__ __forceinline__ int carry(float &f) {
 }
 
 // AdvancePosition in the split form: xi += v dt/dx.
+__device__ __forceinline__ void push_one(int (&c)[3], float (&f)[3], const float (&v)[3], float3 dtdx) {
+  f[0] = f[0] + v[0] * dtdx.x;
+  f[1] = f[1] + v[1] * dtdx.y;
+  f[2] = f[2] + v[2] * dtdx.z;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) c[d] = (int16_t)(c[d] + carry(f[d]));
+}
+
 __global__ void __launch_bounds__(kT) k_sp_push(ParticlesSplit p, int64_t n, float3 dtdx) {
   const int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (q >= n) return;
-  float fx = p.f[0][q] + p.v[0][q] * dtdx.x;
-  float fy = p.f[1][q] + p.v[1][q] * dtdx.y;
-  float fz = p.f[2][q] + p.v[2][q] * dtdx.z;
-  p.c[0][q] = (int16_t)(p.c[0][q] + carry(fx));
-  p.c[1][q] = (int16_t)(p.c[1][q] + carry(fy));
-  p.c[2][q] = (int16_t)(p.c[2][q] + carry(fz));
-  p.f[0][q] = fx;
-  p.f[1][q] = fy;
-  p.f[2][q] = fz;
+  int c[3] = {p.c[0][q], p.c[1][q], p.c[2][q]};
+  float f[3] = {p.f[0][q], p.f[1][q], p.f[2][q]};
+  const float v[3] = {p.v[0][q], p.v[1][q], p.v[2][q]};
+  push_one(c, f, v, dtdx);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    p.c[d][q] = (int16_t)c[d];
+    p.f[d][q] = f[d];
+  }
 }
 
 // xi < 1/2 is x < Lmin; xi > n + 1/2 is x > Lmax.
@@ -128,46 +136,123 @@ __device__ __forceinline__ int32_t wave_add1(int32_t *counter, int32_t k) {
   return ret;
 }
 
-// Sort key of a kept particle (its lower node and species), -1 for a deleted one.
-__global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, GridDims g,
-                                                 int wrap, int32_t *__restrict__ key,
+// Cell and offset of particle q as the sort sees it: pushed first when q <
+// npush (the step's fused AdvancePosition), wrapped when `wrap`.  False if deleted.
+__device__ __forceinline__ bool sort_coords(const ParticlesSplit &p, int64_t q, int64_t npush,
+                                            const GridDims &g, int wrap, float3 dtdx, int (&c)[3],
+                                            float (&f)[3]) {
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    c[d] = p.c[d][q];
+    f[d] = p.f[d][q];
+  }
+  if (q < npush) {
+    const float v[3] = {p.v[0][q], p.v[1][q], p.v[2][q]};
+    push_one(c, f, v, dtdx);
+  }
+  if (sp_delete(g, c, f)) return false;
+  if (wrap) {
+    sp_wrap(g, c, f);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) c[d] = (int16_t)c[d];
+  }
+  return true;
+}
+
+// Sort key of a kept particle (its lower node and species), -1 for a deleted
+// one, and its rank among the particles of its key.  A block takes kFlagPer x
+// 256 consecutive particles; they arrive nearly sorted, so most keys lie in a
+// short stretch from the first ones': those are counted in LDS (the count
+// before is the rank within the block), each key then takes one atomic on its
+// histogram entry, whose return places the block's particles of that key.
+// The other keys (particles that moved a row or a plane on) are added a wave at
+// a time.  With the ranks known the scatter adds nothing: at 128^3 with 64 particles a
+// cell (1.4e8) flag and scatter take 1.31 + 3.15 ms, where a
+// wave's adds in both passes took 1.09 + 4.02; the step's push, 1.14 ms as a pass of its
+// own, costs them 0.1.
+constexpr int kFlagPer = 4;
+constexpr int kFlagWin = 1024;           // keys counted in LDS
+constexpr int kFlagBack = 128;           // of them below the first particle's
+
+__global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, int64_t npush, GridDims g,
+                                                 int wrap, float3 dtdx, int32_t *__restrict__ key,
+                                                 int32_t *__restrict__ rank,
                                                  int32_t *__restrict__ hist) {
-  const int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x;
-  int32_t k = -1;                          // lanes past n stay for the wave's adds
-  if (q < n) {
-    int c[3] = {p.c[0][q], p.c[1][q], p.c[2][q]};
-    const float f[3] = {p.f[0][q], p.f[1][q], p.f[2][q]};
-    if (!sp_delete(g, c, f)) {
-      if (wrap) {
-        sp_wrap(g, c, f);
-        p.c[0][q] = (int16_t)c[0];
-        p.c[1][q] = (int16_t)c[1];
-        p.c[2][q] = (int16_t)c[2];
-      }
+  __shared__ int32_t cnt[kFlagWin];
+  __shared__ int32_t first;
+  for (int e = threadIdx.x; e < kFlagWin; e += kT) cnt[e] = 0;
+  if (threadIdx.x == 0) first = 0;
+  const int64_t q0 = (int64_t)blockIdx.x * (kT * kFlagPer) + threadIdx.x;
+  const int32_t cells = (int32_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
+  int32_t k[kFlagPer], r[kFlagPer];
+#pragma unroll
+  for (int h = 0; h < kFlagPer; ++h) {
+    const int64_t q = q0 + h * kT;
+    k[h] = -1;                           // lanes past n stay for the wave's adds
+    int c[3];
+    float f[3];
+    if (q < n && sort_coords(p, q, npush, g, wrap, dtdx, c, f)) {
       const bool in = c[0] >= 0 && c[1] >= 0 && c[2] >= 0 && c[0] <= g.nx && c[1] <= g.ny &&
                       c[2] <= g.nz;
       // key (cell, species): the deposit then sees runs of one cell and species
-      const int32_t cells = (int32_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
-      k = in ? (int32_t)lin_key(g, c[0], c[1], c[2]) * g.S + ((int32_t)p.sp[q] - 1) : cells * g.S;
+      k[h] = in ? (int32_t)lin_key(g, c[0], c[1], c[2]) * g.S + ((int32_t)p.sp[q] - 1) : cells * g.S;
     }
-    key[q] = k;
   }
-  wave_add1(hist, k);
+  __syncthreads();
+  {
+    const uint64_t kept = __ballot(k[0] >= 0);
+    if (threadIdx.x < 64 && kept) {      // the first wave's first kept particle
+      const int32_t kf = __builtin_amdgcn_readlane(k[0], (int)__builtin_ctzll(kept));
+      if (threadIdx.x == 0) first = kf > kFlagBack ? kf - kFlagBack : 0;
+    }
+  }
+  __syncthreads();
+  const int32_t k0 = first;
+#pragma unroll
+  for (int h = 0; h < kFlagPer; ++h) {
+    const bool near = k[h] >= k0 && k[h] - k0 < kFlagWin;
+    r[h] = -1;
+    if (near) r[h] = atomicAdd(&cnt[k[h] - k0], 1);
+    const int32_t far = wave_add1(hist, near ? -1 : k[h]);
+    if (!near) r[h] = far;
+  }
+  __syncthreads();
+  // each counted key's place in the histogram, over its count
+  for (int e = threadIdx.x; e < kFlagWin; e += kT) {
+    const int32_t m = cnt[e];
+    if (m) cnt[e] = atomicAdd(&hist[k0 + e], m);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < kFlagPer; ++h) {
+    const int64_t q = q0 + h * kT;
+    if (q >= n) continue;
+    if (k[h] >= k0 && k[h] - k0 < kFlagWin) r[h] += cnt[k[h] - k0];
+    key[q] = k[h];
+    rank[q] = r[h];
+  }
 }
 
+// Every kept particle to its place, off[key] + rank.  Bound: streaming (43 B
+// read, 35 written a particle; the places of a wave's particles are nearly one run);
+// it moves 13.3 GB in 3.15 ms at 1.4e8 particles (4.2 TB/s; a copy reaches 5.1).
 __global__ void __launch_bounds__(kT) k_sp_scatter(ParticlesSplit src, ParticlesSplit dst, int64_t n,
+                                                    int64_t npush, GridDims g, int wrap, float3 dtdx,
                                                     const int32_t *__restrict__ key,
-                                                    const int32_t *__restrict__ off,
-                                                    int32_t *__restrict__ cursor) {
+                                                    const int32_t *__restrict__ rank,
+                                                    const int32_t *__restrict__ off) {
   const int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x;
-  const int32_t k = q < n ? key[q] : -1;   // lanes past n stay for the wave's adds
-  const int32_t r = wave_add1(cursor, k);
-  if (k < 0 || r < 0) return;
-  const int64_t at = (int64_t)off[k] + r;
+  if (q >= n) return;
+  const int32_t k = key[q];
+  if (k < 0) return;
+  int c[3];
+  float f[3];
+  sort_coords(src, q, npush, g, wrap, dtdx, c, f);
+  const int64_t at = (int64_t)off[k] + rank[q];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    dst.c[d][at] = src.c[d][q];
-    dst.f[d][at] = src.f[d][q];
+    dst.c[d][at] = (int16_t)c[d];
+    dst.f[d][at] = f[d];
     dst.v[d][at] = src.v[d][q];
   }
   dst.sp[at] = src.sp[q];
@@ -2122,20 +2207,27 @@ __global__ void __launch_bounds__(kT) k_sp_to_aos(ParticlesSplit p, int64_t firs
 
 // ---------------------------------------------------------------------------
 
-int sp_sort(picard_ctx *c, int wrap) {
+static float3 push_factor(const picard_ctx *c, double dt) {
+  return make_float3((float)(dt / c->gd.dxyz[0]), (float)(dt / c->gd.dxyz[1]),
+                     (float)(dt / c->gd.dxyz[2]));
+}
+
+// The first `npush` particles are pushed by dt on the way (picard_step).
+int sp_sort(picard_ctx *c, int wrap, int64_t npush, double dt) {
   const GridDims &g = c->gd;
   const int64_t n = c->n;
   const int64_t K = c->K * g.S;           // (cell, species) keys; bucket K: out-of-grid keepers
+  const float3 dtdx = push_factor(c, dt);
   PICARD_HIP(hipMemsetAsync(c->s.hist, 0, sizeof(int32_t) * (K + 2), c->stream));
-  PICARD_HIP(hipMemsetAsync(c->s.cursor, 0, sizeof(int32_t) * (K + 1), c->stream));
   if (n > 0) {
-    k_sp_flag<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->ps, n, g, wrap, c->s.key, c->s.hist);
+    k_sp_flag<<<grid_blocks(n, kT * kFlagPer), kT, 0, c->stream>>>(c->ps, n, npush, g, wrap, dtdx,
+                                                                   c->s.key, c->s.perm, c->s.hist);
     PICARD_HIP(hipGetLastError());
   }
   PICARD_TRY(scan_exclusive_i32(c, c->s.hist, c->s.hist, K + 1));
   if (n > 0) {
-    k_sp_scatter<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->ps, c->ps2, n, c->s.key, c->s.hist,
-                                                           c->s.cursor);
+    k_sp_scatter<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->ps, c->ps2, n, npush, g, wrap, dtdx,
+                                                           c->s.key, c->s.perm, c->s.hist);
     PICARD_HIP(hipGetLastError());
   }
   PICARD_HIP(hipMemcpyAsync(c->host_counters, c->s.hist + K + 1, sizeof(int32_t),
@@ -2148,11 +2240,9 @@ int sp_sort(picard_ctx *c, int wrap) {
   return PICARD_OK;
 }
 
-int sp_push(picard_ctx *c, double dt) {
-  if (c->n <= 0) return PICARD_OK;
-  const float3 dtdx = make_float3((float)(dt / c->gd.dxyz[0]), (float)(dt / c->gd.dxyz[1]),
-                                  (float)(dt / c->gd.dxyz[2]));
-  k_sp_push<<<grid_blocks(c->n, kT), kT, 0, c->stream>>>(c->ps, c->n, dtdx);
+int sp_push(picard_ctx *c, double dt, int64_t n) {
+  if (n <= 0) return PICARD_OK;
+  k_sp_push<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->ps, n, push_factor(c, dt));
   PICARD_HIP(hipGetLastError());
   return PICARD_OK;
 }
