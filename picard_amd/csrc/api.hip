@@ -142,13 +142,12 @@ void release(picard_ctx *c) {
   dfree(c->js);
   dfree(c->s.flags);
   dfree(c->s.scan);
-  for (int q = 0; q < 6; ++q) dfree(c->s.work[q]);
+  dfree(c->s.work[0]);
   dfree(c->s.scan_tmp);
   dfree(c->s.counters);
   dfree(c->s.key);
   dfree(c->s.perm);
   dfree(c->s.hist);
-  dfree(c->s.cursor);
   dfree(c->s.stage);
   dfree(c->s.stage_sp);
   dfree(c->s.partials);
@@ -240,7 +239,10 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   if (!c->split) {
     PICARD_TRY(dalloc(&c->s.flags, cap));
     PICARD_TRY(dalloc(&c->s.scan, cap + 1));
-    for (int q = 0; q < 6; ++q) PICARD_TRY(dalloc(&c->s.work[q], cap + 1));
+    // one allocation: each pair holds cap doubles too
+    const int64_t stride = (cap + 64) / 64 * 64;
+    PICARD_TRY(dalloc(&c->s.work[0], 6 * stride));
+    for (int q = 1; q < 6; ++q) c->s.work[q] = c->s.work[0] + q * stride;
   }
   // buckets: (species, cell) keys of both deposits and of the split form's
   // sort, plus the sort's out-of-grid bucket
@@ -252,7 +254,6 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   PICARD_TRY(dalloc(&c->s.key, cap));
   PICARD_TRY(dalloc(&c->s.perm, cap));
   PICARD_TRY(dalloc(&c->s.hist, nb + 1));
-  if (!c->split) PICARD_TRY(dalloc(&c->s.cursor, nb));
   const int64_t ncell = (int64_t)g.nx * g.ny * g.nz;
   int64_t pb = grid_blocks(g.G > ncell ? g.G : ncell, 256);
   const int64_t pb3 = interior_launch(g.nx, g.ny, g.nz).blocks();

@@ -26,8 +26,8 @@ constexpr int kStencilT = 256;
 //
 // The reference accumulates N(s, node) sequentially over pp = n..1.  To get the
 // same sums bit for bit in parallel, particles are bucketed by (species, lower
-// node) and every (species, node) output merges its 8 contributing buckets in
-// descending particle index, adding in exactly the reference's order.
+// node), each bucket in descending particle index, and every (species, node) output
+// merges its 8 contributing buckets and adds in exactly the reference's order.
 
 __device__ __forceinline__ int64_t cell_key(const GridDims &g, int s0, const CicLoc &L) {
   const int64_t K = (int64_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
@@ -37,6 +37,7 @@ __device__ __forceinline__ int64_t cell_key(const GridDims &g, int s0, const Cic
 
 __global__ void __launch_bounds__(kT) k_dep_key(ParticlesF64 p, int64_t n, GridDims g,
                                                  int32_t *__restrict__ key,
+                                                 int32_t *__restrict__ rank,
                                                  int32_t *__restrict__ hist,
                                                  int32_t *__restrict__ errors) {
   const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
@@ -50,48 +51,55 @@ __global__ void __launch_bounds__(kT) k_dep_key(ParticlesF64 p, int64_t n, GridD
   }
   const int32_t k = (int32_t)cell_key(g, s0, L);
   key[i] = k;
-  atomicAdd(&hist[k], 1);
+  rank[i] = atomicAdd(&hist[k], 1);        // its place in the bucket, in no order yet
 }
 
 __global__ void __launch_bounds__(kT) k_dep_scatter(int64_t n, const int32_t *__restrict__ key,
                                                      const int32_t *__restrict__ off,
-                                                     int32_t *__restrict__ cursor,
+                                                     const int32_t *__restrict__ rank,
                                                      int32_t *__restrict__ perm) {
   const int64_t i = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (i >= n) return;
   const int32_t k = key[i];
   if (k < 0) return;
-  const int32_t pos = off[k] + atomicAdd(&cursor[k], 1);
-  perm[pos] = (int32_t)i;
+  perm[off[k] + rank[i]] = (int32_t)i;
 }
 
-// Each bucket sorted by descending particle index (insertion sort; buckets
-// hold a few dozen particles).
-__global__ void __launch_bounds__(kT) k_dep_bucket_sort(int64_t nbuckets,
-                                                         const int32_t *__restrict__ off,
-                                                         int32_t *__restrict__ perm) {
-  const int64_t b = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (b >= nbuckets) return;
-  const int32_t lo = off[b], hi = off[b + 1];
-  for (int32_t a = lo + 1; a < hi; ++a) {
-    const int32_t v = perm[a];
-    int32_t q = a - 1;
-    while (q >= lo && perm[q] < v) {
-      perm[q + 1] = perm[q];
-      --q;
-    }
-    perm[q + 1] = v;
+// Each bucket in descending particle index, one thread per particle: its place is the
+// number of greater indices in its bucket (a wave's lanes share two or three buckets, so
+// the reads are broadcasts; a thread sorting a bucket alone took 0.47 ms where this
+// takes 0.29 with the offsets, 8.4e6 particles).  REST also leaves the particle's in-cell
+// offsets there, so that they are formed once and not for each of its eight nodes.
+template <bool REST>
+__global__ void __launch_bounds__(kT) k_dep_order(ParticlesF64 p, GridDims g, int64_t nb,
+                                                   const int32_t *__restrict__ key,
+                                                   const int32_t *__restrict__ off,
+                                                   const int32_t *__restrict__ perm,
+                                                   int32_t *__restrict__ sorted,
+                                                   double *__restrict__ rx, double *__restrict__ ry,
+                                                   double *__restrict__ rz) {
+  const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (t >= off[nb]) return;
+  const int32_t q = perm[t];
+  const int32_t k = key[q], lo = off[k], hi = off[k + 1];
+  int32_t at = lo;
+  for (int32_t a = lo; a < hi; ++a) at += perm[a] > q;
+  sorted[at] = q;
+  if (REST) {
+    const CicLoc L = cic_locate(g, p.r[0][q], p.r[1][q], p.r[2][q]);
+    rx[at] = L.rest[0];
+    ry[at] = L.rest[1];
+    rz[at] = L.rest[2];
   }
 }
 
 // One thread per (node, species): 8-way merge by descending particle index.
-// FLUX also accumulates the number fluxes of ParticlesGridifyAll
-// (ParticlesGridifyAll.f90:126-212), F(s, c, node) += F_k n2p(s) v_c, in the
-// same order; Fraw is laid out (s fastest, then c, then node).
-template <bool FLUX>
+// With the number fluxes of ParticlesGridifyAll (ParticlesGridifyAll.f90:126-212), F(s, c,
+// node) += F_k n2p(s) v_c, in the same order; Fraw is laid out (s fastest, then c,
+// then node).
 __global__ void __launch_bounds__(kT) k_dep_gather(ParticlesF64 p, GridDims g, const double *n2p,
                                                     const int32_t *__restrict__ off,
-                                                    const int32_t *__restrict__ perm,
+                                                    const int32_t *__restrict__ sorted,
                                                     double *__restrict__ Nraw,
                                                     double *__restrict__ Fraw) {
   const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
@@ -126,7 +134,7 @@ __global__ void __launch_bounds__(kT) k_dep_gather(ParticlesF64 p, GridDims g, c
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
       if (head[o] < end[o]) {
-        const int32_t pp = perm[head[o]];
+        const int32_t pp = sorted[head[o]];
         if (pp > bestp) {
           bestp = pp;
           best = o;
@@ -143,16 +151,213 @@ __global__ void __launch_bounds__(kT) k_dep_gather(ParticlesF64 p, GridDims g, c
     const double fz = (best & 4) ? L.rest[2] : L.drest[2];
     const double F = fx * fy * fz / g.dV;
     acc = acc + F * w;
-    if (FLUX) {
-      const double Fw = F * w;
-      fl[0] = fl[0] + Fw * p.r[3][bestp];
-      fl[1] = fl[1] + Fw * p.r[4][bestp];
-      fl[2] = fl[2] + Fw * p.r[5][bestp];
-    }
+    const double Fw = F * w;
+    fl[0] = fl[0] + Fw * p.r[3][bestp];
+    fl[1] = fl[1] + Fw * p.r[4][bestp];
+    fl[2] = fl[2] + Fw * p.r[5][bestp];
   }
   Nraw[node * g.S + s0] = acc;
-  if (FLUX)
-    for (int c = 0; c < 3; ++c) Fraw[(node * 3 + c) * g.S + s0] = fl[c];
+  for (int c = 0; c < 3; ++c) Fraw[(node * 3 + c) * g.S + s0] = fl[c];
+}
+
+// Without the fluxes a block takes one species' nodes i0.. of one row (j, k).  Their
+// cells are four rows' (j - 1 | j, k - 1 | k), each row one contiguous stretch of the
+// sorted particles.  The four buckets of one x are a column; node n takes columns n and
+// n + 1.  A particle's place among its column's is its place in its own bucket plus
+// the number of greater indices in the other three, found by bisection (they descend); its
+// place among a node's is that plus the number of greater ones in the other column. Its two weights
+// go to those places in LDS, and a lane per node adds them in order.  All of it reads
+// contiguous memory.  Bound: LDS latency, so many small blocks; 0.64 ms for 8.4e6 particles, 16
+// a cell and species, where one thread per node with 64 lanes at 512 places took 4.39.
+// Whole deposits at 8, 32, 64 and 128 a cell and species on 48^3: 0.27, 1.24, 3.2, 12.6 ms
+// against 0.71, 6.6, 17.6, 44.6; with half the particles held 0.26, 1.34, 5.1, 12.7, with
+// twice as many the first two are slower by half.
+constexpr int kRowSeg = 64;              // nodes of a block at most: one wave adds them
+constexpr int kRowCap = 1024;            // particles in LDS: 30 KB, five blocks per CU
+
+// entries of d[lo .. hi), descending, greater than q
+__device__ __forceinline__ int greater_in(const int32_t *d, int lo, int hi, int32_t q) {
+  const int first = lo;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (d[mid] > q) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo - first;
+}
+
+// F1..F8 of ParticlesGridify.f90:81-88: node offset 1 takes rest, 0 takes dx - rest
+__device__ __forceinline__ double dep_weight(const GridDims &g, bool ox, bool oy, bool oz, double x,
+                                             double y, double z) {
+  const double fx = ox ? x : g.dxyz[0] - x;
+  const double fy = oy ? y : g.dxyz[1] - y;
+  const double fz = oz ? z : g.dxyz[2] - z;
+  return fx * fy * fz / g.dV;
+}
+
+__global__ void __launch_bounds__(kT) k_dep_rows(GridDims g, int seg, int nseg, int64_t blocks,
+                                                  const double *n2p,
+                                                  const int32_t *__restrict__ off,
+                                                  const int32_t *__restrict__ sorted,
+                                                  const double *__restrict__ rx,
+                                                  const double *__restrict__ ry,
+                                                  const double *__restrict__ rz,
+                                                  double *__restrict__ Nraw) {
+  __shared__ int32_t own[kRowCap], col[kRowCap];
+  __shared__ int16_t place[kRowCap], cellof[kRowCap];
+  __shared__ double val[2 * kRowCap + kRowSeg];
+  __shared__ int32_t H[8], B[9];         // a lone node's buckets
+  __shared__ int32_t E[4][kRowSeg + 2];  // first sorted particle of row r's cell m
+  __shared__ int32_t C[kRowSeg + 2];     // particles of the columns before m
+  // neighbouring rows on one XCD: they share half their cells
+  const int64_t per = (blocks + 7) / 8;
+  const int64_t v = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (v >= blocks) return;
+  const int i0 = (int)(v % nseg) * seg + 1;
+  const int nn = min(seg, g.X - i0 + 1);
+  int64_t row = v / nseg;
+  const int j = (int)(row % g.Y) + 1;
+  row /= g.Y;
+  const int k = (int)(row % g.Z) + 1;
+  const int s0 = (int)(row / g.Z);
+  const int64_t K = (int64_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
+  const int lane = threadIdx.x & 63;
+  // row r: cells (j - (r & 1), k - (r >> 1)); cell m: x = i0 - 1 + m; those outside are empty
+  for (int e = threadIdx.x; e < 4 * (nn + 2); e += kT) {
+    const int r = e / (nn + 2), m = e % (nn + 2);
+    const int cj = j - (r & 1), ck = k - (r >> 1);
+    int32_t o = 0;
+    if (cj >= 1 && ck >= 1 && cj <= g.ny + 1 && ck <= g.nz + 1) {
+      const int64_t b = (int64_t)s0 * K + (int64_t)(g.nx + 1) * ((cj - 1) + (int64_t)(g.ny + 1) * (ck - 1));
+      o = off[b + min(max(i0 - 2 + m, 0), g.nx + 1)];
+    }
+    E[r][m] = o;
+  }
+  __syncthreads();
+  for (int m = threadIdx.x; m < nn + 2; m += kT)
+    C[m] = (E[0][m] - E[0][0]) + (E[1][m] - E[1][0]) + (E[2][m] - E[2][0]) + (E[3][m] - E[3][0]);
+  __syncthreads();
+  const double w = n2p[s0];
+  int n0 = 0;
+  while (n0 < nn) {
+    // as many nodes as fit
+    const int fit = (int)__popcll(__ballot(lane >= n0 && lane < nn && C[lane + 2 <= nn + 1 ? lane + 2 : 0] - C[n0] <= kRowCap));
+    if (fit == 0) {
+      // A node of more particles than fit, alone: its eight buckets (lane l: row l & 3 of
+      // cell n0 + (l >> 2)) in stretches.  No bucket gives more than kRowCap / 8 and all
+      // give down to the same index, the greatest that any holds after that many.
+      const int l0 = lane & 7, m0 = n0 + (l0 >> 2);
+      int32_t head = E[l0 & 3][m0];
+      const int32_t end = E[l0 & 3][m0 + 1];
+      double acc = 0.0;
+      for (;;) {
+        if (threadIdx.x < 64) {
+          int32_t pivot = end - head > kRowCap / 8 ? sorted[head + kRowCap / 8] : -1;
+          for (int o = 1; o < 8; o <<= 1) pivot = max(pivot, __shfl_xor(pivot, o));
+          const int take = greater_in(sorted, head, min(head + kRowCap / 8, end), pivot);
+          int before = 0;
+          for (int o = 0; o < 8; ++o) {
+            const int t = __shfl(take, o);
+            if (o < l0) before += t;
+          }
+          if (lane < 8) {
+            H[l0] = head;
+            B[l0] = before;
+            if (l0 == 7) B[8] = before + take;
+          }
+          head += take;
+        }
+        __syncthreads();
+        const int tot = B[8];
+        if (tot == 0) break;
+        auto bucket = [&](int e) {
+          int l = 0;
+          for (int o = 1; o < 8; ++o) l += e >= B[o];
+          return l;
+        };
+        for (int e = threadIdx.x; e < tot; e += kT) {
+          const int l = bucket(e);
+          own[e] = sorted[H[l] + (e - B[l])];
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < tot; e += kT) {
+          const int l = bucket(e);
+          const int32_t a = H[l] + (e - B[l]), q = own[e];
+          int t = e - B[l];
+          for (int o = 1; o < 8; ++o) t += greater_in(own, B[l ^ o], B[(l ^ o) + 1], q);
+          val[t] = dep_weight(g, l < 4, l & 1, l & 2, rx[a], ry[a], rz[a]) * w;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0)
+          for (int t = 0; t < tot; ++t) acc = acc + val[t];
+      }
+      if (threadIdx.x == 0) Nraw[node_index(g, i0 + n0, j, k) * g.S + s0] = acc;
+      __syncthreads();
+      ++n0;
+      continue;
+    }
+    const int n1 = n0 + fit;             // nodes n0 .. n1 - 1, cells n0 .. n1
+    const int c0 = C[n0], tot = C[n1 + 1] - c0;
+    int rb[5];
+    rb[0] = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rb[r + 1] = rb[r] + (E[r][n1 + 1] - E[r][n0]);
+    for (int e = threadIdx.x; e < tot; e += kT) {
+      const int r = (e >= rb[1]) + (e >= rb[2]) + (e >= rb[3]);
+      own[e] = sorted[E[r][n0] + (e - rb[r])];
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < tot; e += kT) {
+      const int r = (e >= rb[1]) + (e >= rb[2]) + (e >= rb[3]);
+      const int a = E[r][n0] + (e - rb[r]);
+      int lo = n0, hi = n1;              // last cell with E[r][m] <= a
+      while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (E[r][mid] <= a) lo = mid;
+        else hi = mid - 1;
+      }
+      const int m = lo;
+      const int32_t q = own[e];
+      int at = C[m] - c0 + (a - E[r][m]);
+#pragma unroll
+      for (int o = 1; o < 4; ++o) {
+        const int r2 = r ^ o;
+        const int b2 = rb[r2] - E[r2][n0];
+        at += greater_in(own, b2 + E[r2][m], b2 + E[r2][m + 1], q);
+      }
+      col[at] = q;
+      place[e] = (int16_t)at;
+      cellof[e] = (int16_t)m;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < tot; e += kT) {
+      const int r = (e >= rb[1]) + (e >= rb[2]) + (e >= rb[3]);
+      const int a = E[r][n0] + (e - rb[r]);
+      const double x = rx[a], y = ry[a], z = rz[a];
+      const int m = cellof[e], at = place[e] - (C[m] - c0);
+      const int32_t q = own[e];
+#pragma unroll
+      for (int o = 0; o < 2; ++o) {
+        const int n = m - 1 + o, m2 = o ? m + 1 : m - 1;       // the node, its other column
+        if (n < n0 || n >= n1) continue;
+        const int t = at + greater_in(col, C[m2] - c0, C[m2 + 1] - c0, q);
+        // the nodes' sums before this one's, and one place between nodes for the banks
+        val[C[n + 1] - C[n0 + 1] + C[n] - c0 + (n - n0) + t] =
+            dep_weight(g, o, r & 1, r & 2, x, y, z) * w;
+      }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < fit) {
+      const int n = n0 + threadIdx.x;
+      const double *vals = &val[C[n + 1] - C[n0 + 1] + C[n] - c0 + threadIdx.x];
+      const int cnt = C[n + 2] - C[n];
+      double acc = 0.0;                  // N = 0.0d0 (ParticlesGridify.f90:59)
+      for (int t = 0; t < cnt; ++t) acc = acc + vals[t];
+      Nraw[node_index(g, i0 + n, j, k) * g.S + s0] = acc;
+    }
+    __syncthreads();
+    n0 = n1;
+  }
 }
 
 // Guard handling of one dimension on one rank (ParticlesGridify.f90:129-285):
@@ -1148,30 +1353,41 @@ int launch_gridify(picard_ctx *c, bool flux) {
   const int64_t n = c->n;
   const int64_t nb = (int64_t)g.S * c->K;
   PICARD_HIP(hipMemsetAsync(c->s.hist, 0, sizeof(int32_t) * (nb + 1), c->stream));
-  PICARD_HIP(hipMemsetAsync(c->s.cursor, 0, sizeof(int32_t) * nb, c->stream));
   PICARD_HIP(hipMemsetAsync(c->s.counters, 0, sizeof(int32_t), c->stream));
   if (n > 0) {
-    k_dep_key<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, n, g, c->s.key, c->s.hist,
+    k_dep_key<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, n, g, c->s.key, c->s.scan, c->s.hist,
                                                         c->s.counters);
     PICARD_HIP(hipGetLastError());
   }
   PICARD_TRY(scan_exclusive_i32(c, c->s.hist, c->s.hist, nb));
+  // the outflow's scratch, free here: the sorted indices and, over pairs of
+  // its int32 arrays, the in-cell offsets
+  int32_t *sorted = c->s.flags;
+  double *rest[3];
+  for (int d = 0; d < 3; ++d) rest[d] = reinterpret_cast<double *>(c->s.work[2 * d]);
   if (n > 0) {
-    k_dep_scatter<<<grid_blocks(n, kT), kT, 0, c->stream>>>(n, c->s.key, c->s.hist, c->s.cursor,
+    k_dep_scatter<<<grid_blocks(n, kT), kT, 0, c->stream>>>(n, c->s.key, c->s.hist, c->s.scan,
                                                             c->s.perm);
     PICARD_HIP(hipGetLastError());
-    k_dep_bucket_sort<<<grid_blocks(nb, kT), kT, 0, c->stream>>>(nb, c->s.hist, c->s.perm);
+    if (flux)
+      k_dep_order<false><<<grid_blocks(n, kT), kT, 0, c->stream>>>(
+          c->p, g, nb, c->s.key, c->s.hist, c->s.perm, sorted, nullptr, nullptr, nullptr);
+    else
+      k_dep_order<true><<<grid_blocks(n, kT), kT, 0, c->stream>>>(
+          c->p, g, nb, c->s.key, c->s.hist, c->s.perm, sorted, rest[0], rest[1], rest[2]);
     PICARD_HIP(hipGetLastError());
   }
   if (flux) {
     PICARD_TRY(ensure_flux(c));
-    k_dep_gather<true><<<grid_blocks(g.G * g.S, kT), kT, 0, c->stream>>>(
-        c->p, g, c->consts, c->s.hist, c->s.perm, c->Nraw, c->Fraw);
+    k_dep_gather<<<grid_blocks(g.G * g.S, kT), kT, 0, c->stream>>>(
+        c->p, g, c->consts, c->s.hist, sorted, c->Nraw, c->Fraw);
     PICARD_HIP(hipGetLastError());
     k_fold_flux<<<grid_blocks(g.G, kT), kT, 0, c->stream>>>(g, c->Fraw, c->F);
   } else {
-    k_dep_gather<false><<<grid_blocks(g.G * g.S, kT), kT, 0, c->stream>>>(
-        c->p, g, c->consts, c->s.hist, c->s.perm, c->Nraw, nullptr);
+    const int nseg = (g.X + kRowSeg - 1) / kRowSeg, seg = (g.X + nseg - 1) / nseg;
+    const int64_t blocks = (int64_t)nseg * g.Y * g.Z * g.S;
+    k_dep_rows<<<(unsigned)((blocks + 7) / 8 * 8), kT, 0, c->stream>>>(
+        g, seg, nseg, blocks, c->consts, c->s.hist, sorted, rest[0], rest[1], rest[2], c->Nraw);
   }
   PICARD_HIP(hipGetLastError());
   k_fold_charge<<<grid_blocks(g.G, kT), kT, 0, c->stream>>>(g, c->Nraw, c->N, c->C,

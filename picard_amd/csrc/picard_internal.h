@@ -90,7 +90,8 @@ struct DeviceScratch {
   // generic
   int32_t *flags = nullptr;        // per particle
   int32_t *scan = nullptr;         // per particle (+1)
-  int32_t *work[6] = {};           // per particle each: outflow rotation/stream buffers
+  int32_t *work[6] = {};           // per particle each, one allocation: outflow rotation/stream
+                                   // buffers; in the deposit each pair an array of doubles
   int32_t *scan_tmp = nullptr;     // block sums of the recursive scan
   int64_t scan_tmp_len = 0;
   int32_t *counters = nullptr;     // small device counters (errors, totals)
@@ -98,7 +99,6 @@ struct DeviceScratch {
   int32_t *key = nullptr;          // per particle
   int32_t *perm = nullptr;         // per particle (split form: rank within its key)
   int32_t *hist = nullptr;         // S*K + 1
-  int32_t *cursor = nullptr;       // S*K (FP64 forms)
   // staging for uploads/downloads (AoS)
   double *stage = nullptr;
   int32_t *stage_sp = nullptr;
