@@ -9,6 +9,7 @@
 #include <string>
 
 #include "picard_internal.h"
+#include "readback.h"
 #include "sched.h"
 
 namespace picard {
@@ -155,6 +156,8 @@ void release(picard_ctx *c) {
   c->tev.clear();
   for (hipEvent_t &e : c->solve_ev)
     if (e) (void)hipEventDestroy(e), e = nullptr;
+  delete c->readback;
+  c->readback = nullptr;
   if (c->js_host) (void)hipHostFree(c->js_host);
   if (c->host_counters) (void)hipHostFree(c->host_counters);
   c->js_host = nullptr;
@@ -263,6 +266,8 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   c->s.partials_len = pb;
   PICARD_TRY(dalloc(&c->s.partials, 4 * pb));     // two launches' worth (read + write) and scratch
   PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->js_host), sizeof(JacobiState)));
+  // allocating its chunks, 0.25 ms each pair, is worth it from a few MB on
+  c->readback = new Readback(int64_t(4) << 20);
   PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->host_counters), 16 * sizeof(int32_t)));
   // the reference zeroes U, N, E and the particle arrays at start (picard.f90:434-439)
   PICARD_HIP(hipMemsetAsync(c->U, 0, sizeof(double) * g.G, c->stream));
@@ -578,11 +583,14 @@ int picard_field_read(picard_ctx *c, int32_t which, double *host, int64_t count)
     set_error("field_read: unknown field or wrong element count");
     return PICARD_ERR_ARG;
   }
-  if (c->split && which == PICARD_FIELD_E) PICARD_TRY(sp_widen_e(c));
-  PICARD_HIP(hipMemcpyAsync(host, field_ptr(c, which), sizeof(double) * len,
-                            hipMemcpyDeviceToHost, c->stream));
-  PICARD_HIP(hipStreamSynchronize(c->stream));
-  return PICARD_OK;
+  if (c->split && which == PICARD_FIELD_E) {
+    bool taken = false;
+    PICARD_TRY(c->readback->widen(c->device, c->stream, host, reinterpret_cast<const float4 *>(c->E32),
+                                  c->gd.G, &taken));
+    if (taken) return PICARD_OK;
+    PICARD_TRY(sp_widen_e(c));
+  }
+  return c->readback->copy(c->device, c->stream, host, field_ptr(c, which), sizeof(double) * len);
 }
 
 int picard_field_write(picard_ctx *c, int32_t which, const double *host, int64_t count) {

@@ -48,6 +48,7 @@
 
 #include "../../include/picard_ensemble.h"
 #include "picard_internal.h"
+#include "readback.h"
 #include "reduce.h"
 #include "rng.h"
 #include "spectral.h"
@@ -1613,6 +1614,8 @@ struct picard_ensemble {
   int device = 0;
   int cus = 256;
   hipStream_t stream = nullptr;
+  // the simulations share its chunks; 0.05 MB takes the runtime 14 us, and 27 through one
+  Readback readback{int64_t(1) << 16};
   Arenas A{};
   PartArena P[2]{};
   int cur = 0;                       // arena holding the sorted particles
@@ -2544,19 +2547,16 @@ int picard_ensemble_field_read(picard_ensemble *e, int32_t slot, int32_t which, 
   else if (which == PICARD_FIELD_C) src = e->A.C + h.g.off;
   else if (which == PICARD_FIELD_N) src = e->A.N + 2 * h.g.off;
   else {
+    bool taken = false;
+    PICARD_TRY(e->readback.widen(e->device, e->stream, host, e->A.E32 + h.g.off, G, &taken));
+    if (taken) return PICARD_OK;
     PICARD_HIP(hipMalloc(reinterpret_cast<void **>(&tmp), sizeof(double) * 3 * G));
     k_widen<<<256, kT, 0, e->stream>>>(e->A.E32 + h.g.off, G, tmp);
     src = tmp;
   }
-  const hipError_t ec = hipMemcpyAsync(host, src, sizeof(double) * want, hipMemcpyDeviceToHost,
-                                       e->stream);
-  const hipError_t es = hipStreamSynchronize(e->stream);
+  const int rc = e->readback.copy(e->device, e->stream, host, src, sizeof(double) * want);
   if (tmp) (void)hipFree(tmp);
-  if (ec != hipSuccess || es != hipSuccess) {
-    set_error("picard_ensemble_field_read: copy failed");
-    return PICARD_ERR_HIP;
-  }
-  return PICARD_OK;
+  return rc;
 }
 
 int picard_ensemble_particles_read(picard_ensemble *e, int32_t slot, double *rp, int32_t *sp,

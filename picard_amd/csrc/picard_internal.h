@@ -109,6 +109,7 @@ struct DeviceScratch {
 };
 
 struct SpecState;                  // spectral.hip
+class Readback;                    // readback.h
 
 }  // namespace picard
 
@@ -193,6 +194,7 @@ struct picard_ctx {
 
   picard::JacobiState *js = nullptr;   // device
   picard::JacobiState *js_host = nullptr;   // pinned mirror
+  picard::Readback *readback = nullptr;
   int32_t *host_counters = nullptr;    // pinned mirror of scratch.counters
 
   picard::DeviceScratch s;

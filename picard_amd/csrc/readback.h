@@ -1,0 +1,37 @@
+// readback.h -- device arrays to pageable host memory through pinned chunks,
+// several host threads copying out of them.
+#pragma once
+#include <mutex>
+
+#include "picard_internal.h"
+
+namespace picard {
+
+class Readback {
+ public:
+  // arrays of fewer than `direct` bytes go the runtime's way
+  explicit Readback(int64_t direct) : direct_(direct) {}
+  ~Readback();
+  // host[0 .. bytes) = dev, in the stream's order; returns when it is there
+  int copy(int device, hipStream_t stream, void *host, const void *dev, int64_t bytes);
+  // host[3 q + d] = component d of E[q], q < n.  *taken = false, and nothing done, for
+  // few and where `host` is memory that the GPU reaches itself.
+  int widen(int device, hipStream_t stream, double *host, const float4 *E, int64_t n, bool *taken);
+
+ private:
+  static constexpr int kMaxWorkers = 6;
+  struct Worker {
+    char *pin[2] = {nullptr, nullptr};
+    hipEvent_t ev[2] = {nullptr, nullptr};
+  };
+  template <typename OUT>
+  int run(int device, hipStream_t stream, const char *dev, int64_t bytes, const OUT &out);
+  template <typename OUT>
+  hipError_t work(Worker &w, int device, hipStream_t stream, const char *dev, int64_t bytes,
+                  int64_t chunk, int first, int step, const OUT &out);
+  const int64_t direct_;
+  std::mutex mu_;
+  Worker w_[kMaxWorkers];
+};
+
+}  // namespace picard
