@@ -49,6 +49,7 @@
 #include "../../include/picard_ensemble.h"
 #include "picard_internal.h"
 #include "readback.h"
+#include "split_particles.h"
 #include "reduce.h"
 #include "rng.h"
 #include "spectral.h"
@@ -57,8 +58,6 @@ namespace picard {
 namespace ens {
 
 constexpr int kT = 256;
-constexpr double kFix = 1099511627776.0;      // 2^40: deposit weights
-constexpr double kFixInv = 1.0 / 1099511627776.0;
 constexpr unsigned long long kStopUnits = 1ull << 40;   // the threshold in residual units
 constexpr double kTau = 6.2831853071795864769252867665590;
 constexpr double kEC = 1.60217646e-19, kMP = 1.6726216e-27, kME = 9.1093819e-31;
@@ -161,7 +160,8 @@ struct Arenas {
   unsigned long long *Nfix;
   float4 *E32;
   float *r32, *e32[kEBufs];
-  int32_t *hist, *cursor, *key;
+  int32_t *hist;
+  int32_t *rank;            // per particle: its place among those of its key
   int64_t kcap;             // key capacity
   // eigenbasis solve: three buffers, tiles {slot, first element, index}, product
   // tiles {slot, first output, first column} per axis, partial sums per tile
@@ -289,125 +289,93 @@ __global__ void k_inflow_commit(Arenas A, int64_t cap) {
   g->n += g->inflow_total;
 }
 
-// AdvancePosition on the split coordinates: xi += v dt/dx.
-__device__ __forceinline__ int carry(float &f) {
-  const float fl = floorf(f);
-  f = f - fl;
-  int c = (int)fl;
-  if (f >= 1.0f) {
-    f = 0.0f;
-    c += 1;
-  }
-  return c;
-}
-
-__global__ void __launch_bounds__(kT) k_push(Arenas A, PartArena p) {
-  const int64_t n = A.g->n;
-  for (int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x; q < n; q += (int64_t)gridDim.x * kT) {
-    const float dtdx = A.sims[p.sim[q]].dtdx;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      float f = p.f[d][q] + p.v[d][q] * dtdx;
-      p.c[d][q] = (int16_t)(p.c[d][q] + carry(f));
-      p.f[d][q] = f;
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// sort: BCoutflow (x faces, and the band one domain width out in every
+// sort: AdvancePosition on the split coordinates (xi += v dt/dx), BCoutflow (x faces,
+// and the band one domain width out in every
 // dimension, BCoutflow.f90:28-66) and ParticlesTransfer's periodic wrap of y
-// and z (ParticlesTransfer.f90:494-519) on the split coordinates, then a
+// and z (ParticlesTransfer.f90:494-519), then a
 // counting sort over every slot's key range.  Particles of slots that left
-// are dropped.
+// are dropped.  Both passes form a particle's cell and key, so that only its rank is
+// kept between them: 35 bytes read and 4 written, then 39 read and 37 written.  24
+// simulations of 16^3-64^3: 3.02 ms as push, flag and scatter with a wave's atomics
+// in both, now 2.37.
 
-__device__ __forceinline__ bool below(int c, float f) { return c < 0 || (c == 0 && f < 0.5f); }
-__device__ __forceinline__ bool above(int c, float f, int n) { return c > n || (c == n && f > 0.5f); }
-
-// One atomic per distinct key and wave: the lanes sharing the leader's key
-// take ranks by lane order after the value the leader's add returned.  Every
-// lane stays in the loop (its condition is the wave-uniform pending mask).
-__device__ __forceinline__ int32_t wave_add1(int32_t *counter, int32_t k) {
-  const int lane = lane_id();
-  bool pending = k >= 0;
-  int32_t ret = -1;
-  uint64_t todo = __ballot(pending);
-  while (todo) {
-    const int leader = (int)__builtin_ctzll(todo);
-    const int32_t kl = __builtin_amdgcn_readlane(k, leader);
-    const bool mine = pending && k == kl;
-    const uint64_t m = __ballot(mine) | (1ull << leader);
-    int32_t base = 0;
-    if (lane == leader) base = atomicAdd(&counter[kl], (int32_t)__popcll(m));
-    base = __builtin_amdgcn_readlane(base, leader);
-    if (mine) {
-      ret = base + (int32_t)__popcll(m & ((1ull << lane) - 1ull));
-      pending = false;
-    }
-    todo &= ~m;
+// Cell, offset and key of particle q after the push: false if it is dropped, with
+// *lost if it left its grid.
+__device__ __forceinline__ bool sort_particle(const Arenas &A, const PartArena &p, int64_t q,
+                                              int (&c)[3], float (&f)[3], int32_t &k, bool *lost) {
+  const SimDev &sd = A.sims[p.sim[q]];
+  if (!sd.live) return false;
+  const int nn[3] = {sd.nx, sd.ny, sd.nz};
+  float v[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    c[d] = p.c[d][q];
+    f[d] = p.f[d][q];
+    v[d] = p.v[d][q];
   }
-  return ret;
+  push_one(c, f, v, make_float3(sd.dtdx, sd.dtdx, sd.dtdx));
+  bool del = below(c[0], f[0]) || above(c[0], f[0], nn[0]);            // x in/outflow
+#pragma unroll
+  for (int d = 0; d < 3; ++d)
+    if (below(c[d] + nn[d], f[d]) || above(c[d] - nn[d], f[d], nn[d])) del = true;
+  if (del) return false;
+#pragma unroll
+  for (int d = 2; d >= 1; --d) {                     // z then y (x is not periodic)
+    if (below(c[d], f[d])) c[d] += nn[d];
+    if (above(c[d], f[d], nn[d])) c[d] -= nn[d];
+  }
+  if (!(c[0] >= 0 && c[1] >= 0 && c[2] >= 0 && c[0] <= nn[0] && c[1] <= nn[1] && c[2] <= nn[2])) {
+    *lost = true;
+    return false;
+  }
+  const int32_t lin = c[0] + (sd.nx + 1) * (c[1] + (sd.ny + 1) * c[2]);
+  k = sd.kbase + 2 * lin + ((int32_t)p.sp[q] - 1);
+  return true;
 }
 
 __global__ void __launch_bounds__(kT) k_flag(Arenas A, PartArena p) {
+  __shared__ KeyWindow win;
   const int64_t n = A.g->n;
-  int nerr = 0;
-  // block-uniform trip count: every lane of a wave takes part in wave_add1
-  for (int64_t b0 = (int64_t)blockIdx.x * kT; b0 < n; b0 += (int64_t)gridDim.x * kT) {
-    const int64_t q = b0 + threadIdx.x;
-    int32_t k = -1;
-    if (q < n) {
-      const int slot = p.sim[q];
-      const SimDev &sd = A.sims[slot];
-      if (sd.live) {
-        const int nn[3] = {sd.nx, sd.ny, sd.nz};
-        int c[3] = {p.c[0][q], p.c[1][q], p.c[2][q]};
-        const float f[3] = {p.f[0][q], p.f[1][q], p.f[2][q]};
-        bool del = below(c[0], f[0]) || above(c[0], f[0], nn[0]);      // x in/outflow
+  bool lost = false;
+  for (int64_t b0 = (int64_t)blockIdx.x * (kT * kFlagPer); b0 < n;
+       b0 += (int64_t)gridDim.x * (kT * kFlagPer)) {             // block-uniform
+    int32_t k[kFlagPer], r[kFlagPer];
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-          if (below(c[d] + nn[d], f[d]) || above(c[d] - nn[d], f[d], nn[d])) del = true;
-        if (!del) {
-#pragma unroll
-          for (int d = 2; d >= 1; --d) {           // z then y (x is not periodic)
-            if (below(c[d], f[d])) c[d] += nn[d];
-            if (above(c[d], f[d], nn[d])) c[d] -= nn[d];
-          }
-          if (c[0] >= 0 && c[1] >= 0 && c[2] >= 0 && c[0] <= nn[0] && c[1] <= nn[1] &&
-              c[2] <= nn[2]) {
-            p.c[1][q] = (int16_t)c[1];
-            p.c[2][q] = (int16_t)c[2];
-            const int32_t lin = c[0] + (sd.nx + 1) * (c[1] + (sd.ny + 1) * c[2]);
-            k = sd.kbase + 2 * lin + ((int32_t)p.sp[q] - 1);
-          } else {
-            ++nerr;
-          }
-        }
-      }
-      A.key[q] = k;
+    for (int h = 0; h < kFlagPer; ++h) {
+      const int64_t q = b0 + h * kT + threadIdx.x;
+      int c[3];
+      float f[3];
+      k[h] = -1;
+      if (q < n) (void)sort_particle(A, p, q, c, f, k[h], &lost);
     }
-    wave_add1(A.hist, k);
+    count_keys(k, r, A.hist, win);
+#pragma unroll
+    for (int h = 0; h < kFlagPer; ++h) {
+      const int64_t q = b0 + h * kT + threadIdx.x;
+      if (q < n) A.rank[q] = r[h];
+    }
   }
-  if (nerr) atomicOr(&A.g->err, 2);
+  if (lost) atomicOr(&A.g->err, 2);
 }
 
 // One particle per thread over a grid sized for the arena's capacity (the
 // count is in device memory, so the captured launch cannot size itself to
-// it): blocks past the count leave at once, and every wave in range walks a
-// single key-cursor-copy chain instead of hundreds in a grid-stride loop.
+// it): blocks past the count leave at once.
 __global__ void __launch_bounds__(kT) k_scatter(Arenas A, PartArena src, PartArena dst) {
   const int64_t n = A.g->n;
-  const int64_t b0 = (int64_t)blockIdx.x * kT;
-  if (b0 >= n) return;                                   // block-uniform
-  const int64_t q = b0 + threadIdx.x;
-  const int32_t k = q < n ? A.key[q] : -1;               // lanes past n take part in the adds
-  const int32_t r = wave_add1(A.cursor, k);
-  if (k < 0 || r < 0) return;
-  const int64_t at = (int64_t)A.hist[k] + r;
+  const int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (q >= n) return;
+  int c[3];
+  float f[3];
+  int32_t k;
+  bool lost = false;
+  if (!sort_particle(A, src, q, c, f, k, &lost)) return;
+  const int64_t at = (int64_t)A.hist[k] + A.rank[q];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    dst.c[d][at] = src.c[d][q];
-    dst.f[d][at] = src.f[d][q];
+    dst.c[d][at] = (int16_t)c[d];
+    dst.f[d][at] = f[d];
     dst.v[d][at] = src.v[d][q];
   }
   dst.sp[at] = src.sp[q];
@@ -433,24 +401,27 @@ __global__ void k_ranges(Arenas A) {
 // deposit (ParticlesGridify.f90:59-121): int64 fixed point, runs of one
 // (slot, cell, species) summed in registers, one atomic per corner and run.
 
-constexpr int kDepChunk = 16;
+constexpr int kDepChunk = 8;
+constexpr int kDepRounds = 2;
 constexpr int kDepSeg = 128;          // nodes per LDS segment of the deposit
 
 // A thread adds the fixed-point weights of each run of one (cell, species)
-// among its kDepChunk sorted particles in registers and flushes one add per
+// among its kDepChunk sorted particles, loaded 16 bytes at a time so that a wave's
+// loads are contiguous, in registers and flushes one add per
 // corner when the run ends.  The adds are staged in LDS per block chunk of
-// kT * kDepChunk particles: from the chunk's first particle (slot s0, lower
+// kDepRounds * kT * kDepChunk particles: from the chunk's first particle (slot s0, lower
 // node b0) the corners of runs of the same slot with lower nodes in [b0, b0 +
 // kDepSeg - 1) fall in four node segments b0 + {0, X, XY, XY + X} + [0,
 // kDepSeg), added with LDS atomics; other runs go straight to memory.  The
 // block then adds each nonzero segment entry to memory once.  Integer sums:
-// the same result as one atomic per particle.
+// the same result as one atomic per particle.  24 simulations of 16^3-64^3: 1.90 ms
+// reading a particle at a time, now 0.39.
 __global__ void __launch_bounds__(kT) k_deposit(Arenas A, PartArena p) {
   __shared__ unsigned long long seg[4 * kDepSeg * 2];
   __shared__ int64_t seg_b0;
   __shared__ int seg_slot;
   const int64_t n = A.g->n;
-  const int64_t span = (int64_t)kT * kDepChunk;
+  const int64_t span = (int64_t)kT * kDepChunk * kDepRounds;
   for (int64_t cb = (int64_t)blockIdx.x * span; cb < n; cb += (int64_t)gridDim.x * span) {
     if (threadIdx.x == 0) {
       int slot0 = -1;
@@ -469,11 +440,10 @@ __global__ void __launch_bounds__(kT) k_deposit(Arenas A, PartArena p) {
     __syncthreads();
     const int slot0 = seg_slot;
     const int64_t b0 = seg_b0;
-    const int64_t q0 = cb + (int64_t)threadIdx.x * kDepChunk;
-    const int64_t q1 = q0 + kDepChunk < n ? q0 + kDepChunk : n;    // empty past n
     int64_t cur = -1;
-    int cur_s = 0, cur_slot = -1;
-    int64_t X = 0, XY = 0;
+    int cur_s = 0, cur_slot = -1;       // slot of the geometry below, and of the run
+    int nx = 0, ny = 0, nz = 0;
+    int64_t X = 0, XY = 0, gbase = 0;
     unsigned long long W[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     auto flush = [&]() {
       if (cur < 0) return;
@@ -484,37 +454,57 @@ __global__ void __launch_bounds__(kT) k_deposit(Arenas A, PartArena p) {
           atomicAdd(&seg[((o >> 1) * kDepSeg + off + (o & 1)) * 2 + cur_s], W[o]);
           W[o] = 0;
         }
-        return;
-      }
+      } else {
 #pragma unroll
-      for (int o = 0; o < 8; ++o) {
-        const int64_t node = cur + (o & 1) + X * ((o >> 1) & 1) + XY * (o >> 2);
-        atomicAdd(&A.Nfix[2 * node + cur_s], W[o]);
-        W[o] = 0;
+        for (int o = 0; o < 8; ++o) {
+          const int64_t node = cur + (o & 1) + X * ((o >> 1) & 1) + XY * (o >> 2);
+          atomicAdd(&A.Nfix[2 * node + cur_s], W[o]);
+          W[o] = 0;
+        }
       }
+      cur = -1;
     };
-    for (int64_t q = q0; q < q1; ++q) {
-      const int sl = p.sim[q];
-      const SimDev &sd = A.sims[sl];
-      const int i = p.c[0][q], j = p.c[1][q], k = p.c[2][q];
-      if (i < 0 || j < 0 || k < 0 || i > sd.nx || j > sd.ny || k > sd.nz) continue;
-      const int64_t Xs = sd.X, XYs = (int64_t)sd.X * sd.Y;
-      const int64_t node = sd.gbase + i + Xs * j + XYs * k;
-      const int s = p.sp[q] - 1;
-      if (node != cur || s != cur_s) {
-        flush();
-        cur = node;
-        cur_s = s;
-        cur_slot = sl;
-        X = Xs;
-        XY = XYs;
-      }
-      const float fx = p.f[0][q], fy = p.f[1][q], fz = p.f[2][q];
-      const float wx[2] = {1.0f - fx, fx}, wy[2] = {1.0f - fy, fy}, wz[2] = {1.0f - fz, fz};
+#pragma unroll 1
+    for (int rd = 0; rd < kDepRounds; ++rd) {
+      const int64_t q0 = cb + ((int64_t)rd * kT + threadIdx.x) * kDepChunk;
+      if (q0 >= n) break;
+      int ci[8], cj[8], ck[8], sp[8], sim[8];
+      float fx[8], fy[8], fz[8];
+      load8(p.sim, q0, n, sim);
+      load8(p.c[0], q0, n, ci);
+      load8(p.c[1], q0, n, cj);
+      load8(p.c[2], q0, n, ck);
+      load8(p.sp, q0, n, sp);
+      load8(p.f[0], q0, n, fx);
+      load8(p.f[1], q0, n, fy);
+      load8(p.f[2], q0, n, fz);
 #pragma unroll
-      for (int o = 0; o < 8; ++o) {
-        const float w = wx[o & 1] * wy[(o >> 1) & 1] * wz[o >> 2];
-        W[o] += (unsigned long long)(double(w) * kFix);
+      for (int h = 0; h < kDepChunk; ++h) {
+        if (q0 + h >= n) break;
+        if (sim[h] != cur_slot) {
+          flush();
+          cur_slot = sim[h];
+          const SimDev &sd = A.sims[cur_slot];
+          nx = sd.nx;
+          ny = sd.ny;
+          nz = sd.nz;
+          X = sd.X;
+          XY = (int64_t)sd.X * sd.Y;
+          gbase = sd.gbase;
+        }
+        const int i = ci[h], j = cj[h], k = ck[h];
+        if (i < 0 || j < 0 || k < 0 || i > nx || j > ny || k > nz) continue;
+        const int64_t node = gbase + i + X * j + XY * k;
+        const int s = sp[h] - 1;
+        if (node != cur || s != cur_s) {
+          flush();
+          cur = node;
+          cur_s = s;
+        }
+        const float wx[2] = {1.0f - fx[h], fx[h]}, wy[2] = {1.0f - fy[h], fy[h]},
+                    wz[2] = {1.0f - fz[h], fz[h]};
+#pragma unroll
+        for (int o = 0; o < 8; ++o) W[o] += weight_units(wx[o & 1] * wy[(o >> 1) & 1] * wz[o >> 2]);
       }
     }
     flush();
@@ -534,7 +524,6 @@ __global__ void __launch_bounds__(kT) k_deposit(Arenas A, PartArena p) {
     __syncthreads();                    // the segments are cleared for the next chunk
   }
 }
-
 
 // ---------------------------------------------------------------------------
 // per-node kernels over node tiles {slot, first node}: 256 nodes each
@@ -2125,9 +2114,7 @@ static int launch_pre(picard_ensemble *e, int cur) {
   const int gp = grid_particles(e);
   k_inflow<<<gp, kT, 0, st>>>(A, X, e->cap);
   k_inflow_commit<<<1, 64, 0, st>>>(A, e->cap);
-  k_push<<<gp, kT, 0, st>>>(A, X);
   k_fill_i32<<<1024, kT, 0, st>>>(A.hist, A.kcap + 1, 0);
-  k_fill_i32<<<1024, kT, 0, st>>>(A.cursor, A.kcap + 1, 0);
   k_flag<<<gp, kT, 0, st>>>(A, X);
   PICARD_HIP(hipGetLastError());
   PICARD_TRY(scan_exclusive_stream(st, A.hist, A.hist, A.kcap, e->scan_tmp, e->scan_tmp_len));
@@ -2280,9 +2267,9 @@ int picard_sim_footprint(const picard_sim_params *p, int64_t *grid_bytes, int64_
   int32_t fch;
   slot_sizes(p, &nodes, &cells, &dist, &face, &keys, &fch);
   // U, u0, u1, C (FP64), N, Nfix (2 species), E32 (16 B), r32, the
-  // correction buffers, distance table, face partials, keys (hist + cursor)
+  // correction buffers, distance table, face partials, keys (hist)
   const int64_t b = nodes * (8 * 4 + 16 + 16 + 16) + cells * (4 + 4 * kEBufs) + dist * 8 +
-                    face * 8 + keys * 8 +
+                    face * 8 + keys * 4 +
                     cells * 2 * 8 * 3;       // the eigenbasis solve's buffers, rows padded
   if (grid_bytes) *grid_bytes = b;
   if (particles)
@@ -2375,8 +2362,7 @@ int picard_ensemble_create(const picard_ensemble_config *cfg, picard_ensemble **
   for (int q = 0; q < kEBufs; ++q) PICARD_TRY(dalloc_n(e, &A.e32[q], e->max_cells));
   for (int q = 0; q < 3; ++q) PICARD_TRY(dalloc_n(e, &A.sp[q], 2 * e->max_cells));
   PICARD_TRY(dalloc_n(e, &A.hist, kcap + 1));
-  PICARD_TRY(dalloc_n(e, &A.cursor, kcap + 1));
-  PICARD_TRY(dalloc_n(e, &A.key, e->cap));
+  PICARD_TRY(dalloc_n(e, &A.rank, e->cap));
   e->scan_tmp_len = scan_tmp_required(kcap);
   PICARD_TRY(dalloc_n(e, &e->scan_tmp, e->scan_tmp_len));
   for (int q = 0; q < 2; ++q) {

@@ -24,6 +24,7 @@
 #include "picard_internal.h"
 #include "reduce.h"
 #include "sched.h"
+#include "split_particles.h"
 
 namespace picard {
 namespace {
@@ -33,32 +34,8 @@ constexpr int kT = 256;
 // tile; eight blocks per CU at 8 waves per SIMD; 1024-thread blocks measured
 // slower)
 constexpr int kStencilT = 256;
-constexpr double kFix = 1099511627776.0;       // 2^40
-constexpr double kFixInv = 1.0 / 1099511627776.0;
-
 __device__ __forceinline__ int64_t lin_key(const GridDims &g, int i, int j, int k) {
   return (int64_t)i + (int64_t)(g.nx + 1) * ((int64_t)j + (int64_t)(g.ny + 1) * k);
-}
-
-// Carry a coordinate offset into [0, 1): returns the integer carry.
-__device__ __forceinline__ int carry(float &f) {
-  const float fl = floorf(f);
-  f = f - fl;
-  int c = (int)fl;
-  if (f >= 1.0f) {           // f - floor(f) rounded up to 1
-    f = 0.0f;
-    c += 1;
-  }
-  return c;
-}
-
-// AdvancePosition in the split form: xi += v dt/dx.
-__device__ __forceinline__ void push_one(int (&c)[3], float (&f)[3], const float (&v)[3], float3 dtdx) {
-  f[0] = f[0] + v[0] * dtdx.x;
-  f[1] = f[1] + v[1] * dtdx.y;
-  f[2] = f[2] + v[2] * dtdx.z;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) c[d] = (int16_t)(c[d] + carry(f[d]));
 }
 
 __global__ void __launch_bounds__(kT) k_sp_push(ParticlesSplit p, int64_t n, float3 dtdx) {
@@ -73,12 +50,6 @@ __global__ void __launch_bounds__(kT) k_sp_push(ParticlesSplit p, int64_t n, flo
     p.c[d][q] = (int16_t)c[d];
     p.f[d][q] = f[d];
   }
-}
-
-// xi < 1/2 is x < Lmin; xi > n + 1/2 is x > Lmax.
-__device__ __forceinline__ bool below(int c, float f) { return c < 0 || (c == 0 && f < 0.5f); }
-__device__ __forceinline__ bool above(int c, float f, int n) {
-  return c > n || (c == n && f > 0.5f);
 }
 
 // BCoutflow.f90:28-66 on the split coordinates: flow faces, and the band one
@@ -102,38 +73,6 @@ __device__ __forceinline__ void sp_wrap(const GridDims &g, int c[3], const float
     if (below(c[d], f[d])) c[d] += n[d];
     if (above(c[d], f[d], n[d])) c[d] -= n[d];
   }
-}
-
-// counter[k] += 1 for every lane of the wave with k >= 0, one atomic per
-// distinct key: the lanes sharing the leader's key (the lowest pending lane)
-// take ranks by lane order after the value the leader's add of their count
-// returned.  Returns what the lane's own add of 1 would have returned in one
-// order of the adds (-1 for k < 0).  Particles arrive nearly sorted by key,
-// so a wave holds two or three keys and the adds do not meet on one address
-// lane after lane.  Every lane stays in the loop (its condition is the
-// wave-uniform mask of pending lanes) and values cross lanes only through
-// readlane, which reads the lane whatever the exec mask; the leader's bit
-// leaves the mask every pass, so the loop ends within 64 passes.
-__device__ __forceinline__ int32_t wave_add1(int32_t *counter, int32_t k) {
-  const int lane = (int)(threadIdx.x & 63);
-  bool pending = k >= 0;
-  int32_t ret = -1;
-  uint64_t todo = __ballot(pending);
-  while (todo) {
-    const int leader = (int)__builtin_ctzll(todo);
-    const int32_t kl = __builtin_amdgcn_readlane(k, leader);
-    const bool mine = pending && k == kl;
-    const uint64_t m = __ballot(mine) | (1ull << leader);
-    int32_t base = 0;
-    if (lane == leader) base = atomicAdd(&counter[kl], (int32_t)__popcll(m));
-    base = __builtin_amdgcn_readlane(base, leader);
-    if (mine) {
-      ret = base + (int32_t)__popcll(m & ((1ull << lane) - 1ull));
-      pending = false;
-    }
-    todo &= ~m;
-  }
-  return ret;
 }
 
 // Cell and offset of particle q as the sort sees it: pushed first when q <
@@ -160,35 +99,19 @@ __device__ __forceinline__ bool sort_coords(const ParticlesSplit &p, int64_t q, 
 }
 
 // Sort key of a kept particle (its lower node and species), -1 for a deleted
-// one, and its rank among the particles of its key.  A block takes kFlagPer x
-// 256 consecutive particles; they arrive nearly sorted, so most keys lie in a
-// short stretch from the first ones': those are counted in LDS (the count
-// before is the rank within the block), each key then takes one atomic on its
-// histogram entry, whose return places the block's particles of that key.
-// The other keys (particles that moved a row or a plane on) are added a wave at
-// a time.  With the ranks known the scatter adds nothing: at 128^3 with 64 particles a
-// cell (1.4e8) flag and scatter take 1.31 + 3.15 ms, where a
-// wave's adds in both passes took 1.09 + 4.02; the step's push, 1.14 ms as a pass of its
-// own, costs them 0.1.
-constexpr int kFlagPer = 4;
-constexpr int kFlagWin = 1024;           // keys counted in LDS
-constexpr int kFlagBack = 128;           // of them below the first particle's
-
+// one, and its rank among the particles of its key.
 __global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, int64_t npush, GridDims g,
                                                  int wrap, float3 dtdx, int32_t *__restrict__ key,
                                                  int32_t *__restrict__ rank,
                                                  int32_t *__restrict__ hist) {
-  __shared__ int32_t cnt[kFlagWin];
-  __shared__ int32_t first;
-  for (int e = threadIdx.x; e < kFlagWin; e += kT) cnt[e] = 0;
-  if (threadIdx.x == 0) first = 0;
+  __shared__ KeyWindow win;
   const int64_t q0 = (int64_t)blockIdx.x * (kT * kFlagPer) + threadIdx.x;
   const int32_t cells = (int32_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
   int32_t k[kFlagPer], r[kFlagPer];
 #pragma unroll
   for (int h = 0; h < kFlagPer; ++h) {
     const int64_t q = q0 + h * kT;
-    k[h] = -1;                           // lanes past n stay for the wave's adds
+    k[h] = -1;
     int c[3];
     float f[3];
     if (q < n && sort_coords(p, q, npush, g, wrap, dtdx, c, f)) {
@@ -198,36 +121,11 @@ __global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, int
       k[h] = in ? (int32_t)lin_key(g, c[0], c[1], c[2]) * g.S + ((int32_t)p.sp[q] - 1) : cells * g.S;
     }
   }
-  __syncthreads();
-  {
-    const uint64_t kept = __ballot(k[0] >= 0);
-    if (threadIdx.x < 64 && kept) {      // the first wave's first kept particle
-      const int32_t kf = __builtin_amdgcn_readlane(k[0], (int)__builtin_ctzll(kept));
-      if (threadIdx.x == 0) first = kf > kFlagBack ? kf - kFlagBack : 0;
-    }
-  }
-  __syncthreads();
-  const int32_t k0 = first;
-#pragma unroll
-  for (int h = 0; h < kFlagPer; ++h) {
-    const bool near = k[h] >= k0 && k[h] - k0 < kFlagWin;
-    r[h] = -1;
-    if (near) r[h] = atomicAdd(&cnt[k[h] - k0], 1);
-    const int32_t far = wave_add1(hist, near ? -1 : k[h]);
-    if (!near) r[h] = far;
-  }
-  __syncthreads();
-  // each counted key's place in the histogram, over its count
-  for (int e = threadIdx.x; e < kFlagWin; e += kT) {
-    const int32_t m = cnt[e];
-    if (m) cnt[e] = atomicAdd(&hist[k0 + e], m);
-  }
-  __syncthreads();
+  count_keys(k, r, hist, win);
 #pragma unroll
   for (int h = 0; h < kFlagPer; ++h) {
     const int64_t q = q0 + h * kT;
     if (q >= n) continue;
-    if (k[h] >= k0 && k[h] - k0 < kFlagWin) r[h] += cnt[k[h] - k0];
     key[q] = k[h];
     rank[q] = r[h];
   }
@@ -284,47 +182,6 @@ constexpr int kDepChunk = 8;
 constexpr int kDepRounds = 2;
 constexpr int kDepSeg = 128;                    // nodes per LDS segment
 constexpr int kDepLdsSpecies = 3;               // species the LDS segments hold
-
-// a[q0 .. q0 + 8) (q0 a multiple of 8), those from n on as zero
-__device__ __forceinline__ void load8(const float *a, int64_t q0, int64_t n, float (&o)[8]) {
-  if (q0 + 8 <= n) {
-    *reinterpret_cast<float4 *>(&o[0]) = *reinterpret_cast<const float4 *>(a + q0);
-    *reinterpret_cast<float4 *>(&o[4]) = *reinterpret_cast<const float4 *>(a + q0 + 4);
-  } else {
-#pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0.0f;
-  }
-}
-__device__ __forceinline__ void load8(const int16_t *a, int64_t q0, int64_t n, int (&o)[8]) {
-  if (q0 + 8 <= n) {
-    const int4 w = *reinterpret_cast<const int4 *>(a + q0);
-    const int p[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = h & 1 ? p[h >> 1] >> 16 : (int)(int16_t)(p[h >> 1] & 0xffff);
-  } else {
-#pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0;
-  }
-}
-__device__ __forceinline__ void load8(const uint8_t *a, int64_t q0, int64_t n, int (&o)[8]) {
-  if (q0 + 8 <= n) {
-    const uint2 w = *reinterpret_cast<const uint2 *>(a + q0);
-#pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = (int)((h < 4 ? w.x : w.y) >> (8 * (h & 3)) & 0xffu);
-  } else {
-#pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0;
-  }
-}
-
-// (unsigned long long)(w 2^40) for a weight, 0 <= w <= 1 (NaN: 0): below 2^52 the
-// integer is in the low mantissa bits of trunc + 2^52, two adds in place of the
-// conversion's seven operations.
-__device__ __forceinline__ unsigned long long weight_units(float w) {
-  const float w1 = fminf(fmaxf(w, 0.0f), 1.0f);
-  const double v = __builtin_trunc(double(w1) * kFix) + 4503599627370496.0;
-  return (unsigned long long)__double_as_longlong(v) - 0x4330000000000000ull;
-}
 
 template <bool FLUX>
 __global__ void __launch_bounds__(kT) k_sp_deposit(ParticlesSplit p, int64_t n, GridDims g,

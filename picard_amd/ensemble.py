@@ -101,7 +101,7 @@ def footprint(spec: SimSpec) -> tuple[int, int]:
 
 
 # bytes per particle slot of the ensemble's arena: int16 cell x3, FP32 offset
-# x3, FP32 velocity x3, species, slot, id, sort key; two arenas for the sort
+# x3, FP32 velocity x3, species, slot, id, sort rank; two arenas for the sort
 PARTICLE_BYTES = 2 * (6 + 12 + 12 + 1 + 2 + 4) + 4
 
 
