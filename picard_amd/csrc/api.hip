@@ -255,7 +255,7 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   PICARD_TRY(dalloc(&c->s.scan_tmp, c->s.scan_tmp_len));
   PICARD_TRY(dalloc(&c->s.counters, 16));
   PICARD_TRY(dalloc(&c->s.key, cap));
-  PICARD_TRY(dalloc(&c->s.perm, cap));
+  if (!c->split) PICARD_TRY(dalloc(&c->s.perm, cap));
   PICARD_TRY(dalloc(&c->s.hist, nb + 1));
   const int64_t ncell = (int64_t)g.nx * g.ny * g.nz;
   int64_t pb = grid_blocks(g.G > ncell ? g.G : ncell, 256);

@@ -96,8 +96,8 @@ struct DeviceScratch {
   int64_t scan_tmp_len = 0;
   int32_t *counters = nullptr;     // small device counters (errors, totals)
   // deposit (reference order)
-  int32_t *key = nullptr;          // per particle
-  int32_t *perm = nullptr;         // per particle (split form: rank within its key)
+  int32_t *key = nullptr;          // per particle (split form: rank within its key)
+  int32_t *perm = nullptr;         // per particle (FP64 forms)
   int32_t *hist = nullptr;         // S*K + 1
   // staging for uploads/downloads (AoS)
   double *stage = nullptr;

@@ -98,15 +98,20 @@ __device__ __forceinline__ bool sort_coords(const ParticlesSplit &p, int64_t q, 
   return true;
 }
 
-// Sort key of a kept particle (its lower node and species), -1 for a deleted
-// one, and its rank among the particles of its key.
+// Sort key (cell, species), so that the deposit sees runs of one cell and species;
+// particles outside the grid after all of it share a last key.
+__device__ __forceinline__ int32_t sort_key(const GridDims &g, const int (&c)[3], int sp) {
+  const bool in = c[0] >= 0 && c[1] >= 0 && c[2] >= 0 && c[0] <= g.nx && c[1] <= g.ny && c[2] <= g.nz;
+  return in ? (int32_t)lin_key(g, c[0], c[1], c[2]) * g.S + (sp - 1)
+            : (int32_t)((g.nx + 1) * (g.ny + 1) * (g.nz + 1)) * g.S;
+}
+
+// Every kept particle's rank among those of its key.
 __global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, int64_t npush, GridDims g,
-                                                 int wrap, float3 dtdx, int32_t *__restrict__ key,
-                                                 int32_t *__restrict__ rank,
+                                                 int wrap, float3 dtdx, int32_t *__restrict__ rank,
                                                  int32_t *__restrict__ hist) {
   __shared__ KeyWindow win;
   const int64_t q0 = (int64_t)blockIdx.x * (kT * kFlagPer) + threadIdx.x;
-  const int32_t cells = (int32_t)(g.nx + 1) * (g.ny + 1) * (g.nz + 1);
   int32_t k[kFlagPer], r[kFlagPer];
 #pragma unroll
   for (int h = 0; h < kFlagPer; ++h) {
@@ -114,46 +119,37 @@ __global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, int
     k[h] = -1;
     int c[3];
     float f[3];
-    if (q < n && sort_coords(p, q, npush, g, wrap, dtdx, c, f)) {
-      const bool in = c[0] >= 0 && c[1] >= 0 && c[2] >= 0 && c[0] <= g.nx && c[1] <= g.ny &&
-                      c[2] <= g.nz;
-      // key (cell, species): the deposit then sees runs of one cell and species
-      k[h] = in ? (int32_t)lin_key(g, c[0], c[1], c[2]) * g.S + ((int32_t)p.sp[q] - 1) : cells * g.S;
-    }
+    if (q < n && sort_coords(p, q, npush, g, wrap, dtdx, c, f)) k[h] = sort_key(g, c, p.sp[q]);
   }
   count_keys(k, r, hist, win);
 #pragma unroll
   for (int h = 0; h < kFlagPer; ++h) {
     const int64_t q = q0 + h * kT;
-    if (q >= n) continue;
-    key[q] = k[h];
-    rank[q] = r[h];
+    if (q < n) rank[q] = r[h];
   }
 }
 
-// Every kept particle to its place, off[key] + rank.  Bound: streaming (43 B
+// Every kept particle to its place, off[key] + rank.  Bound: streaming (39 B
 // read, 35 written a particle; the places of a wave's particles are nearly one run);
-// it moves 13.3 GB in 3.15 ms at 1.4e8 particles (4.2 TB/s; a copy reaches 5.1).
+// it moves 13.3 GB in 3.04 ms at 1.4e8 particles (4.4 TB/s; a copy reaches 5.1).
 __global__ void __launch_bounds__(kT) k_sp_scatter(ParticlesSplit src, ParticlesSplit dst, int64_t n,
                                                     int64_t npush, GridDims g, int wrap, float3 dtdx,
-                                                    const int32_t *__restrict__ key,
                                                     const int32_t *__restrict__ rank,
                                                     const int32_t *__restrict__ off) {
   const int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (q >= n) return;
-  const int32_t k = key[q];
-  if (k < 0) return;
   int c[3];
   float f[3];
-  sort_coords(src, q, npush, g, wrap, dtdx, c, f);
-  const int64_t at = (int64_t)off[k] + rank[q];
+  if (!sort_coords(src, q, npush, g, wrap, dtdx, c, f)) return;
+  const int sp = src.sp[q];
+  const int64_t at = (int64_t)off[sort_key(g, c, sp)] + rank[q];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     dst.c[d][at] = (int16_t)c[d];
     dst.f[d][at] = f[d];
     dst.v[d][at] = src.v[d][q];
   }
-  dst.sp[at] = src.sp[q];
+  dst.sp[at] = (uint8_t)sp;
   dst.id[at] = src.id[q];
 }
 
@@ -2136,13 +2132,13 @@ int sp_sort(picard_ctx *c, int wrap, int64_t npush, double dt) {
   PICARD_HIP(hipMemsetAsync(c->s.hist, 0, sizeof(int32_t) * (K + 2), c->stream));
   if (n > 0) {
     k_sp_flag<<<grid_blocks(n, kT * kFlagPer), kT, 0, c->stream>>>(c->ps, n, npush, g, wrap, dtdx,
-                                                                   c->s.key, c->s.perm, c->s.hist);
+                                                                   c->s.key, c->s.hist);
     PICARD_HIP(hipGetLastError());
   }
   PICARD_TRY(scan_exclusive_i32(c, c->s.hist, c->s.hist, K + 1));
   if (n > 0) {
     k_sp_scatter<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->ps, c->ps2, n, npush, g, wrap, dtdx,
-                                                           c->s.key, c->s.perm, c->s.hist);
+                                                           c->s.key, c->s.hist);
     PICARD_HIP(hipGetLastError());
   }
   PICARD_HIP(hipMemcpyAsync(c->host_counters, c->s.hist + K + 1, sizeof(int32_t),

@@ -78,9 +78,8 @@ __device__ __forceinline__ int32_t wave_add1(int32_t *counter, int32_t k) {
 // histogram entry, whose return places the block's particles of that key.
 // The other keys (particles that moved a row or a plane on) are added a wave at
 // a time.  With the ranks known the scatter adds nothing: at 128^3 with 64 particles a
-// cell (1.4e8) flag and scatter take 1.31 + 3.15 ms, where a
-// wave's adds in both passes took 1.09 + 4.02; the step's push, 1.14 ms as a pass of its
-// own, costs them 0.1.
+// cell (1.4e8) flag and scatter take 1.13 + 3.04 ms, where a wave's adds in both passes took
+// 1.09 + 4.02; the step's push, 1.14 ms as a pass of its own, costs them 0.1.
 constexpr int kFlagPer = 4;
 constexpr int kFlagWin = 1024;           // keys counted in LDS
 constexpr int kFlagBack = 128;           // of them below the first particle's
