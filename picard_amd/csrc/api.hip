@@ -128,6 +128,7 @@ void release(picard_ctx *c) {
   dfree(c->C);
   dfree(c->D);
   bcpot_fft_release(c);
+  bcpot_modes_release(c);
   spec_release(c);
   dfree(c->haser_off);
   dfree(c->F);

@@ -1,5 +1,7 @@
-// bcpot_fft.hip -- BCpotentials (BCpotentials.f90:51-141) for the FP32-split
-// form: the open-boundary face sums in FP64, evaluated as FFT convolutions.
+// bcpot_fft.hip -- BCpotentials (BCpotentials.f90:51-141) for the FP32-split and
+// the order-free FP64 form where the distance table is not even (a table that the
+// caller wrote; CalcDistance's is, and goes to bcpot_modes.hip): the open-boundary face
+// sums in FP64, evaluated as FFT convolutions.
 //
 // For a flow dimension d, face f and the plane n of cells along d, the
 // reference sums C(cell) * D(offset) over the plane's cells, and the offset
@@ -225,6 +227,11 @@ int bcpot_fft_prepare(picard_ctx *c) {
       set_error("BCpotentials (split form): faces are limited to 512 x 512 cells");
       return PICARD_ERR_ARG;
     }
+  }
+  PICARD_TRY(bcpot_modes_prepare(c, &c->face_modes));
+  for (int d = 0; d < 3 && !c->face_modes; ++d) {
+    if (!g.flow[d]) continue;
+    const FaceGeo fg = make_face_geo(g, d);
     const int64_t plane = (int64_t)fg.M1 * fg.M2;
     for (int f = 0; f < 2; ++f) {
       if (!c->fft_K[d][f])
@@ -270,6 +277,7 @@ int launch_bc_potentials_fft(picard_ctx *c) {
   PICARD_HIP(hipMemsetAsync(c->U, 0, sizeof(double) * g.G, c->stream));   // BCpotentials.f90:36
   const double tau = 6.2831853071795864769252867665590;
   const double kfac = 1.0 / (2.0 * tau * 8.854187817e-12);
+  if (c->face_modes) return launch_bcpot_modes(c, kfac);
   for (int d = 0; d < 3; ++d) {
     if (!g.flow[d]) continue;
     const FaceGeo fg = make_face_geo(g, d);

@@ -1026,6 +1026,8 @@ __global__ void __launch_bounds__(kSpecT) k_sp_axis(Arenas A, int axis, int inv,
     t.nout = axis == 0 ? sd.PX : t.n;
     t.ld = axis == 2 ? P : sd.PX;
     t.gs = axis == 1 ? P : 0;
+    t.ldo = t.ld;
+    t.gso = t.gs;
     t.total = axis == 0 ? (int64_t)sd.ny * sd.nz : (axis == 1 ? (int64_t)sd.PX * sd.nz : P);
     t.gpr = (uint32_t)((axis == 1 ? sd.PX : t.total) / 16);
     if (axis == 0) {

@@ -163,7 +163,14 @@ struct picard_ctx {
   int64_t K = 0;             // deposit cells per species: (nx+1)(ny+1)(nz+1)
   bool have_D = false;
 
-  // split form: FFT evaluation of the open-boundary face sums
+  // split and order-free FP64 forms: open-boundary face sums mode by mode (bcpot_modes.hip):
+  // per axis the Fourier basis of twice its cells, per flow dim the distance table's
+  // eigenvalues, and the transformed charge
+  double *face_fwd[3] = {nullptr, nullptr, nullptr}, *face_inv[3] = {nullptr, nullptr, nullptr};
+  double *face_lam[3] = {nullptr, nullptr, nullptr};
+  double *face_work = nullptr;
+  bool face_modes = false;       // the distance table is even; otherwise FFTs (bcpot_fft.hip)
+  // FFT evaluation of the open-boundary face sums
   double2 *fft_K[3][2] = {};     // per flow dim and face: transformed face kernels, nd planes
   double2 *fft_tw[3][2] = {};    // per flow dim: twiddles of the two transverse lengths
   double2 *fft_work = nullptr;   // transformed charge planes + two face accumulators
@@ -283,6 +290,11 @@ int launch_bcpot_seq(picard_ctx *c, double kfac);
 
 // ---- diag.hip ----
 int diagnostics(picard_ctx *c, const double *mass, picard_diag *out);
+
+// ---- bcpot_modes.hip ----
+int bcpot_modes_prepare(picard_ctx *c, bool *even);
+int launch_bcpot_modes(picard_ctx *c, double kfac);
+void bcpot_modes_release(picard_ctx *c);
 
 // ---- bcpot_fft.hip ----
 int bcpot_fft_prepare(picard_ctx *c);

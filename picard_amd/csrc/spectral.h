@@ -58,6 +58,8 @@ __device__ __forceinline__ double spec_ln(double s, double c, bool *neg) {
 
 // Host: spectral.hip.
 int spec_axis_tables(hipStream_t s, int n, bool flow, double a, double *fwd, double *inv, double *eig);
+struct SpecTile;
+int spec_product(hipStream_t s, const SpecTile &t, bool xaxis);
 double spec_slowest(const int n[3], const int flow[3], const double a[3]);
 
 typedef double d4v __attribute__((ext_vector_type(4)));
@@ -73,14 +75,15 @@ typedef double d4v __attribute__((ext_vector_type(4)));
 //
 // XAXIS: columns are rows of x (data element (col, k) at col * ld + k);
 // otherwise a column group of 16 consecutive doubles sits at (g / gpr) gs +
-// (g % gpr) 16, and element k of a column at + k ld.  `total` columns in all.
+// (g % gpr) 16, and element k of a column at + k ld.  `total` columns in all.  The
+// outputs lie by ldo and gso, where a product changes the axis' length.
 struct SpecTile {
   const double *M;       // basis, [summed index][output index], pitch np
   const double *in;
   double *out;
   int n, np;             // axis cells, basis pitch
   int nout;              // outputs stored per column (x: the padded row, so that padding stays 0)
-  int64_t ld, gs;
+  int64_t ld, gs, ldo, gso;
   int64_t total;
   uint32_t gpr;
 };
@@ -192,10 +195,10 @@ __device__ __forceinline__ void spec_tile(const SpecTile &t, int axis0, int64_t 
         const int64_t col = col0 + wc + 16 * c + (XAXIS ? row : li);
         if (ax >= t.nout || col >= t.total) continue;
         if (XAXIS) {
-          t.out[col * t.ld + ax] = acc[a][c][v];
+          t.out[col * t.ldo + ax] = acc[a][c][v];
         } else {
           const uint32_t g = (uint32_t)(col >> 4);
-          t.out[(int64_t)(g / t.gpr) * t.gs + (int64_t)(g % t.gpr) * 16 + (col & 15) + (int64_t)ax * t.ld] =
+          t.out[(int64_t)(g / t.gpr) * t.gso + (int64_t)(g % t.gpr) * 16 + (col & 15) + (int64_t)ax * t.ldo] =
               acc[a][c][v];
         }
       }

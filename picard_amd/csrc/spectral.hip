@@ -320,7 +320,7 @@ template <int AT, bool XAXIS>
 __global__ void __launch_bounds__(kSpecT) k_spec_axis(SpecTile t, int nat, int64_t nct,
                                                       const SpecState *st) {
   __shared__ double lds[2 * kSpecLds];
-  if (st->skip) return;
+  if (st && st->skip) return;
   const int64_t i = blockIdx.x >> 3;
   const int at = (int)(i % nat);
   const int64_t ct = (i / nat) * 8 + (blockIdx.x & 7);
@@ -362,7 +362,15 @@ void spec_release(picard_ctx *c) {
 // Basis, transpose and eigenvalue parts of one axis; `a` is the Jacobi weight of its neighbours.
 int spec_axis_tables(hipStream_t s, int n, bool flow, double a, double *fwd, double *inv, double *eig) {
   k_spec_basis<<<grid_blocks(spec_mat_len(n), kT), kT, 0, s>>>(n, flow, fwd, inv);
-  k_spec_eig<<<grid_blocks(n, kT), kT, 0, s>>>(n, flow, a, eig);
+  if (eig) k_spec_eig<<<grid_blocks(n, kT), kT, 0, s>>>(n, flow, a, eig);
+  PICARD_HIP(hipGetLastError());
+  return PICARD_OK;
+}
+
+// One basis applied along one axis of one array (bcpot_modes.hip).
+int spec_product(hipStream_t s, const SpecTile &t, bool xaxis) {
+  if (xaxis) launch_axis<true>(s, t, nullptr);
+  else launch_axis<false>(s, t, nullptr);
   PICARD_HIP(hipGetLastError());
   return PICARD_OK;
 }
@@ -438,6 +446,8 @@ int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, bool app
     t.nout = d == 0 ? sg.PX : t.n;
     t.ld = d == 2 ? P : sg.PX;
     t.gs = d == 1 ? P : 0;
+    t.ldo = t.ld;
+    t.gso = t.gs;
     t.total = d == 0 ? (int64_t)g.ny * g.nz : (d == 1 ? (int64_t)sg.PX * g.nz : P);
     t.gpr = (uint32_t)((d == 1 ? sg.PX : t.total) / 16);
     if (d == 0) launch_axis<true>(s, t, st);
