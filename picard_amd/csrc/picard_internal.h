@@ -83,7 +83,7 @@ struct JacobiState {
   int32_t maxit;
   int32_t done;
   int32_t stop_inner;
-  uint32_t arrive;           // block arrival counter for the last-block reduction
+  uint32_t reserved;
 };
 
 struct DeviceScratch {
@@ -260,7 +260,7 @@ int stage_particles(picard_ctx *c, int64_t first, int64_t count, double *stage, 
 int ensure_stage(picard_ctx *c, int64_t want);
 
 // ---- grid.hip ----
-int launch_bnorm(picard_ctx *c, double maxerr);
+int launch_begin(picard_ctx *c, const JacobiState &init, double maxerr, bool copy);
 // flux: also the number fluxes F of ParticlesGridifyAll
 int launch_gridify(picard_ctx *c, bool flux = false);
 int launch_calc_distance(picard_ctx *c);

@@ -24,6 +24,7 @@
 // 128^3 to 1e-10 1.7 ms (FP32 sweeps 620), 160^3 2.5 ms (FP32 sweeps 880).
 // Against the FP64 form that sweeps all the way U differs by 2e-15 to 3e-13
 // (the FP32 sweeps differed by 5e-7 to 5e-6) and the sweep counts are equal.
+#include <algorithm>
 #include <cmath>
 
 #include "picard_internal.h"
@@ -152,11 +153,12 @@ __global__ void __launch_bounds__(kT) k_spec_residual(SpecGeo g, const double *_
 // (pass 0: halvings of the bound) or ascending in q (later passes: a division
 // of the bracket); the last block narrows the bracket and, after the last pass,
 // interpolates ln(norm^2) in it.  Bound: one read of the spectrum and the
-// exponentials (eight per mode that has not decayed away).
+// exponentials (eight per mode that has not decayed away); on small grids the chain of the
+// block's and the last block's sums: the candidates' together, 28 -> 10 us at 16^3.
 __global__ void __launch_bounds__(kT) k_spec_search(SpecGeo g, const double *__restrict__ R,
                                                     double *__restrict__ partials, SpecState *st,
                                                     int pass) {
-  __shared__ double sh[kT / 64];
+  __shared__ double sh[kT / 64][kSpecCand];
   __shared__ double tot[kSpecCand];
   if (st->skip) return;
   double q2[kSpecCand], qmin = 1.0e300;
@@ -180,18 +182,29 @@ __global__ void __launch_bounds__(kT) k_spec_search(SpecGeo g, const double *__r
 #pragma unroll
     for (int i = 0; i < kSpecCand; ++i) acc[i] += w * exp(q2[i] * ln);
   }
+  // the candidates' block sums together, then their totals, 32 lanes each
 #pragma unroll
   for (int i = 0; i < kSpecCand; ++i) {
-    const double s = block_sum(acc[i], sh);
-    if (threadIdx.x == 0) partials[(int64_t)i * gridDim.x + blockIdx.x] = s;
-    __syncthreads();
+    for (int off = 32; off > 0; off >>= 1) acc[i] += __shfl_down(acc[i], off, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][i] = acc[i];
   }
+  __syncthreads();
+  if (threadIdx.x < kSpecCand) {
+    double s = 0.0;
+    for (int w = 0; w < kT / 64; ++w) s += sh[w][threadIdx.x];
+    partials[(int64_t)threadIdx.x * gridDim.x + blockIdx.x] = s;
+  }
+  __syncthreads();                       // before the fence of thread 0
   if (!last_block(&st->arrive)) return;
-  for (int i = 0; i < kSpecCand; ++i) {
-    const double s = final_sum(partials + (int64_t)i * gridDim.x, gridDim.x, sh);
-    if (threadIdx.x == 0) tot[i] = s;
-    __syncthreads();
+  static_assert(kT == 32 * kSpecCand, "32 lanes to a candidate");
+  {
+    const int i = threadIdx.x >> 5;
+    double s = 0.0;
+    for (unsigned q = threadIdx.x & 31; q < gridDim.x; q += 32) s += partials[(int64_t)i * gridDim.x + q];
+    for (int off = 16; off > 0; off >>= 1) s += __shfl_down(s, off, 32);
+    if ((threadIdx.x & 31) == 0) tot[i] = s;
   }
+  __syncthreads();
   if (threadIdx.x) return;
   st->arrive = 0;
   double lo = st->lo, hi = st->hi, flo = st->flo, fhi = st->fhi;
@@ -453,10 +466,10 @@ int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, bool app
     if (d == 0) launch_axis<true>(s, t, st);
     else launch_axis<false>(s, t, st);
   };
-  // blocks of the passes over the array: four per CU at most, eight elements a
-  // thread at least; their partials fit the context's array (the search keeps
+  // blocks of the passes over the array: one per CU while they have work, then eight
+  // elements a thread, four per CU at most; their partials fit the context's array (the search keeps
   // eight sums per block)
-  int64_t nb = (sg.len + 8 * kT - 1) / (8 * kT);
+  int64_t nb = std::max((sg.len + 8 * kT - 1) / (8 * kT), std::min<int64_t>((sg.len + kT - 1) / kT, 256));
   if (nb > 1024) nb = 1024;
   const int64_t cap = 4 * c->s.partials_len / kSpecCand;
   if (nb > cap) nb = cap;

@@ -2470,8 +2470,7 @@ int sp_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t *sweeps) 
   JacobiState init{};
   init.maxit = maxit;
   init.last = 2 * (int64_t)maxit + 1;
-  PICARD_HIP(hipMemcpyAsync(c->js, &init, sizeof(JacobiState), hipMemcpyHostToDevice, c->stream));
-  PICARD_TRY(launch_bnorm(c, maxerr));      // launch 0: b, |b|, the test of ss = 1
+  PICARD_TRY(launch_begin(c, init, maxerr, false));   // launch 0: b, |b|, the test of ss = 1
   const TileSched ts = stencil_sched(c);
   const SweepGeo sg = sweep_sched(c);
   const OuterGeo og = outer_sched(c);
