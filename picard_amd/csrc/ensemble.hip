@@ -470,14 +470,14 @@ __global__ void __launch_bounds__(kT) k_deposit(Arenas A, PartArena p) {
       if (q0 >= n) break;
       int ci[8], cj[8], ck[8], sp[8], sim[8];
       float fx[8], fy[8], fz[8];
-      load8(p.sim, q0, n, sim);
-      load8(p.c[0], q0, n, ci);
-      load8(p.c[1], q0, n, cj);
-      load8(p.c[2], q0, n, ck);
-      load8(p.sp, q0, n, sp);
-      load8(p.f[0], q0, n, fx);
-      load8(p.f[1], q0, n, fy);
-      load8(p.f[2], q0, n, fz);
+      load_chunk(p.sim, q0, n, sim);
+      load_chunk(p.c[0], q0, n, ci);
+      load_chunk(p.c[1], q0, n, cj);
+      load_chunk(p.c[2], q0, n, ck);
+      load_chunk(p.sp, q0, n, sp);
+      load_chunk(p.f[0], q0, n, fx);
+      load_chunk(p.f[1], q0, n, fy);
+      load_chunk(p.f[2], q0, n, fz);
 #pragma unroll
       for (int h = 0; h < kDepChunk; ++h) {
         if (q0 + h >= n) break;

@@ -98,6 +98,10 @@ __device__ __forceinline__ bool sort_coords(const ParticlesSplit &p, int64_t q, 
   return true;
 }
 
+// From here on a block's particles are as many as its registers take: four blocks
+// of 1024 to each of 256 CUs.
+constexpr int64_t kManyParticles = int64_t(1) << 20;
+
 // Sort key (cell, species), so that the deposit sees runs of one cell and species;
 // particles outside the grid after all of it share a last key.
 __device__ __forceinline__ int32_t sort_key(const GridDims &g, const int (&c)[3], int sp) {
@@ -106,15 +110,16 @@ __device__ __forceinline__ int32_t sort_key(const GridDims &g, const int (&c)[3]
             : (int32_t)((g.nx + 1) * (g.ny + 1) * (g.nz + 1)) * g.S;
 }
 
-// Every kept particle's rank among those of its key.
+// Every kept particle's rank among those of its key, PER particles a thread.
+template <int PER>
 __global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, int64_t npush, GridDims g,
                                                  int wrap, float3 dtdx, int32_t *__restrict__ rank,
                                                  int32_t *__restrict__ hist) {
   __shared__ KeyWindow win;
-  const int64_t q0 = (int64_t)blockIdx.x * (kT * kFlagPer) + threadIdx.x;
-  int32_t k[kFlagPer], r[kFlagPer];
+  const int64_t q0 = (int64_t)blockIdx.x * (kT * PER) + threadIdx.x;
+  int32_t k[PER], r[PER];
 #pragma unroll
-  for (int h = 0; h < kFlagPer; ++h) {
+  for (int h = 0; h < PER; ++h) {
     const int64_t q = q0 + h * kT;
     k[h] = -1;
     int c[3];
@@ -123,7 +128,7 @@ __global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, int
   }
   count_keys(k, r, hist, win);
 #pragma unroll
-  for (int h = 0; h < kFlagPer; ++h) {
+  for (int h = 0; h < PER; ++h) {
     const int64_t q = q0 + h * kT;
     if (q < n) rank[q] = r[h];
   }
@@ -159,7 +164,7 @@ __global__ void __launch_bounds__(kT) k_sp_scatter(ParticlesSplit src, Particles
 constexpr double kFluxFix = 16777216.0;         // 2^24
 constexpr double kFluxFixInv = 1.0 / 16777216.0;
 
-// Particles are sorted by (cell, species), so a thread walks kDepChunk
+// Particles are sorted by (cell, species), so a thread walks CHUNK
 // consecutive particles and adds the fixed-point weights of each run of one
 // cell and species in registers, flushing one add per corner when the run
 // ends: integer sums, so the result equals one atomic per particle.
@@ -167,19 +172,23 @@ constexpr double kFluxFixInv = 1.0 / 16777216.0;
 // contiguous stretch of each array: read a particle at a time, lanes 16 particles
 // apart, the kernel fetched 300 bytes a particle where 19 are needed (5.58 ms
 // at 1.4e8 particles; now 0.63, 4.2 TB/s).
-// Without the fluxes the adds are staged in LDS per block: the block's kDepRounds x
-// 2048 sorted particles cover a short stretch of lower nodes from the first one's, b0, so
+// Without the fluxes the adds are staged in LDS per block: the block's ROUNDS x 256 x
+// CHUNK sorted particles cover a short stretch of lower nodes from the first one's, b0, so
 // their corners fall in four node segments b0 + {0, X, XY, XY + X} + [0,
 // kDepSeg); runs whose corners lie inside go to the segments with LDS
 // atomics, the rest straight to memory, and the block then adds each nonzero
 // segment entry to memory once (a few hundred global atomics per block
 // instead of eight per run).
+// CHUNK, ROUNDS: 8 and 2, or 4 and 1 where a block's 4096 particles leave CUs idle or
+// spread over more nodes than a segment holds (fewer than 32 a cell).  Whole ParticlesGridify, us,
+// both ways: 6.6e4 particles 43, 30; 1.8e6 at 16 a cell 52, 41; 4.2e6 at 16 73, 55; 3.5e6 at
+// 32 49, 48; 1.7e7 at 64 123, 145 (with segments of 128 nodes 139).
 constexpr int kDepChunk = 8;
 constexpr int kDepRounds = 2;
-constexpr int kDepSeg = 128;                    // nodes per LDS segment
+constexpr int kDepSeg = 256;                    // nodes per LDS segment
 constexpr int kDepLdsSpecies = 3;               // species the LDS segments hold
 
-template <bool FLUX>
+template <bool FLUX, int CHUNK, int ROUNDS>
 __global__ void __launch_bounds__(kT) k_sp_deposit(ParticlesSplit p, int64_t n, GridDims g,
                                                     unsigned long long *__restrict__ Nfix,
                                                     unsigned long long *__restrict__ Ffix,
@@ -197,7 +206,7 @@ __global__ void __launch_bounds__(kT) k_sp_deposit(ParticlesSplit p, int64_t n, 
       // there leaves the whole block on the direct path)
       int ok = 0;
       int64_t bb = 0;
-      const int64_t qf = (int64_t)blockIdx.x * (kT * kDepChunk * kDepRounds);
+      const int64_t qf = (int64_t)blockIdx.x * (kT * CHUNK * ROUNDS);
       if (qf < n && S <= kDepLdsSpecies) {
         const int i = p.c[0][qf], j = p.c[1][qf], k = p.c[2][qf];
         if (!(i < 0 || j < 0 || k < 0 || i > g.nx || j > g.ny || k > g.nz)) {
@@ -244,25 +253,25 @@ __global__ void __launch_bounds__(kT) k_sp_deposit(ParticlesSplit p, int64_t n, 
   };
   int nerr = 0;
 #pragma unroll 1
-  for (int rd = 0; rd < kDepRounds; ++rd) {
+  for (int rd = 0; rd < ROUNDS; ++rd) {
     const int64_t q0 =
-        (((int64_t)blockIdx.x * kDepRounds + rd) * kT + threadIdx.x) * kDepChunk;
+        (((int64_t)blockIdx.x * ROUNDS + rd) * kT + threadIdx.x) * CHUNK;
     if (q0 >= n) break;
-    int ci[8], cj[8], ck[8], sp[8];
-    float fx[8], fy[8], fz[8], vv[3][FLUX ? 8 : 1];
-    load8(p.c[0], q0, n, ci);
-    load8(p.c[1], q0, n, cj);
-    load8(p.c[2], q0, n, ck);
-    load8(p.sp, q0, n, sp);
-    load8(p.f[0], q0, n, fx);
-    load8(p.f[1], q0, n, fy);
-    load8(p.f[2], q0, n, fz);
+    int ci[CHUNK], cj[CHUNK], ck[CHUNK], sp[CHUNK];
+    float fx[CHUNK], fy[CHUNK], fz[CHUNK], vv[3][FLUX ? CHUNK : 1];
+    load_chunk(p.c[0], q0, n, ci);
+    load_chunk(p.c[1], q0, n, cj);
+    load_chunk(p.c[2], q0, n, ck);
+    load_chunk(p.sp, q0, n, sp);
+    load_chunk(p.f[0], q0, n, fx);
+    load_chunk(p.f[1], q0, n, fy);
+    load_chunk(p.f[2], q0, n, fz);
     if constexpr (FLUX) {
 #pragma unroll
-      for (int d = 0; d < 3; ++d) load8(p.v[d], q0, n, vv[d]);
+      for (int d = 0; d < 3; ++d) load_chunk(p.v[d], q0, n, vv[d]);
     }
 #pragma unroll
-    for (int h = 0; h < kDepChunk; ++h) {
+    for (int h = 0; h < CHUNK; ++h) {
       if (q0 + h >= n) break;
       const int i = ci[h], j = cj[h], k = ck[h];
       if (i < 0 || j < 0 || k < 0 || i > g.nx || j > g.ny || k > g.nz) {
@@ -2131,8 +2140,12 @@ int sp_sort(picard_ctx *c, int wrap, int64_t npush, double dt) {
   const float3 dtdx = push_factor(c, dt);
   PICARD_HIP(hipMemsetAsync(c->s.hist, 0, sizeof(int32_t) * (K + 2), c->stream));
   if (n > 0) {
-    k_sp_flag<<<grid_blocks(n, kT * kFlagPer), kT, 0, c->stream>>>(c->ps, n, npush, g, wrap, dtdx,
-                                                                   c->s.key, c->s.hist);
+    if (n >= kManyParticles)
+      k_sp_flag<kFlagPer><<<grid_blocks(n, kT * kFlagPer), kT, 0, c->stream>>>(
+          c->ps, n, npush, g, wrap, dtdx, c->s.key, c->s.hist);
+    else
+      k_sp_flag<1><<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->ps, n, npush, g, wrap, dtdx, c->s.key,
+                                                             c->s.hist);
     PICARD_HIP(hipGetLastError());
   }
   PICARD_TRY(scan_exclusive_i32(c, c->s.hist, c->s.hist, K + 1));
@@ -2167,12 +2180,16 @@ int sp_gridify(picard_ctx *c, bool flux) {
     PICARD_HIP(hipMemsetAsync(c->Ffix, 0, sizeof(unsigned long long) * 3 * g.S * g.G, c->stream));
   }
   if (c->n > 0) {
+    const int per = kT * kDepChunk * kDepRounds;
     if (flux)
-      k_sp_deposit<true><<<grid_blocks(c->n, kT * kDepChunk * kDepRounds), kT, 0,
-                           c->stream>>>(c->ps, c->n, g, c->Nfix, c->Ffix, c->s.counters);
+      k_sp_deposit<true, kDepChunk, kDepRounds><<<grid_blocks(c->n, per), kT, 0, c->stream>>>(
+          c->ps, c->n, g, c->Nfix, c->Ffix, c->s.counters);
+    else if (c->n >= 4 * kManyParticles && c->n >= 32 * c->K)
+      k_sp_deposit<false, kDepChunk, kDepRounds><<<grid_blocks(c->n, per), kT, 0, c->stream>>>(
+          c->ps, c->n, g, c->Nfix, nullptr, c->s.counters);
     else
-      k_sp_deposit<false><<<grid_blocks(c->n, kT * kDepChunk * kDepRounds), kT, 0,
-                            c->stream>>>(c->ps, c->n, g, c->Nfix, nullptr, c->s.counters);
+      k_sp_deposit<false, 4, 1><<<grid_blocks(c->n, kT * 4), kT, 0, c->stream>>>(
+          c->ps, c->n, g, c->Nfix, nullptr, c->s.counters);
     PICARD_HIP(hipGetLastError());
   }
   k_sp_fold<<<grid_blocks(g.G, kT), kT, 0, c->stream>>>(g, c->Nfix, c->N, c->C, c->consts);

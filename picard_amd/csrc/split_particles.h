@@ -71,7 +71,7 @@ __device__ __forceinline__ int32_t wave_add1(int32_t *counter, int32_t k) {
 }
 
 // Places of a block's keys in a counting sort: hist[k] gains each key's count, r[h] is
-// the particle's rank among all of its key (-1 for k[h] < 0).  A block takes kFlagPer x
+// the particle's rank among all of its key (-1 for k[h] < 0).  A block takes PER x
 // 256 consecutive particles; they arrive nearly sorted, so most keys lie in a
 // short stretch from the first ones': those are counted in LDS (the count
 // before is the rank within the block), each key then takes one atomic on its
@@ -80,6 +80,8 @@ __device__ __forceinline__ int32_t wave_add1(int32_t *counter, int32_t k) {
 // a time.  With the ranks known the scatter adds nothing: at 128^3 with 64 particles a
 // cell (1.4e8) flag and scatter take 1.13 + 3.04 ms, where a wave's adds in both passes took
 // 1.09 + 4.02; the step's push, 1.14 ms as a pass of its own, costs them 0.1.
+// PER: four particles a thread, or one where that leaves CUs idle: a sort of 6.6e4 particles
+// 37 and 34 us, of 1.0e6 49 both ways, of 1.7e7 355 and 390.
 constexpr int kFlagPer = 4;
 constexpr int kFlagWin = 1024;           // keys counted in LDS
 constexpr int kFlagBack = 128;           // of them below the first particle's
@@ -89,7 +91,8 @@ struct KeyWindow {
 };
 
 // Every thread of a block of 256 takes part; returns after a barrier.
-__device__ __forceinline__ void count_keys(const int32_t (&k)[kFlagPer], int32_t (&r)[kFlagPer],
+template <int PER>
+__device__ __forceinline__ void count_keys(const int32_t (&k)[PER], int32_t (&r)[PER],
                                            int32_t *__restrict__ hist, KeyWindow &w) {
   for (int e = threadIdx.x; e < kFlagWin; e += 256) w.cnt[e] = 0;
   const uint64_t kept = __ballot(k[0] >= 0);
@@ -100,7 +103,7 @@ __device__ __forceinline__ void count_keys(const int32_t (&k)[kFlagPer], int32_t
   __syncthreads();
   const int32_t k0 = w.first;
 #pragma unroll
-  for (int h = 0; h < kFlagPer; ++h) {
+  for (int h = 0; h < PER; ++h) {
     const bool near = k[h] >= k0 && k[h] - k0 < kFlagWin;
     r[h] = -1;
     if (near) r[h] = atomicAdd(&w.cnt[k[h] - k0], 1);
@@ -115,51 +118,57 @@ __device__ __forceinline__ void count_keys(const int32_t (&k)[kFlagPer], int32_t
   }
   __syncthreads();
 #pragma unroll
-  for (int h = 0; h < kFlagPer; ++h)
+  for (int h = 0; h < PER; ++h)
     if (k[h] >= k0 && k[h] - k0 < kFlagWin) r[h] += w.cnt[k[h] - k0];
   __syncthreads();
 }
 
-// a[q0 .. q0 + 8) (q0 a multiple of 8, a 16-byte aligned), those from n on as zero
-__device__ __forceinline__ void load8(const float *a, int64_t q0, int64_t n, float (&o)[8]) {
-  if (q0 + 8 <= n) {
-    *reinterpret_cast<float4 *>(&o[0]) = *reinterpret_cast<const float4 *>(a + q0);
-    *reinterpret_cast<float4 *>(&o[4]) = *reinterpret_cast<const float4 *>(a + q0 + 4);
+// a[q0 .. q0 + N) (N 4 or 8, q0 a multiple of N, a 16-byte aligned), those from n on as zero
+template <int N>
+__device__ __forceinline__ void load_chunk(const float *a, int64_t q0, int64_t n, float (&o)[N]) {
+  if (q0 + N <= n) {
+#pragma unroll
+    for (int h = 0; h < N; h += 4)
+      *reinterpret_cast<float4 *>(&o[h]) = *reinterpret_cast<const float4 *>(a + q0 + h);
   } else {
 #pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0.0f;
+    for (int h = 0; h < N; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0.0f;
   }
 }
-__device__ __forceinline__ void load8(const int16_t *a, int64_t q0, int64_t n, int (&o)[8]) {
-  if (q0 + 8 <= n) {
-    const int4 w = *reinterpret_cast<const int4 *>(a + q0);
-    const int p[4] = {w.x, w.y, w.z, w.w};
+template <int N, typename I16>           // int16_t or uint16_t
+__device__ __forceinline__ void load_chunk(const I16 *a, int64_t q0, int64_t n, int (&o)[N]) {
+  static_assert(sizeof(I16) == 2, "16-bit integers");
+  if (q0 + N <= n) {
+    int p[N / 2];
+    if constexpr (N == 8) {
+      const int4 w = *reinterpret_cast<const int4 *>(a + q0);
+      p[0] = w.x, p[1] = w.y, p[2] = w.z, p[3] = w.w;
+    } else {
+      const int2 w = *reinterpret_cast<const int2 *>(a + q0);
+      p[0] = w.x, p[1] = w.y;
+    }
 #pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = h & 1 ? p[h >> 1] >> 16 : (int)(int16_t)(p[h >> 1] & 0xffff);
+    for (int h = 0; h < N; ++h) o[h] = (I16)(h & 1 ? p[h >> 1] >> 16 : p[h >> 1] & 0xffff);
   } else {
 #pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0;
+    for (int h = 0; h < N; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0;
   }
 }
-__device__ __forceinline__ void load8(const uint16_t *a, int64_t q0, int64_t n, int (&o)[8]) {
-  if (q0 + 8 <= n) {
-    const int4 w = *reinterpret_cast<const int4 *>(a + q0);
-    const int p[4] = {w.x, w.y, w.z, w.w};
+template <int N>
+__device__ __forceinline__ void load_chunk(const uint8_t *a, int64_t q0, int64_t n, int (&o)[N]) {
+  if (q0 + N <= n) {
+    uint32_t p[N / 4];
+    if constexpr (N == 8) {
+      const uint2 w = *reinterpret_cast<const uint2 *>(a + q0);
+      p[0] = w.x, p[1] = w.y;
+    } else {
+      p[0] = *reinterpret_cast<const uint32_t *>(a + q0);
+    }
 #pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = h & 1 ? (int)((uint32_t)p[h >> 1] >> 16) : p[h >> 1] & 0xffff;
+    for (int h = 0; h < N; ++h) o[h] = (int)(p[h >> 2] >> (8 * (h & 3)) & 0xffu);
   } else {
 #pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0;
-  }
-}
-__device__ __forceinline__ void load8(const uint8_t *a, int64_t q0, int64_t n, int (&o)[8]) {
-  if (q0 + 8 <= n) {
-    const uint2 w = *reinterpret_cast<const uint2 *>(a + q0);
-#pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = (int)((h < 4 ? w.x : w.y) >> (8 * (h & 3)) & 0xffu);
-  } else {
-#pragma unroll
-    for (int h = 0; h < 8; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0;
+    for (int h = 0; h < N; ++h) o[h] = q0 + h < n ? a[q0 + h] : 0;
   }
 }
 

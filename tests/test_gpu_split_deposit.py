@@ -12,8 +12,9 @@ from picard_amd import _lib, host
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 9, 2047, 2049, 4095, 4097, 20011])
-@pytest.mark.parametrize("dims", [(4, 3, 5), (37, 9, 6)])
+@pytest.mark.parametrize("n,dims", [(n, d) for n in (1, 7, 8, 9, 2047, 2049, 4095, 4097, 20011)
+                                    for d in ((4, 3, 5), (37, 9, 6))]
+                         + [((1 << 20) + 3, (37, 9, 6)), ((1 << 22) + 4099, (37, 9, 6))])
 def test_deposit_counts(n, dims):
     half = tuple(5.0 * v for v in dims)
     cfg = host.Config(nx=dims[0], ny=dims[1], nz=dims[2], flow=(True, False, True),
