@@ -1241,27 +1241,83 @@ __global__ void __launch_bounds__(kT) k_bc_fields(GridDims g, double *__restrict
 constexpr double kFix48 = 281474976710656.0;          // 2^48
 constexpr double kFix48Inv = 1.0 / 281474976710656.0;
 
-__global__ void __launch_bounds__(kT) k_dep_fix64(ParticlesF64 p, int64_t n, GridDims g,
-                                                  unsigned long long *__restrict__ Nfix,
-                                                  int32_t *__restrict__ errors) {
-  const int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (q >= n) return;
-  const CicLoc L = cic_locate(g, p.r[0][q], p.r[1][q], p.r[2][q]);
-  const int s0 = p.sp[q] - 1;
-  if (!cic_in_bounds(g, L) || s0 < 0 || s0 >= g.S) {
-    atomicAdd(errors, 1);
-    return;
-  }
-  const int64_t base = node_index(g, L.idx[0], L.idx[1], L.idx[2]);
+// The particles come bucketed by (species, lower node) as for the reference order, but in
+// no order within a bucket: a thread takes four in turn, adds the weights of a run of one
+// bucket in registers, and a block's runs go to LDS: their corners fall in four segments of
+// nodes, b0 + {0, X, XY, XY + X} + [0, kFixSeg), of its first particle's species (a run beyond
+// goes to memory).  One atomic per corner and particle took 1.10 ms at 6.3e6 particles, 12 a
+// cell and species; the counting, the scatter and this take 0.16 + 0.03 + 0.29.
+constexpr int kFixSeg = 256;
+
+// (unsigned long long)llrint(F 2^48), 0 <= F <= 1 (NaN: 0): the sum with 2^52 rounds to
+// whole units, which are its low mantissa bits
+__device__ __forceinline__ unsigned long long fix48(double F) {
+  const double v = fmin(fmax(F * kFix48, 0.0), 2.0 * kFix48) + 4503599627370496.0;
+  return (unsigned long long)__double_as_longlong(v) - 0x4330000000000000ull;
+}
+
+__global__ void __launch_bounds__(kT) k_dep_fix64(ParticlesF64 p, GridDims g, int64_t nb,
+                                                  const int32_t *__restrict__ off,
+                                                  const int32_t *__restrict__ perm,
+                                                  unsigned long long *__restrict__ Nfix) {
+  __shared__ unsigned long long seg[4 * kFixSeg];
+  __shared__ int64_t first;
+  __shared__ int species;
+  const int64_t n = off[nb];
+  const int64_t q0 = ((int64_t)blockIdx.x * kT + threadIdx.x) * 4;
+  if ((int64_t)blockIdx.x * kT * 4 >= n) return;               // block-uniform
+  for (int e = threadIdx.x; e < 4 * kFixSeg; e += kT) seg[e] = 0;
+  const int64_t X = g.X, XY = (int64_t)g.X * g.Y;
+  int64_t node[4];
+  int sp[4];
+  double rest[4][3];
 #pragma unroll
-  for (int o = 0; o < 8; ++o) {
-    const double fx = (o & 1) ? L.rest[0] : L.drest[0];
-    const double fy = (o & 2) ? L.rest[1] : L.drest[1];
-    const double fz = (o & 4) ? L.rest[2] : L.drest[2];
-    const double F = fx * fy * fz / g.dV;
-    const int64_t node = base + (o & 1) + (int64_t)g.X * ((o >> 1) & 1) +
-                         (int64_t)g.X * g.Y * (o >> 2);
-    atomicAdd(&Nfix[node * g.S + s0], (unsigned long long)llrint(F * kFix48));
+  for (int h = 0; h < 4; ++h) {
+    const int32_t q = perm[q0 + h < n ? q0 + h : n - 1];
+    const CicLoc L = cic_locate(g, p.r[0][q], p.r[1][q], p.r[2][q]);
+    node[h] = node_index(g, L.idx[0], L.idx[1], L.idx[2]);
+    sp[h] = p.sp[q] - 1;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) rest[h][d] = L.rest[d];
+  }
+  if (threadIdx.x == 0) {
+    first = node[0];
+    species = sp[0];
+  }
+  __syncthreads();
+  const int64_t b0 = first;
+  const int s0 = species;
+  unsigned long long W[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    if (q0 + h >= n) break;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      const double fx = (o & 1) ? rest[h][0] : g.dxyz[0] - rest[h][0];
+      const double fy = (o & 2) ? rest[h][1] : g.dxyz[1] - rest[h][1];
+      const double fz = (o & 4) ? rest[h][2] : g.dxyz[2] - rest[h][2];
+      W[o] += fix48(fx * fy * fz / g.dV);
+    }
+    if (h < 3 && q0 + h + 1 < n && node[h + 1] == node[h] && sp[h + 1] == sp[h]) continue;
+    const int64_t at = node[h] - b0;
+    const bool in = sp[h] == s0 && at >= 0 && at + 1 < kFixSeg;
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      if (in) {
+        atomicAdd(&seg[(o >> 1) * kFixSeg + (int)at + (o & 1)], W[o]);
+      } else {
+        const int64_t to = node[h] + (o & 1) + X * ((o >> 1) & 1) + XY * (o >> 2);
+        atomicAdd(&Nfix[to * g.S + sp[h]], W[o]);
+      }
+      W[o] = 0;
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < 4 * kFixSeg; e += kT) {
+    const unsigned long long v = seg[e];
+    if (!v) continue;
+    const int r = e / kFixSeg;
+    atomicAdd(&Nfix[(b0 + e % kFixSeg + X * (r & 1) + XY * (r >> 1)) * g.S + s0], v);
   }
 }
 
@@ -1340,13 +1396,33 @@ int kstamp_collect(picard_ctx *c, int n) {
 
 // ---------------------------------------------------------------------------
 
+// Particles by (species, lower node): c->s.hist the buckets' starts, c->s.perm the
+// particles, those outside the grid counted.
+static int bucket_particles(picard_ctx *c) {
+  const GridDims &g = c->gd;
+  const int64_t n = c->n, nb = (int64_t)g.S * c->K;
+  PICARD_HIP(hipMemsetAsync(c->s.hist, 0, sizeof(int32_t) * (nb + 1), c->stream));
+  PICARD_HIP(hipMemsetAsync(c->s.counters, 0, sizeof(int32_t), c->stream));
+  if (n > 0)
+    k_dep_key<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, n, g, c->s.key, c->s.scan, c->s.hist,
+                                                        c->s.counters);
+  PICARD_HIP(hipGetLastError());
+  PICARD_TRY(scan_exclusive_i32(c, c->s.hist, c->s.hist, nb));
+  if (n > 0)
+    k_dep_scatter<<<grid_blocks(n, kT), kT, 0, c->stream>>>(n, c->s.key, c->s.hist, c->s.scan,
+                                                            c->s.perm);
+  PICARD_HIP(hipGetLastError());
+  return PICARD_OK;
+}
+
 static int launch_gridify_fixed(picard_ctx *c) {
   const GridDims &g = c->gd;
   const int64_t n = c->n;
-  PICARD_HIP(hipMemsetAsync(c->s.counters, 0, sizeof(int32_t), c->stream));
+  PICARD_TRY(bucket_particles(c));
   k_zero_u64<<<grid_blocks((int64_t)g.S * g.G, kT), kT, 0, c->stream>>>(c->Nfix, (int64_t)g.S * g.G);
   if (n > 0)
-    k_dep_fix64<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, n, g, c->Nfix, c->s.counters);
+    k_dep_fix64<<<grid_blocks(n, kT * 4), kT, 0, c->stream>>>(c->p, g, (int64_t)g.S * c->K, c->s.hist,
+                                                              c->s.perm, c->Nfix);
   k_fold_fix64<<<grid_blocks(g.G, kT), kT, 0, c->stream>>>(g, c->Nfix, c->N, c->C, c->consts);
   PICARD_HIP(hipGetLastError());
   PICARD_HIP(hipMemcpyAsync(c->host_counters, c->s.counters, sizeof(int32_t),
@@ -1365,23 +1441,13 @@ int launch_gridify(picard_ctx *c, bool flux) {
   const GridDims &g = c->gd;
   const int64_t n = c->n;
   const int64_t nb = (int64_t)g.S * c->K;
-  PICARD_HIP(hipMemsetAsync(c->s.hist, 0, sizeof(int32_t) * (nb + 1), c->stream));
-  PICARD_HIP(hipMemsetAsync(c->s.counters, 0, sizeof(int32_t), c->stream));
-  if (n > 0) {
-    k_dep_key<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, n, g, c->s.key, c->s.scan, c->s.hist,
-                                                        c->s.counters);
-    PICARD_HIP(hipGetLastError());
-  }
-  PICARD_TRY(scan_exclusive_i32(c, c->s.hist, c->s.hist, nb));
+  PICARD_TRY(bucket_particles(c));
   // the outflow's scratch, free here: the sorted indices and, over pairs of
   // its int32 arrays, the in-cell offsets
   int32_t *sorted = c->s.flags;
   double *rest[3];
   for (int d = 0; d < 3; ++d) rest[d] = reinterpret_cast<double *>(c->s.work[2 * d]);
   if (n > 0) {
-    k_dep_scatter<<<grid_blocks(n, kT), kT, 0, c->stream>>>(n, c->s.key, c->s.hist, c->s.scan,
-                                                            c->s.perm);
-    PICARD_HIP(hipGetLastError());
     if (flux)
       k_dep_order<false><<<grid_blocks(n, kT), kT, 0, c->stream>>>(
           c->p, g, nb, c->s.key, c->s.hist, c->s.perm, sorted, nullptr, nullptr, nullptr);
