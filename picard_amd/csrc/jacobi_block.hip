@@ -8,7 +8,7 @@
 // extent with a halo of T rows on every side, takes T sweeps on chip, each
 // valid on one row less all around, and stores the tile: one launch and one
 // trip to memory per T sweeps, for (TY + 2T)(TZ + 2T) / (TY TZ) times the loads
-// (from L2: an XCD's blocks own a z slab).  A wave owns one y row and all the tile's z planes
+// (from L2: an XCD's blocks own neighbouring tiles).  A wave owns one y row and all the tile's z planes
 // in registers, so z-neighbours are its own and x-neighbours come by wave
 // shifts; only the y-neighbours go through LDS, one write and two reads a row.
 // Every cell's arithmetic is k_jacobi_pass's, in its operand order; a periodic
@@ -50,14 +50,16 @@ __global__ void __launch_bounds__(64 * (TY + 2 * T)) k_jacobi_block(BlockGeo g,
                                                                      double *__restrict__ out,
                                                                      const double *__restrict__ b) {
   constexpr int NY = TY + 2 * T, NZ = TZ + 2 * T;
-  __shared__ double rows[NY][NZ][64 * CX];
+  // two copies where they fit: then one barrier a sweep
+  constexpr int NB = T > 2 && 2 * NY * NZ * CX * 512 <= 150 * 1024 ? 2 : 1;
+  __shared__ double rows[NB][NY][NZ][64 * CX];
   const int lane = (int)threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.y);
-  // tile: z tiles of XCD blockIdx.x % 8, y fastest
-  const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-  const int za = (xcd * g.nzt) >> 3, zb = ((xcd + 1) * g.nzt) >> 3;
-  const int tz = za + q / g.nyt, ty = q % g.nyt;
-  if (tz >= zb) return;                        // the whole block
+  // tile: an eighth of them, y fastest, to XCD blockIdx.x % 8 (whole z slabs gave
+  // some XCDs more tiles than CUs: 4.2 us a sweep at 40x60x70, now 2.4)
+  const int tile = (int)(blockIdx.x & 7) * (int)(gridDim.x >> 3) + (int)(blockIdx.x >> 3);
+  if (tile >= g.nyt * g.nzt) return;           // the whole block
+  const int tz = tile / g.nyt, ty = tile % g.nyt;
   const int y0 = ty * TY, z0 = tz * TZ;
   // the wave's row: interior (or an image of one), a flow guard, or nothing
   int y = y0 - T + w;
@@ -95,22 +97,25 @@ __global__ void __launch_bounds__(64 * (TY + 2 * T)) k_jacobi_block(BlockGeo g,
 #pragma unroll
     for (int c = 0; c < CX; ++c) {
       u[zi][c] = ur[xo[c]];
-      bf[zi][c] = br[xo[c]];
+      if (zi > 0 && zi < NZ - 1) bf[zi][c] = br[xo[c]];
     }
-    if (!PX) end[zi] = ur[eo];
+    if (!PX && zi > 0 && zi < NZ - 1) end[zi] = ur[eo];
   }
 #pragma unroll
-  for (int zi = 0; zi < NZ; ++zi) {
+  for (int zi = 1; zi < NZ - 1; ++zi) {
 #pragma unroll
     for (int c = 0; c < CX; ++c) bf[zi][c] = g.af * bf[zi][c];
   }
 #pragma unroll
   for (int s = 1; s <= T; ++s) {
-    if (s > 1) __syncthreads();                // the last sweep's reads
+    auto &buf = rows[NB == 2 ? s & 1 : 0];
+    if (NB == 1 && s > 1) __syncthreads();     // the last sweep's reads
+    if (w >= s - 1 && w <= NY - s) {           // those that a row of this sweep reads
 #pragma unroll
-    for (int zi = s; zi < NZ - s; ++zi)
+      for (int zi = s; zi < NZ - s; ++zi)
 #pragma unroll
-      for (int c = 0; c < CX; ++c) rows[w][zi][lane + 64 * c] = u[zi][c];
+        for (int c = 0; c < CX; ++c) buf[w][zi][lane + 64 * c] = u[zi][c];
+    }
     __syncthreads();
     if (!inner || w < s || w >= NY - s) continue;   // the whole wave
     // the y-neighbours of every plane first: one wait for LDS a sweep
@@ -119,10 +124,15 @@ __global__ void __launch_bounds__(64 * (TY + 2 * T)) k_jacobi_block(BlockGeo g,
     for (int zi = s; zi < NZ - s; ++zi)
 #pragma unroll
       for (int c = 0; c < CX; ++c) {
-        un[zi][c] = rows[w + 1][zi][lane + 64 * c];
-        us[zi][c] = rows[w - 1][zi][lane + 64 * c];
+        un[zi][c] = buf[w + 1][zi][lane + 64 * c];
+        us[zi][c] = buf[w - 1][zi][lane + 64 * c];
       }
-    {
+    // planes that all are swept, away from flow guards, without the selects
+    const bool every = T > 2 && (zin & (((1u << (NZ - 2 * s)) - 1) << s)) == (((1u << (NZ - 2 * s)) - 1) << s);
+#pragma unroll
+    for (int way = T > 2 ? 0 : 1; way < 2; ++way) {
+      const bool all = way == 0;
+      if (all != every) continue;
       double below[CX];
 #pragma unroll
       for (int c = 0; c < CX; ++c) below[c] = u[s - 1][c];
@@ -134,7 +144,7 @@ __global__ void __launch_bounds__(64 * (TY + 2 * T)) k_jacobi_block(BlockGeo g,
         // a plane that is not swept (a flow guard, or beyond one) keeps its
         // value by a select: a branch per row left each row's LDS reads and its
         // chain of ten operations unoverlapped (64^3: 3.4 us a sweep)
-        const bool swept = zin >> zi & 1;
+        const bool swept = all || (zin >> zi & 1);
 #pragma unroll
         for (int c = 0; c < CX; ++c) {
           double uw = lane_below(cur[c]), ue = lane_above(cur[c]);
@@ -172,10 +182,10 @@ template <int CX, int T, int TY, int TZ>
 void launch(hipStream_t s, BlockGeo g, const double *in, double *out, const double *b) {
   g.nyt = (g.ny + TY - 1) / TY;
   g.nzt = (g.nz + TZ - 1) / TZ;
-  const int slab = (g.nzt + 7) / 8;            // z tiles of an XCD, at most
+  const int blocks = (g.nyt * g.nzt + 7) / 8 * 8;
   const dim3 block(64, TY + 2 * T);
-  if (g.px) k_jacobi_block<CX, T, TY, TZ, true><<<8 * slab * g.nyt, block, 0, s>>>(g, in, out, b);
-  else k_jacobi_block<CX, T, TY, TZ, false><<<8 * slab * g.nyt, block, 0, s>>>(g, in, out, b);
+  if (g.px) k_jacobi_block<CX, T, TY, TZ, true><<<blocks, block, 0, s>>>(g, in, out, b);
+  else k_jacobi_block<CX, T, TY, TZ, false><<<blocks, block, 0, s>>>(g, in, out, b);
 }
 
 }  // namespace
@@ -186,25 +196,37 @@ bool jacobi_block_eligible(const GridDims &g) { return g.nx <= 128; }
 
 // Tile and sweeps per launch, by what is resident at once on 256 CUs: beyond
 // that a launch runs in rounds and every round pays the trip to memory. Measured,
-// us per sweep (a pass of one sweep: 11.1 at 32^3, 17 at 49x72x60, 15.9 at 64^3):
-//   rows to 64: 2x2 rows x 4 sweeps 1.68 at 32^3 (256 tiles; 4x4: 2.22);
-//   4x4 x 4 2.35 at 64^3 (256 tiles; x 2: 2.39, 2x2 x 4: 5.1);
-//   4x4 x 2 2.92 at 49x72x60 (270 tiles; x 4: 3.86) and 3.59 at 64x96x96
-//   (576; x 4: 5.9);
-//   rows to 128: 4x4 x 2 4.80 at 72^3 (324 tiles, two resident a CU; 6x6: 5.02)
-//   and 6.40 at 128x100x96 (600; 6x6, 272: 8.56); 6x6 x 2 5.22 at 96^3 (256,
+// us per sweep (a pass of one sweep: 11.1 at 32^3, 17 at 49x72x60, 15.9 at 64^3), 4.4 us of
+// a launch being its start, loads and stores:
+//   rows to 64, the smallest tile that has at most 256, x 4 sweeps: 2x2 1.59 at 32^3 (4x4: 2.2);
+//   3x3 1.83 at 48^3 (4x4: 2.05); 4x4 2.19 at 64^3 (x 2 sweeps: 2.4, 2x2 x 4: 5.1); 5x4
+//   2.40 at 49x72x60 and 6x4 2.71 at 64x96x64 (4x4 x 2: 2.92 and 3.16);
+//   beyond, 4x4 x 2 3.68 at 64x96x96 (576 tiles; 6x6 x 4: 4.04, registers spilled);
+//   rows to 128: 4x4 x 2 4.75 at 72^3 (324 tiles, two resident a CU; 6x6: 5.02)
+//   and 6.45 at 128x100x96 (600; 6x6, 272: 8.56); 6x6 x 2 5.21 at 96^3 (256,
 //   one a CU; 4x4, 576: 6.63).
-enum BlockPlan { kRows22x4, kRows44x4, kRows44x2, kWide44x2, kWide66x2 };
+// Before the planes that a sweep needs alone were loaded and stored in LDS, the rows kept
+// twice there (one barrier a sweep) and the selects left out away from flow guards: 1.69
+// at 32^3, 2.39 at 64^3.
+enum BlockPlan { kRows22x4, kRows33x4, kRows44x4, kRows54x4, kRows64x4, kRows44x2, kWide44x2, kWide66x2 };
 
 static BlockPlan block_plan(const GridDims &g) {
-  auto tiles = [&](int t) { return (int64_t)((g.ny + t - 1) / t) * ((g.nz + t - 1) / t); };
-  if (g.nx <= 64) return tiles(2) <= 256 ? kRows22x4 : (tiles(4) <= 256 ? kRows44x4 : kRows44x2);
-  return tiles(6) <= 256 && tiles(4) > 512 ? kWide66x2 : kWide44x2;
+  auto tiles = [&](int ty, int tz) {
+    return (int64_t)((g.ny + ty - 1) / ty) * ((g.nz + tz - 1) / tz);
+  };
+  if (g.nx <= 64) {
+    if (tiles(2, 2) <= 256) return kRows22x4;
+    if (tiles(3, 3) <= 256) return kRows33x4;
+    if (tiles(4, 4) <= 256) return kRows44x4;
+    if (tiles(5, 4) <= 256) return kRows54x4;
+    return tiles(6, 4) <= 256 ? kRows64x4 : kRows44x2;
+  }
+  return tiles(6, 6) <= 256 && tiles(4, 4) > 512 ? kWide66x2 : kWide44x2;
 }
 
 int jacobi_block_sweeps(const GridDims &g) {
   const BlockPlan p = block_plan(g);
-  return p == kRows22x4 || p == kRows44x4 ? 4 : 2;
+  return p <= kRows64x4 ? 4 : 2;
 }
 
 // Iterates from -> from + jacobi_block_sweeps * launches in the rotating
@@ -230,7 +252,10 @@ int launch_jacobi_block(picard_ctx *c, int64_t from, int64_t launches) {
     double *out = c->jb[(from + T) % 3];
     switch (plan) {
       case kRows22x4: launch<1, 4, 2, 2>(c->stream, bg, in, out, c->b); break;
+      case kRows33x4: launch<1, 4, 3, 3>(c->stream, bg, in, out, c->b); break;
       case kRows44x4: launch<1, 4, 4, 4>(c->stream, bg, in, out, c->b); break;
+      case kRows54x4: launch<1, 4, 5, 4>(c->stream, bg, in, out, c->b); break;
+      case kRows64x4: launch<1, 4, 6, 4>(c->stream, bg, in, out, c->b); break;
       case kRows44x2: launch<1, 2, 4, 4>(c->stream, bg, in, out, c->b); break;
       case kWide44x2: launch<2, 2, 4, 4>(c->stream, bg, in, out, c->b); break;
       case kWide66x2: launch<2, 2, 6, 6>(c->stream, bg, in, out, c->b); break;

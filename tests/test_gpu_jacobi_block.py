@@ -28,6 +28,9 @@ pytestmark = pytest.mark.gpu
     ((127, 4, 5), (False, False, True), dict(maxit=2000)),
     ((129, 4, 6), (True, False, True), dict(maxit=2000)),               # wider: one sweep per launch
     ((66, 97, 92), (True, False, False), dict(maxit=60)),  # tiles of six rows
+    ((11, 41, 47), (True, False, True), dict(maxit=300)),  # of 3 x 3
+    ((33, 66, 65), (False, True, False), dict(maxit=60)),  # of 5 x 4
+    ((10, 86, 62), (True, False, False), dict(maxit=120)),              # of 6 x 4
     ((20, 18, 16), (True, False, False), dict(maxerr=1e-30, maxit=201)),
     ((20, 18, 16), (False, True, True), dict(maxit=120)),
 ])
