@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <hip/hip_ext.h>
 
+#include "bisect.h"
 #include "cic.h"
 #include "picard_internal.h"
 #include "reduce.h"
@@ -175,17 +176,6 @@ __global__ void __launch_bounds__(kT) k_dep_gather(ParticlesF64 p, GridDims g, c
 // twice as many the first two are slower by half.
 constexpr int kRowSeg = 64;              // nodes of a block at most: one wave adds them
 constexpr int kRowCap = 1024;            // particles in LDS: 30 KB, five blocks per CU
-
-// entries of d[lo .. hi), descending, greater than q
-__device__ __forceinline__ int greater_in(const int32_t *d, int lo, int hi, int32_t q) {
-  const int first = lo;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (d[mid] > q) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo - first;
-}
 
 // F1..F8 of ParticlesGridify.f90:81-88: node offset 1 takes rest, 0 takes dx - rest
 __device__ __forceinline__ double dep_weight(const GridDims &g, bool ox, bool oy, bool oz, double x,
