@@ -35,11 +35,13 @@ jobs/s, 32^3-160^3 grids, step counts scaled by 1/100), run after the forms
 and reported as `server` in the same line (`--no-server` skips it; `--server`
 runs it alone with its own options).
 
-Prints one JSON line with the roofline of the dominant kernel (the split
-form's FP32 Jacobi sweep, timed live over one launch in 16 by the kernel's
-own clock, with HIP events around the same launches beside it), the rate a
-plain stream with the same byte mix and array size reaches beside it, and a
-CPU baseline of the oracle on a bounded sample."""
+Prints one JSON line with the roofline of the split form's largest phase, the
+particles' sort (timed live through BCoutflow, a push before each call), and a CPU
+baseline of the oracle on a bounded sample.  With --sweeps-per-launch, which makes the
+split solve sweep all the way, or --form fp64 it is the roofline of the Jacobi sweep
+instead: timed live over one launch in 16 by the kernel's own clock, with HIP
+events around the same launches beside it, and the rate that a plain stream with the same
+byte mix and array size reaches."""
 from __future__ import annotations
 
 import argparse
@@ -67,13 +69,35 @@ def _rel(a, b):
     return float(np.linalg.norm(a - b) / nb) if nb > 0 else float(np.linalg.norm(a))
 
 
+# bytes a particle of the split form's sort: counting pass 19 read (cell 6, offset 12, species 1)
+# and 4 written (rank), scatter 39 read (all 35 and the rank) and 35 written
+SORT_BYTES = 19 + 4 + 39 + 35
+
+
+def sort_rate(dom, reps=3):
+    """The sort (counting pass, scan, scatter) through BCoutflow, each after
+    a push of every particle and between synchronizations; the fastest."""
+    best = None
+    for _ in range(reps):
+        dom.advance_position()
+        dom.synchronize()
+        n = dom.num_local
+        t = time.perf_counter()
+        dom.bc_outflow()
+        dom.synchronize()
+        t = time.perf_counter() - t
+        if best is None or t < best["seconds"]:
+            best = {"seconds": t, "particles": n}
+    return best
+
+
 def run_form(cfg, precision, steps, warmup, capture_after=1, order_free=False,
              sweeps_per_launch=0):
     """W warmup + K timed steps of one form; returns timings (whole and per
     step, with the solve phase's wall time per step from HIP events) and the
     fields after step `capture_after` (read outside the timed region).
-    sweeps_per_launch > 0 caps the split solve's sweeps per launch (else the
-    library's default, 2)."""
+    sweeps_per_launch > 0 makes the split solve sweep, with at most that many
+    per launch."""
     from picard_amd import _lib, host
     d = host.derive(cfg)
     ncell = cfg.nx * cfg.ny * cfg.nz
@@ -131,6 +155,7 @@ def run_form(cfg, precision, steps, warmup, capture_after=1, order_free=False,
     if fields is None:
         fields = {k: dom.field(w) for k, w in (("U", _lib.FIELD_U), ("E", _lib.FIELD_E),
                                                 ("N", _lib.FIELD_N))}
+    sort = sort_rate(dom) if precision == _lib.PICARD_FP32_SPLIT else None
     dom.close()
     log(f"{name}: {steps} steps in {elapsed:.2f} s, sweeps {sweeps}, solve phase "
         f"{solve_ms / max(solves, 1):.1f} ms per step, solve kernel "
@@ -139,7 +164,7 @@ def run_form(cfg, precision, steps, warmup, capture_after=1, order_free=False,
     return dict(pushed=pushed, elapsed=elapsed, sweeps=sweeps, jac_ms=jac_ms,
                 jac_launches=jac_launches, jac_sweeps=jac_sweeps, clk_ms=clk_ms,
                 clk_launches=clk_launches, solve_ms=solve_ms,
-                solves=solves, per_step=per_step,
+                solves=solves, per_step=per_step, sort=sort,
                 warm_steps=warm_steps, fields=fields, captured_at=min(capture_after, it))
 
 
@@ -218,6 +243,8 @@ def solve_only(cfg, form, sweeps, inner=0):
     d = host.derive(cfg)
     prec = _lib.PICARD_FP32_SPLIT if form == "split" else _lib.PICARD_FP64
     dom = host.Domain(cfg, max_particles=1024, d=d, precision=prec)
+    if form == "split":                 # a choice of sweeps makes the solve sweep all the way
+        dom.split_sweeps_per_launch(2)
     if inner > 0 and form == "split":
         dom.split_solver(inner)
     dom.calc_distance()
@@ -516,8 +543,8 @@ def main():
                     help="error mode: N steps of both forms from the same plasma, split vs FP64 "
                          "errors per step and particle trajectories after the last")
     ap.add_argument("--sweeps-per-launch", type=int, default=0, choices=(0, 1, 2, 3),
-                    help="at most this many FP32 sweeps per launch of the split solve "
-                         "(0: the library's default, 2)")
+                    help="make the split solve sweep all the way, at most this many FP32 sweeps "
+                         "per launch (0: the library's default, the solve in the eigenbasis)")
     ap.add_argument("--stream-ref", type=int, default=0, metavar="N",
                     help="print the stream reference rate for N float32 elements and exit")
     ap.add_argument("--stream-rates", action="store_true",
@@ -685,32 +712,10 @@ def main():
                else "k_mx_pair") if spl["split"] > 1.5 else "k_mx_sweep")
              if headname == "split"
              else ("k_jacobi_pass2" if cfg.nx % 2 == 0 else "k_jacobi_pass"))
-    stream = stream_reference(ncell) if headname == "split" else None
-    out = {
-        "metric": METRIC,
-        "value": value,
-        "unit": "particle-steps/s",
-        "n_gpus": 1,
-        "steps": head_steps,
-        "warmup": args.warmup,
-        "ms_per_step": 1e3 * head["elapsed"] / head_steps,
-        "higher_is_better": True,
-        "scaling": "weak",
-        "vs_baseline": None,
-        "dtype": "f32+f64" if headname == "split" else "f64",
-        "data": "synthetic (device Philox plasma, inflow and Haser production)",
-        "config": {
-            "workload": f"{cfg.nx}^3 cells dx=10 m, H+ and e- at 32 per cell, 400 km/s, 10 eV, "
-                        f"B=(0,0,5 nT), x in/outflow, y/z periodic, dt=0.1/w_pe, Jacobi tol 1e-6, "
-                        f"Haser 18 amu source Q={host.HASER_Q_USED:.2g}/s (stated "
-                        f"{host.HASER_Q_STATED:.0e}/s scaled to ~2^18 ions/step), "
-                        f"value = {headname} form",
-            "grid": [cfg.nx, cfg.ny, cfg.nz],
-            "forms": per_form,
-            "split_over_fp64": ratio,
-            "split_error_vs_fp64": errors,
-        },
-        "roofline": {
+    swept = headname == "fp64" or args.sweeps_per_launch > 0
+    stream = stream_reference(ncell) if headname == "split" and swept else None
+    if swept:
+        roofline = {
             "bound": "hbm",
             "kernel": kname,
             "achieved": achieved,
@@ -737,7 +742,52 @@ def main():
                                               "step's end calls for it"}.get(kname, kname),
             "stream_reference": stream,
             "frac_of_stream": (achieved / stream["GBs"]) if stream else None,
+        }
+    else:
+        # the split form solves the field in its eigenbasis; its step's largest part is
+        # the particles' sort, timed live after the steps
+        sort = head["sort"]
+        moved = SORT_BYTES * sort["particles"]
+        achieved = moved / sort["seconds"] / 1e9
+        roofline = {
+            "bound": "hbm",
+            "kernel": "k_sp_scatter",
+            "phase": "the particles' sort: k_sp_flag, scan, k_sp_scatter",
+            "achieved": achieved,
+            "peak": HBM_PEAK_GBS,
+            "unit": "GB/s",
+            "frac": achieved / HBM_PEAK_GBS,
+            "traffic": traffic_from_profiles("k_sp_scatter"),
+            "bytes_per_particle": SORT_BYTES,
+            "particles": sort["particles"],
+            "phase_ms": 1e3 * sort["seconds"],
+            "duration_from": "host clock between synchronizations, the fastest of 3 calls",
+        }
+    out = {
+        "metric": METRIC,
+        "value": value,
+        "unit": "particle-steps/s",
+        "n_gpus": 1,
+        "steps": head_steps,
+        "warmup": args.warmup,
+        "ms_per_step": 1e3 * head["elapsed"] / head_steps,
+        "higher_is_better": True,
+        "scaling": "weak",
+        "vs_baseline": None,
+        "dtype": "f32+f64" if headname == "split" else "f64",
+        "data": "synthetic (device Philox plasma, inflow and Haser production)",
+        "config": {
+            "workload": f"{cfg.nx}^3 cells dx=10 m, H+ and e- at 32 per cell, 400 km/s, 10 eV, "
+                        f"B=(0,0,5 nT), x in/outflow, y/z periodic, dt=0.1/w_pe, Jacobi tol 1e-6, "
+                        f"Haser 18 amu source Q={host.HASER_Q_USED:.2g}/s (stated "
+                        f"{host.HASER_Q_STATED:.0e}/s scaled to ~2^18 ions/step), "
+                        f"value = {headname} form",
+            "grid": [cfg.nx, cfg.ny, cfg.nz],
+            "forms": per_form,
+            "split_over_fp64": ratio,
+            "split_error_vs_fp64": errors,
         },
+        "roofline": roofline,
         "cpu_baseline": None,
     }
     if not args.no_server and args.form == "both":
