@@ -367,7 +367,9 @@ def ensemble_bench(count, steps, warmup, tune_sweeps=32, baseline=True, seed=202
                tile=dict(cells_per_thread=tile.cells_per_thread, blocks_per_cu=tile.blocks_per_cu),
                tuner_us_per_sweep=[float(v) for v in times],
                solve_fraction=solve_ms / 1e3 / el,
-               solve_sweep_bytes_per_s=12.0 * cell_sweeps / (solve_ms / 1e3) if solve_ms else 0.0,
+               # of solves by sweeps; in closed form none is taken
+               solve_sweep_bytes_per_s=(12.0 * cell_sweeps / (solve_ms / 1e3)
+                                        if solve_ms and any(q["chunks"] for q in per) else None),
                sims=count, cells=int(sum(s.cells for s in specs)))
     if baseline:
         tot_ps, tot_s = 0, 0.0
@@ -528,7 +530,7 @@ def main():
                          "FP64 step at 256^3 takes ~23 s, a split one ~4 s)")
     ap.add_argument("--fp64-warmup", type=int, default=1)
     ap.add_argument("--no-order-free", action="store_true",
-                    help="skip the order-free FP64 form (fixed-point deposit, FFT face sums)")
+                    help="skip the order-free FP64 form (fixed-point deposit, face sums by modes)")
     ap.add_argument("--grid", type=int, default=256)
     ap.add_argument("--form", choices=("both", "split", "fp64"), default="both")
     ap.add_argument("--no-cpu-baseline", action="store_true")

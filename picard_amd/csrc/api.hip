@@ -235,6 +235,7 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
     PICARD_TRY(dalloc(&c->jb_mem[q], g.G + 2));
     c->jb[q] = c->jb_mem[q] + 1;
   }
+  PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->js_host), kHostState));
   if (spec_eligible(c)) PICARD_TRY(spec_create(c));
   PICARD_TRY(dalloc(&c->b_mem, g.G + 2));
   c->b = c->b_mem + 1;
@@ -266,7 +267,6 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   if (pb < 8 * 256) pb = 8 * 256;                 // the Jacobi pass kernels: at most 256 blocks per XCD
   c->s.partials_len = pb;
   PICARD_TRY(dalloc(&c->s.partials, 4 * pb));     // two launches' worth (read + write) and scratch
-  PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->js_host), sizeof(JacobiState)));
   // allocating its chunks, 0.25 ms each pair, is worth it from a few MB on
   c->readback = new Readback(int64_t(4) << 20);
   PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->host_counters), 16 * sizeof(int32_t)));

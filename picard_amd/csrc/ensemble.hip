@@ -1111,6 +1111,7 @@ __global__ void __launch_bounds__(kT) k_sp_faces(Arenas A) {
     const double *M = sd.inv[AXIS] + (AXIS == 1 ? j : k);
     const int n = AXIS == 1 ? sd.ny : sd.nz, np = spec_cols(n), ld = AXIS == 1 ? 1 : sd.ny;
     double v = 0.0;
+#pragma unroll 8
     for (int o = 0; o < n; ++o) v += M[(int64_t)o * np] * in[(int64_t)o * ld];
     if (AXIS == 1) {
       A.sp[1][sd.sbase + (int64_t)tl.a * fn + q] = v;
@@ -1148,6 +1149,7 @@ __global__ void __launch_bounds__(kT) k_sp_distance_eig(Arenas A, int slot) {
     const double *in = A.sp[AXIS - 1] + sd.sbase + x +
                        (AXIS == 1 ? (int64_t)sd.PX * sd.ny * z : (int64_t)sd.PX * y);
     double v = 0.0;
+#pragma unroll 8
     for (int o = 0; o < n; ++o) v += sd.fwd[AXIS][(int64_t)o * np + kc] * in[o * ld];
     v /= sd.fwd[AXIS][kc];
     if (AXIS == 1) A.sp[1][sd.sbase + t] = v;

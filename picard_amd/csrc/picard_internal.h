@@ -110,6 +110,7 @@ struct DeviceScratch {
 
 struct SpecState;                  // spectral.hip
 class Readback;                    // readback.h
+constexpr int kHostState = 1024;   // bytes of the solve's pinned mirrors
 
 }  // namespace picard
 
@@ -124,7 +125,7 @@ struct picard_ctx {
   int64_t n = 0;             // num_local (authoritative on the host)
   picard::ParticlesF64 p{};
   bool split = false;        // PICARD_FP32_SPLIT
-  // FP64 form with PICARD_DEPOSIT_FIXED_POINT: fixed-point deposit and FFT
+  // FP64 form with PICARD_DEPOSIT_FIXED_POINT: fixed-point deposit and mode-by-mode
   // face sums (order-free, within 1e-12 of the reference order)
   bool order_free = false;
   picard::ParticlesSplit ps{}, ps2{};
@@ -183,7 +184,8 @@ struct picard_ctx {
   double *spec_inv[3] = {nullptr, nullptr, nullptr};
   double *spec_eig[3] = {nullptr, nullptr, nullptr};   // and eigenvalue parts
   double spec_lnmax = 0.0;                             // largest ln|lambda|
-  picard::SpecState *spec_st = nullptr, *spec_host = nullptr;
+  double *spec_mem = nullptr;    // the allocation of all of these
+  picard::SpecState *spec_st = nullptr, *spec_host = nullptr;   // its pinned mirror: behind js_host
 
   // number fluxes of ParticlesGridifyAll (allocated on first use)
   double *F = nullptr;                 // F(species, 3, node)

@@ -20,8 +20,8 @@
 //
 // Cost: nine axis transforms of 2 n operations a cell, whatever the number of
 // sweeps (about 3 n^2 to 1e-6).  Measured, whole solve with its last sweeps
-// against sweeping: 16^3 0.29 ms (FP32 sweeps 7.3), 64^3 0.5 ms (FP64 sweeps 280),
-// 128^3 to 1e-10 1.7 ms (FP32 sweeps 620), 160^3 2.5 ms (FP32 sweeps 880).
+// against sweeping: 16^3 0.19 ms (FP32 sweeps 7.3), 64^3 0.37 ms (FP64 sweeps 280),
+// 128^3 to 1e-10 0.74 ms (FP32 sweeps 620), 160^3 1.1 ms (FP32 sweeps 880).
 // Against the FP64 form that sweeps all the way U differs by 2e-15 to 3e-13
 // (the FP32 sweeps differed by 5e-7 to 5e-6) and the sweep counts are equal.
 #include <algorithm>
@@ -65,7 +65,9 @@ struct SpecGeo {
   const double *eig[3];             // per axis: 4 a sin^2 (n values), then 4 a cos^2
 };
 
-__global__ void __launch_bounds__(kT) k_spec_basis(int n, int flow, double *fwd, double *inv) {
+// A basis, its transpose and, unless eig is null, the axis' eigenvalue rows.
+__global__ void __launch_bounds__(kT) k_spec_basis(int n, int flow, double a, double *fwd, double *inv,
+                                                   double *eig) {
   const int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x;
   const int np = spec_cols(n);
   if (t >= spec_mat_len(n)) return;
@@ -73,15 +75,12 @@ __global__ void __launch_bounds__(kT) k_spec_basis(int n, int flow, double *fwd,
   const bool in = r < n && c < n;
   fwd[t] = in ? spec_basis(n, flow != 0, r, c) : 0.0;
   inv[t] = in ? spec_basis(n, flow != 0, c, r) : 0.0;
-}
-
-__global__ void __launch_bounds__(kT) k_spec_eig(int n, int flow, double a, double *eig) {
-  const int k = (int)blockIdx.x * kT + (int)threadIdx.x;
-  if (k >= n) return;
-  const double h = spec_half_angle(n, flow != 0, k);
-  const double s = sinpi(h), c = cospi(h);
-  eig[k] = 4.0 * a * s * s;
-  eig[n + k] = 4.0 * a * c * c;
+  if (eig && r == 0 && c < n) {
+    const double h = spec_half_angle(n, flow != 0, c);
+    const double s = sinpi(h), q = cospi(h);
+    eig[c] = 4.0 * a * s * s;
+    eig[n + c] = 4.0 * a * q * q;
+  }
 }
 
 // Ends a reduction: true in the block that finishes last, after every
@@ -363,19 +362,13 @@ bool spec_eligible(const picard_ctx *c) {
 }
 
 void spec_release(picard_ctx *c) {
-  for (double *&p : c->spec_buf)
-    if (p) (void)hipFree(p), p = nullptr;
-  for (int d = 0; d < 3; ++d)
-    for (double **p : {&c->spec_fwd[d], &c->spec_inv[d], &c->spec_eig[d]})
-      if (*p) (void)hipFree(*p), *p = nullptr;
-  if (c->spec_st) (void)hipFree(c->spec_st), c->spec_st = nullptr;
-  if (c->spec_host) (void)hipHostFree(c->spec_host), c->spec_host = nullptr;
+  if (c->spec_mem) (void)hipFree(c->spec_mem);
+  c->spec_mem = nullptr;
 }
 
 // Basis, transpose and eigenvalue parts of one axis; `a` is the Jacobi weight of its neighbours.
 int spec_axis_tables(hipStream_t s, int n, bool flow, double a, double *fwd, double *inv, double *eig) {
-  k_spec_basis<<<grid_blocks(spec_mat_len(n), kT), kT, 0, s>>>(n, flow, fwd, inv);
-  if (eig) k_spec_eig<<<grid_blocks(n, kT), kT, 0, s>>>(n, flow, a, eig);
+  k_spec_basis<<<grid_blocks(spec_mat_len(n), kT), kT, 0, s>>>(n, flow, a, fwd, inv, eig);
   PICARD_HIP(hipGetLastError());
   return PICARD_OK;
 }
@@ -407,21 +400,34 @@ int spec_create(picard_ctx *c) {
   const int n[3] = {g.nx, g.ny, g.nz};
   const double d2[3] = {g.dxyz[0] * g.dxyz[0], g.dxyz[1] * g.dxyz[1], g.dxyz[2] * g.dxyz[2]};
   const double sum = 1.0 / d2[0] + 1.0 / d2[1] + 1.0 / d2[2];
-  const int64_t len = (int64_t)((g.nx + 15) & ~15) * g.ny * g.nz;
-  for (double *&p : c->spec_buf) PICARD_HIP(hipMalloc(&p, sizeof(double) * len));
+  // one allocation, its parts at multiples of 256 bytes
+  auto part = [](int64_t doubles) { return (doubles + 31) & ~int64_t(31); };
+  const int64_t len = part((int64_t)((g.nx + 15) & ~15) * g.ny * g.nz);
+  const int64_t state = part((int64_t)(sizeof(SpecState) + sizeof(double) - 1) / (int64_t)sizeof(double));
+  int64_t total = 3 * len + state;
+  for (int d = 0; d < 3; ++d) total += 2 * spec_mat_len(n[d]) + part(2 * n[d]);
+  PICARD_HIP(hipMalloc(&c->spec_mem, sizeof(double) * total));
+  double *p = c->spec_mem;
+  auto take = [&](int64_t doubles) {
+    double *q = p;
+    p += doubles;
+    return q;
+  };
+  for (double *&b : c->spec_buf) b = take(len);
   double w[3];
   for (int d = 0; d < 3; ++d) {
-    PICARD_HIP(hipMalloc(&c->spec_fwd[d], sizeof(double) * spec_mat_len(n[d])));
-    PICARD_HIP(hipMalloc(&c->spec_inv[d], sizeof(double) * spec_mat_len(n[d])));
-    PICARD_HIP(hipMalloc(&c->spec_eig[d], sizeof(double) * 2 * n[d]));
+    c->spec_fwd[d] = take(spec_mat_len(n[d]));     // a multiple of 16 x 64 doubles
+    c->spec_inv[d] = take(spec_mat_len(n[d]));
+    c->spec_eig[d] = take(part(2 * n[d]));
     w[d] = 0.5 / (d2[d] * sum);                       // ax, ay, az of CalcEpotential.f90:44-47
     PICARD_TRY(spec_axis_tables(c->stream, n[d], g.flow[d], w[d], c->spec_fwd[d], c->spec_inv[d],
                                 c->spec_eig[d]));
   }
   c->spec_lnmax = spec_slowest(n, g.flow, w);
-  PICARD_HIP(hipMalloc(&c->spec_st, sizeof(SpecState)));
+  c->spec_st = reinterpret_cast<SpecState *>(take(state));
   PICARD_HIP(hipMemsetAsync(c->spec_st, 0, sizeof(SpecState), c->stream));
-  PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->spec_host), sizeof(SpecState)));
+  static_assert(sizeof(JacobiState) <= kHostState / 2 && sizeof(SpecState) <= kHostState / 2, "pinned mirrors");
+  c->spec_host = reinterpret_cast<SpecState *>(reinterpret_cast<char *>(c->js_host) + kHostState / 2);
   return PICARD_OK;
 }
 

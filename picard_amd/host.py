@@ -468,7 +468,7 @@ class Domain:
     def __init__(self, cfg: Config, max_particles: int | None = None, device: int = 0,
                  d: Derived | None = None, precision: int = _lib.PICARD_FP64,
                  order_free: bool = False):
-        """order_free: the FP64 form with the fixed-point deposit and the FFT
+        """order_free: the FP64 form with the fixed-point deposit and the mode-by-mode
         face sums (PICARD_DEPOSIT_FIXED_POINT) instead of the reference's
         summation orders."""
         self.cfg = cfg
