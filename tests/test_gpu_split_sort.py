@@ -61,3 +61,23 @@ def test_step_is_its_phases(dims, flow, ppc, speed):
     assert out[0][0] == out[1][0]
     assert np.array_equal(out[0][1], out[1][1])
     assert np.array_equal(out[0][2], out[1][2])
+
+
+def test_step_that_fails_has_pushed():
+    """A step whose produced particles do not fit ends after its push, as the phases would."""
+    cfg = host.Config(nx=6, ny=5, nz=4, flow=(True, False, False), gmin=(-30.0, -25.0, -20.0),
+                      gmax=(30.0, 25.0, 20.0), ppc=(0, 3, 0, 0, 0, 0, 0, 0))
+    d = host.derive(cfg)
+    out = []
+    for fused in (True, False):
+        dom = host.Domain(cfg, max_particles=6 * 5 * 4 * 6 + 5, d=d, precision=_lib.PICARD_FP32_SPLIT)
+        dom.calc_distance()
+        dom.generate_initial(9)
+        if fused:
+            with pytest.raises(_lib.PicardError):
+                dom.step((np.zeros((50, 8)), np.ones(50, np.int32)))
+        else:
+            dom.advance_position()
+        out.append(_rows(dom))
+        dom.close()
+    assert np.array_equal(out[0], out[1])
