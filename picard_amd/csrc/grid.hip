@@ -1232,11 +1232,13 @@ constexpr double kFix48 = 281474976710656.0;          // 2^48
 constexpr double kFix48Inv = 1.0 / 281474976710656.0;
 
 // The particles come bucketed by (species, lower node) as for the reference order, but in
-// no order within a bucket: a thread takes four in turn, adds the weights of a run of one
-// bucket in registers, and a block's runs go to LDS: their corners fall in four segments of
-// nodes, b0 + {0, X, XY, XY + X} + [0, kFixSeg), of its first particle's species (a run beyond
-// goes to memory).  One atomic per corner and particle took 1.10 ms at 6.3e6 particles, 12 a
-// cell and species; the counting, the scatter and this take 0.16 + 0.03 + 0.29.
+// no order within a bucket.  A block takes 256 of them, one a thread, and adds their weights
+// in LDS: their corners fall in four segments of
+// nodes, b0 + {0, X, XY, XY + X} + [0, kFixSeg), of its first particle's species (a particle
+// beyond goes to memory).  One atomic in memory per corner and particle took 1.10 ms at 6.3e6
+// particles, 12 a cell and species; the counting, the scatter and this take 0.16 + 0.03 + 0.15
+// (two a thread 0.16, four 0.18; four on end, a run's weights added in registers first, 0.29:
+// its reads then lie four apart).
 constexpr int kFixSeg = 256;
 
 // (unsigned long long)llrint(F 2^48), 0 <= F <= 1 (NaN: 0): the sum with 2^52 rounds to
@@ -1253,53 +1255,34 @@ __global__ void __launch_bounds__(kT) k_dep_fix64(ParticlesF64 p, GridDims g, in
   __shared__ unsigned long long seg[4 * kFixSeg];
   __shared__ int64_t first;
   __shared__ int species;
-  const int64_t n = off[nb];
-  const int64_t q0 = ((int64_t)blockIdx.x * kT + threadIdx.x) * 4;
-  if ((int64_t)blockIdx.x * kT * 4 >= n) return;               // block-uniform
+  const int64_t n = off[nb], q0 = (int64_t)blockIdx.x * kT, t = q0 + threadIdx.x;
+  if (q0 >= n) return;                                         // block-uniform
   for (int e = threadIdx.x; e < 4 * kFixSeg; e += kT) seg[e] = 0;
   const int64_t X = g.X, XY = (int64_t)g.X * g.Y;
-  int64_t node[4];
-  int sp[4];
-  double rest[4][3];
-#pragma unroll
-  for (int h = 0; h < 4; ++h) {
-    const int32_t q = perm[q0 + h < n ? q0 + h : n - 1];
-    const CicLoc L = cic_locate(g, p.r[0][q], p.r[1][q], p.r[2][q]);
-    node[h] = node_index(g, L.idx[0], L.idx[1], L.idx[2]);
-    sp[h] = p.sp[q] - 1;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) rest[h][d] = L.rest[d];
-  }
+  const int32_t q = perm[t < n ? t : n - 1];
+  const CicLoc L = cic_locate(g, p.r[0][q], p.r[1][q], p.r[2][q]);
+  const int64_t node = node_index(g, L.idx[0], L.idx[1], L.idx[2]);
+  const int sp = p.sp[q] - 1;
   if (threadIdx.x == 0) {
-    first = node[0];
-    species = sp[0];
+    first = node;
+    species = sp;
   }
   __syncthreads();
   const int64_t b0 = first;
   const int s0 = species;
-  unsigned long long W[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-  for (int h = 0; h < 4; ++h) {
-    if (q0 + h >= n) break;
-#pragma unroll
-    for (int o = 0; o < 8; ++o) {
-      const double fx = (o & 1) ? rest[h][0] : g.dxyz[0] - rest[h][0];
-      const double fy = (o & 2) ? rest[h][1] : g.dxyz[1] - rest[h][1];
-      const double fz = (o & 4) ? rest[h][2] : g.dxyz[2] - rest[h][2];
-      W[o] += fix48(fx * fy * fz / g.dV);
-    }
-    if (h < 3 && q0 + h + 1 < n && node[h + 1] == node[h] && sp[h + 1] == sp[h]) continue;
-    const int64_t at = node[h] - b0;
-    const bool in = sp[h] == s0 && at >= 0 && at + 1 < kFixSeg;
+  if (t < n) {
+    const int64_t at = node - b0;
+    const bool in = sp == s0 && at >= 0 && at + 1 < kFixSeg;
 #pragma unroll
     for (int o = 0; o < 8; ++o) {
+      const unsigned long long w =
+          fix48(dep_weight(g, o & 1, o & 2, o & 4, L.rest[0], L.rest[1], L.rest[2]));
       if (in) {
-        atomicAdd(&seg[(o >> 1) * kFixSeg + (int)at + (o & 1)], W[o]);
+        atomicAdd(&seg[(o >> 1) * kFixSeg + (int)at + (o & 1)], w);
       } else {
-        const int64_t to = node[h] + (o & 1) + X * ((o >> 1) & 1) + XY * (o >> 2);
-        atomicAdd(&Nfix[to * g.S + sp[h]], W[o]);
+        const int64_t to = node + (o & 1) + X * ((o >> 1) & 1) + XY * (o >> 2);
+        atomicAdd(&Nfix[to * g.S + sp], w);
       }
-      W[o] = 0;
     }
   }
   __syncthreads();
@@ -1411,7 +1394,7 @@ static int launch_gridify_fixed(picard_ctx *c) {
   PICARD_TRY(bucket_particles(c));
   k_zero_u64<<<grid_blocks((int64_t)g.S * g.G, kT), kT, 0, c->stream>>>(c->Nfix, (int64_t)g.S * g.G);
   if (n > 0)
-    k_dep_fix64<<<grid_blocks(n, kT * 4), kT, 0, c->stream>>>(c->p, g, (int64_t)g.S * c->K, c->s.hist,
+    k_dep_fix64<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, g, (int64_t)g.S * c->K, c->s.hist,
                                                               c->s.perm, c->Nfix);
   k_fold_fix64<<<grid_blocks(g.G, kT), kT, 0, c->stream>>>(g, c->Nfix, c->N, c->C, c->consts);
   PICARD_HIP(hipGetLastError());
