@@ -126,7 +126,8 @@ __global__ void __launch_bounds__(kT) k_sp_flag(ParticlesSplit p, int64_t n, int
     float f[3];
     if (q < n && sort_coords(p, q, npush, g, wrap, dtdx, c, f)) k[h] = sort_key(g, c, p.sp[q]);
   }
-  count_keys(k, r, hist, win);
+  const int32_t row = (g.nx + 1) * g.S;
+  count_keys(k, r, hist, win, row, row * (g.ny + 1));
 #pragma unroll
   for (int h = 0; h < PER; ++h) {
     const int64_t q = q0 + h * kT;

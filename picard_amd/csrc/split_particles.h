@@ -72,54 +72,69 @@ __device__ __forceinline__ int32_t wave_add1(int32_t *counter, int32_t k) {
 
 // Places of a block's keys in a counting sort: hist[k] gains each key's count, r[h] is
 // the particle's rank among all of its key (-1 for k[h] < 0).  A block takes PER x
-// 256 consecutive particles; they arrive nearly sorted, so most keys lie in a
-// short stretch from the first ones': those are counted in LDS (the count
-// before is the rank within the block), each key then takes one atomic on its
-// histogram entry, whose return places the block's particles of that key.
-// The other keys (particles that moved a row or a plane on) are added a wave at
-// a time.  With the ranks known the scatter adds nothing: at 128^3 with 64 particles a
-// cell (1.4e8) flag and scatter take 1.13 + 3.04 ms, where a wave's adds in both passes took
+// 256 consecutive particles; they arrive nearly sorted and move a cell or so, so most
+// keys lie in a short stretch from the first one's, or in the same stretch a row
+// (`row` keys) or a plane (`plane`) before or after.  Those five are counted in LDS
+// (the count before is the rank within the block), each key then takes one atomic on
+// its histogram entry, whose return places the block's particles of that key.  The
+// other keys are added a wave at a time.  With the ranks known the scatter adds
+// nothing: at 128^3 with 64 particles a cell (1.4e8) flag and scatter take 0.94 + 3.04 ms,
+// where one stretch of 1024 keys took 1.17 + 3.04, and a wave's adds in both passes
 // 1.09 + 4.02; the step's push, 1.14 ms as a pass of its own, costs them 0.1.
-// PER: four particles a thread, or one where that leaves CUs idle: a sort of 6.6e4 particles
-// 37 and 34 us, of 1.0e6 49 both ways, of 1.7e7 355 and 390.
+// The stretch: 512 / 640 / 768 / 1024 keys take 0.92 / 0.94 / 0.96 / 1.08 ms there (more
+// to clear, fewer blocks to a CU), 207 / 175 / 162 / 126 us with two particles a cell, whose
+// 1024 spread over as many keys (one stretch of 1024: 185).
+// PER: four particles a thread, or one where that leaves CUs idle (with one stretch, a
+// sort of 6.6e4 particles 37 and 34 us, of 1.0e6 49 both ways, of 1.7e7 355 and 390).
 constexpr int kFlagPer = 4;
-constexpr int kFlagWin = 1024;           // keys counted in LDS
+constexpr int kFlagWin = 640;            // keys of a stretch
 constexpr int kFlagBack = 128;           // of them below the first particle's
 struct KeyWindow {
-  int32_t cnt[kFlagWin];
+  int32_t cnt[5 * kFlagWin];
   int32_t first;
 };
 
-// Every thread of a block of 256 takes part; returns after a barrier.
+// Every thread of a block of 256 takes part, `row` and `plane` are the block's; returns after a barrier.
 template <int PER>
 __device__ __forceinline__ void count_keys(const int32_t (&k)[PER], int32_t (&r)[PER],
-                                           int32_t *__restrict__ hist, KeyWindow &w) {
-  for (int e = threadIdx.x; e < kFlagWin; e += 256) w.cnt[e] = 0;
+                                           int32_t *__restrict__ hist, KeyWindow &w, int32_t row,
+                                           int32_t plane) {
+  for (int e = threadIdx.x; e < 5 * kFlagWin; e += 256) w.cnt[e] = 0;
   const uint64_t kept = __ballot(k[0] >= 0);
   if (threadIdx.x < 64) {                // the first wave's first kept particle
     const int32_t kf = kept ? __builtin_amdgcn_readlane(k[0], (int)__builtin_ctzll(kept)) : 0;
-    if (threadIdx.x == 0) w.first = kf > kFlagBack ? kf - kFlagBack : 0;
+    if (threadIdx.x == 0) w.first = kf - kFlagBack;
   }
   __syncthreads();
   const int32_t k0 = w.first;
+  const int32_t on[5] = {0, row, -row, plane, -plane};
+  int at[PER];                           // the count's place: by the key alone; -1: elsewhere
 #pragma unroll
   for (int h = 0; h < PER; ++h) {
-    const bool near = k[h] >= k0 && k[h] - k0 < kFlagWin;
+    at[h] = -1;
+#pragma unroll
+    for (int m = 4; m >= 0; --m) {
+      const uint32_t d = (uint32_t)k[h] - (uint32_t)k0 - (uint32_t)on[m];
+      if (d < (uint32_t)kFlagWin) at[h] = m * kFlagWin + (int)d;
+    }
+    if (k[h] < 0) at[h] = -1;
     r[h] = -1;
-    if (near) r[h] = atomicAdd(&w.cnt[k[h] - k0], 1);
-    const int32_t far = wave_add1(hist, near ? -1 : k[h]);
-    if (!near) r[h] = far;
+    if (at[h] >= 0) r[h] = atomicAdd(&w.cnt[at[h]], 1);
+    const int32_t far = wave_add1(hist, at[h] >= 0 ? -1 : k[h]);
+    if (at[h] < 0) r[h] = far;
   }
   __syncthreads();
   // each counted key's place in the histogram, over its count
-  for (int e = threadIdx.x; e < kFlagWin; e += 256) {
-    const int32_t m = w.cnt[e];
-    if (m) w.cnt[e] = atomicAdd(&hist[k0 + e], m);
-  }
+#pragma unroll
+  for (int m = 0; m < 5; ++m)
+    for (int e = threadIdx.x; e < kFlagWin; e += 256) {
+      const int32_t c = w.cnt[m * kFlagWin + e];
+      if (c) w.cnt[m * kFlagWin + e] = atomicAdd(&hist[(uint32_t)k0 + (uint32_t)on[m] + e], c);
+    }
   __syncthreads();
 #pragma unroll
   for (int h = 0; h < PER; ++h)
-    if (k[h] >= k0 && k[h] - k0 < kFlagWin) r[h] += w.cnt[k[h] - k0];
+    if (at[h] >= 0) r[h] += w.cnt[at[h]];
   __syncthreads();
 }
 
