@@ -1661,35 +1661,37 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
         set_error("CalcEpotential: pass accounting out of step");
         return PICARD_ERR_STATE;
       }
-      batch = 64;
+      batch = batch < 32 ? 16 : 64;
     }
   };
   bool done = false, few = false;
   if (spec_eligible(c) && last > 64) {
-    // to a few iterates before the stop, then the sweeps with the stop test;
-    // a solve that passes one of the first two tests may have been taken past
-    // its stop and starts again with a wider margin
+    // to a few iterates before the stop, no iterate before passing the test, then
+    // the sweeps with it; a solve that passes one of its first two tests may have been taken past
+    // its stop by rounding and starts again with a wider margin
     const bool exact = !c->split && !c->order_free;
-    for (int margin = 4; !done && margin <= 1024; margin *= 16) {
+    for (int margin = 3; !done && margin <= 1024; margin *= 16) {
       PICARD_TRY(begin());
-      // the FP64 forms' first sweep reads the halo U came in with
+      // the FP64 forms' first sweep reads the halo U came in with, and so does the test of iterate 1
       const int64_t base = c->split ? 0 : 1;
       if (base) pass(1, 1, nullptr, nullptr, nullptr);
-      int64_t to = -1;
-      PICARD_TRY(spec_step(c, base ? c->jb[1] : c->U, base, margin, !exact, &to));
+      int64_t to = -1, ahead = 0;
+      PICARD_TRY(spec_step(c, base ? c->jb[1] : c->U, base ? c->U : nullptr, base, margin, !exact, &to,
+                           &ahead));
       if (to < 0) {
         if (c->split) return kNoSpecStep;
-        few = to == -1;
+        few = to == kSpecFewLeft;
         break;
       }
       const int T = jacobi_block_sweeps(g);
       if (exact) {                // the same iterates by sweeps that leave out the test
         const int64_t launches = (to - base) / T;
+        ahead += to - (base + T * launches);
         to = base + T * launches;
         PICARD_TRY(launch_jacobi_block(c, base, launches));
       }
-      PICARD_TRY(sweep(to + 1, to + 1, margin + (exact ? T : 0) + 4));
-      done = fin.result == last || fin.result > to + 2;
+      PICARD_TRY(sweep(to + 1, to + 1, ahead + 4));
+      done = to >= maxit || fin.result > to + 2;
     }
   }
   if (!done) {

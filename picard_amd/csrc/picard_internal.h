@@ -279,7 +279,9 @@ bool spec_eligible(const picard_ctx *c);
 int spec_create(picard_ctx *c);
 void spec_release(picard_ctx *c);
 // apply = false: only finds the iterate
-int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, bool apply, int64_t *to);
+constexpr int64_t kSpecFewLeft = -1, kSpecNoNorm = -2, kSpecNotClear = -3;
+int spec_step(picard_ctx *c, const double *u, const double *old, int64_t base, int margin, bool apply, int64_t *to,
+              int64_t *ahead);
 
 // ---- jacobi_block.hip ----
 int jacobi_block_sweeps(const GridDims &g);   // sweeps per launch

@@ -13,12 +13,19 @@
 //
 // The stop rule's residual takes the previous iterate's values across periodic
 // boundaries (CalcEpotential.f90:83-92), which makes it J0 r_{p-1}: one Jacobi
-// step of the plain residual with zeros beyond every boundary.  Its norm is
-// not a sum over eigenvectors, so the search finds the crossing of the plain
-// norm first, evaluates the rule's own norm there in space, and corrects by
-// the slope.
+// step of the plain residual with zeros beyond every boundary.  Without a periodic axis its norm is
+// the plain one's, which falls from iterate to iterate.  With one it is not a sum over eigenvectors,
+// and it may pass the threshold, rise again, and stay below while modes that never decay (the mean of
+// a box without an open axis, the checkerboard of even edges) hold the plain norm above.  So the
+// step goes no further than the iterates that provably do not pass:
+//     |J0 r_{p-1}|^2 >= f(p) - B(p),   f(p) = |r_p|^2,
+// B the part across the boundaries, 2 a (u_0 . v_n-1 + u_n-1 . v_0) of the first and last planes of
+// u = r_p and v = r_{p-1} for each periodic axis.  For the first iterates B is
+// formed as it stands; for the others every mode of a plane's sum enters with its modulus, which
+// falls with p, as f does, so that f(q) - B(p) > threshold^2 clears all iterates p to q.  Once the
+// slow modes are left that loses a few iterates at most (k_spec_clear).
 //
-// Cost: nine axis transforms of 2 n operations a cell, whatever the number of
+// Cost: six axis transforms of 2 n operations a cell, whatever the number of
 // sweeps (about 3 n^2 to 1e-6).  Measured, whole solve with its last sweeps
 // against sweeping: 16^3 0.19 ms (FP32 sweeps 7.3), 64^3 0.37 ms (FP64 sweeps 280),
 // 128^3 to 1e-10 0.74 ms (FP32 sweeps 620), 160^3 1.1 ms (FP32 sweeps 880).
@@ -33,17 +40,25 @@
 
 namespace picard {
 
-constexpr int kSpecCand = 8;        // stop candidates per pass over the spectrum
+constexpr int kSpecCand = 8;        // candidates per pass over the spectrum
 constexpr int kSpecPasses = 3;
+// iterates that are looked at for the rule's norm: the first kSpecFirst one by one, then kSpecLater
+// in growing and again falling distances up to the plain norm's crossing
+constexpr int kSpecFirst = 16;
+constexpr int kSpecLater = 40;
+constexpr int kSpecLook = kSpecFirst + kSpecLater;
+constexpr int kSpecEach = 4;        // of them in one block
 
 // Device state of one search.  `skip`: no step is taken (0: go on).
 struct SpecState {
   double q[kSpecCand];              // candidates, in sweeps after the base iterate
   double lo, hi, flo, fhi;          // bracket of the plain norm's crossing, and the norms^2 there
   double T, f0;                     // threshold^2, the base residual's norm^2
-  double q1, slope;                 // crossing, and d ln(norm^2) / d sweep there
+  double look[kSpecLater];          // the later iterates that are looked at, ascending
+  double end;                       // the last of them: the crossing, or the last that is tested
   double steps;                     // sweeps the step covers
   int64_t to;                       // iterate the step ends on
+  int64_t ahead;                    // sweeps from there to about the stop
   int32_t skip;
   uint32_t arrive;
 };
@@ -51,7 +66,7 @@ struct SpecState {
 namespace {
 
 constexpr int kT = 256;
-enum { kSpecGo = 0, kSpecFew = 1, kSpecBad = 2 };
+enum { kSpecGo = 0, kSpecFew = 1, kSpecBad = 2, kSpecUnclear = 3 };
 // fewer sweeps than this are not worth the step (about 30 launches)
 constexpr int kSpecFewest = 32;
 
@@ -89,7 +104,7 @@ __device__ __forceinline__ bool last_block(uint32_t *arrive) {
   __shared__ bool last;
   if (threadIdx.x == 0) {
     __threadfence();
-    last = atomicAdd(arrive, 1u) == gridDim.x - 1;
+    last = atomicAdd(arrive, 1u) == n_blocks() - 1;
   }
   __syncthreads();
   if (last) __threadfence();
@@ -97,19 +112,21 @@ __device__ __forceinline__ bool last_block(uint32_t *arrive) {
 }
 
 // r = b - A u of the base iterate with periodic images of u itself, into the
-// compact layout (padding zero), and its norm; the last block sets up the search.
+// compact layout (padding zero), and its norm; the last block sets up the search.  `old`: the iterate
+// before, whose halo the rule's residual of this one takes; its norm is looked at as well.
 __global__ void __launch_bounds__(kT) k_spec_residual(SpecGeo g, const double *__restrict__ u,
+                                                      const double *__restrict__ old,
                                                       const double *__restrict__ b,
                                                       double *__restrict__ out,
                                                       double *__restrict__ partials,
                                                       const JacobiState *js, SpecState *st,
                                                       int64_t base, double lnmax) {
   __shared__ double sh[kT / 64];
-  double acc = 0.0;
+  double acc = 0.0, acc_rule = 0.0;
   for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < g.len; t += (int64_t)gridDim.x * kT) {
     const uint32_t row = (uint32_t)(t / g.PX), x = (uint32_t)(t % g.PX);
     const uint32_t y = row % (uint32_t)g.ny, z = row / (uint32_t)g.ny;
-    double r = 0.0;
+    double r = 0.0, rule = 0.0;
     if ((int)x < g.nx) {
       const int64_t c = (x + 1) + g.X * (int64_t)(y + 1) + g.XY * (int64_t)(z + 1);
       const int64_t e = g.px && (int)x == g.nx - 1 ? c - (g.nx - 1) : c + 1;
@@ -121,14 +138,35 @@ __global__ void __launch_bounds__(kT) k_spec_residual(SpecGeo g, const double *_
       const double u2 = 2.0 * u[c];
       r = b[c] - ((u[e] + u[w] - u2) / g.dx2 + (u[n] + u[s] - u2) / g.dy2 +
                   (u[tp] + u[bt] - u2) / g.dz2);
+      rule = r;
+      if (old) {
+        const int64_t XY = g.XY;
+        if (e != c + 1) rule += (u[e] - old[c + 1]) / g.dx2;
+        if (w != c - 1) rule += (u[w] - old[c - 1]) / g.dx2;
+        if (n != c + g.X) rule += (u[n] - old[c + g.X]) / g.dy2;
+        if (s != c - g.X) rule += (u[s] - old[c - g.X]) / g.dy2;
+        if (tp != c + XY) rule += (u[tp] - old[c + XY]) / g.dz2;
+        if (bt != c - XY) rule += (u[bt] - old[c - XY]) / g.dz2;
+      }
     }
     out[t] = r;
     acc += r * r;
+    acc_rule += rule * rule;
   }
   const double s = block_sum(acc, sh);
   if (threadIdx.x == 0) partials[blockIdx.x] = s;
+  if (old) {
+    __syncthreads();
+    const double s_rule = block_sum(acc_rule, sh);
+    if (threadIdx.x == 0) partials[gridDim.x + blockIdx.x] = s_rule;
+  }
   if (!last_block(&st->arrive)) return;
   const double f0 = final_sum(partials, gridDim.x, sh);
+  double f0_rule = f0;
+  if (old) {
+    __syncthreads();
+    f0_rule = final_sum(partials + gridDim.x, gridDim.x, sh);
+  }
   if (threadIdx.x) return;
   st->arrive = 0;
   st->f0 = f0;
@@ -137,7 +175,7 @@ __global__ void __launch_bounds__(kT) k_spec_residual(SpecGeo g, const double *_
   st->to = -1;
   const double span = (double)(js->last - base);
   // an infinite or NaN residual is left to the sweeps, as is a solve that has stopped
-  st->skip = !(f0 < 1.0e300) || !(T < 1.0e300) ? kSpecBad : (js->slot[base & 1].done || f0 <= T ? kSpecFew : kSpecGo);
+  st->skip = !(f0 < 1.0e300) || !(T < 1.0e300) ? kSpecBad : (js->slot[base & 1].done || f0 <= T || !(f0_rule > 1.000001 * T) ? kSpecFew : kSpecGo);
   // no mode decays slower than the slowest one
   double hi = span;
   if (T > 0.0 && lnmax < 0.0) hi = fmin(span, ceil(log(T / f0) / (2.0 * lnmax)) + 1.0);
@@ -148,6 +186,21 @@ __global__ void __launch_bounds__(kT) k_spec_residual(SpecGeo g, const double *_
   for (int i = 0; i < kSpecCand; ++i) st->q[i] = fmax(1.0, floor(ldexp(hi, -i)));
 }
 
+// The iterate the step ends on: `margin` before the last that is known not to pass, or before the end
+// of the solve when that is the last one tested, by more than rounding moves the norm.
+__device__ __forceinline__ void spec_finish(const JacobiState *js, SpecState *st, int64_t base, int margin,
+                                            double clear, double above, double left) {
+  const bool all = clear >= (double)((int64_t)js->maxit - 1 - base) && above > 1.02 * st->T;
+  const int64_t to = (all ? js->last : base + (int64_t)clear) - margin;
+  if (to - base < kSpecFewest || to > 0x7fffff00) {
+    st->skip = st->end > 4.0 * kSpecFewest ? kSpecUnclear : kSpecFew;
+    return;
+  }
+  st->to = to;
+  st->ahead = margin + (int64_t)(all ? 0.0 : fmin(left, 1024.0));
+  st->steps = (double)(to - base);
+}
+
 // sum w lambda^(2 q) over the spectrum for the pass's candidates, descending
 // (pass 0: halvings of the bound) or ascending in q (later passes: a division
 // of the bracket); the last block narrows the bracket and, after the last pass,
@@ -155,7 +208,8 @@ __global__ void __launch_bounds__(kT) k_spec_residual(SpecGeo g, const double *_
 // exponentials (eight per mode that has not decayed away); on small grids the chain of the
 // block's and the last block's sums: the candidates' together, 28 -> 10 us at 16^3.
 __global__ void __launch_bounds__(kT) k_spec_search(SpecGeo g, const double *__restrict__ R,
-                                                    double *__restrict__ partials, SpecState *st,
+                                                    double *__restrict__ partials, const JacobiState *js,
+                                                    SpecState *st, int64_t base, int margin, int seams,
                                                     int pass) {
   __shared__ double sh[kT / 64][kSpecCand];
   __shared__ double tot[kSpecCand];
@@ -224,23 +278,204 @@ __global__ void __launch_bounds__(kT) k_spec_search(SpecGeo g, const double *__r
       st->q[i] = fmax(1.0, floor(lo + (hi - lo) * (double)(i + 1) / (double)(kSpecCand + 1)));
     return;
   }
-  double q1 = hi, slope = 0.0;
-  if (fhi >= 0.0 && hi > lo) {
+  // the crossing; nothing is tested past maxit
+  double end = hi;
+  if (fhi < 0.0) {
+    end = 1.0e300;
+  } else if (hi > lo) {
     const double a = log(flo), c = log(fmax(fhi, 1.0e-300));
-    slope = (c - a) / (hi - lo);
-    if (st->T > 0.0 && slope < 0.0) q1 = fmin(hi, fmax(lo, lo + (log(st->T) - a) / slope));
+    if (st->T > 0.0 && c < a) end = fmin(hi, fmax(lo, lo + (log(st->T) - a) * (hi - lo) / (c - a)));
   }
-  st->q1 = fmax(1.0, ceil(q1));
-  st->slope = slope;
+  end = fmax(0.0, fmin(ceil(end), (double)((int64_t)js->maxit - 1 - base)));
+  st->end = end;
+  if (end < (double)kSpecFewest) {
+    st->skip = kSpecFew;
+    return;
+  }
+  // 20 in a geometric progression to half way, 12 evenly on, 8 closing in on the end
+  const double half = fmax((double)kSpecFirst, 0.5 * end), step = (end - half) / 13.0;
+  const double ratio = exp(log(half / kSpecFirst) / 20.0);
+  double q = kSpecFirst, near = step;
+  for (int i = 0; i < kSpecLater; ++i) {
+    if (i >= 32) q = i == kSpecLater - 1 ? end : end - (near *= 0.5);
+    st->look[i] = fmin(end, floor(q));
+    q = i < 19 ? q * ratio : half + step * (double)(i - 19);
+  }
+  // without a periodic axis the plain norm is the rule's
+  if (!seams) spec_finish(js, st, base, margin, end <= lo ? end : end - 1.0, end <= lo ? flo : 0.0, 0.0);
 }
 
-// The spectrum of r_{q1-1} (what = 0) or of the step's change of U, -af times
-// the sum of its sweeps' residuals (what = 1).
-__global__ void __launch_bounds__(kT) k_spec_scale(SpecGeo g, const double *__restrict__ R,
-                                                   double *__restrict__ out, const SpecState *st,
-                                                   int what) {
+// Sum of w_i over the block for N values a thread, in thread 0 .. N - 1 of the block.
+template <int N>
+__device__ __forceinline__ double sum_each(double (&v)[N], double (*sh)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    for (int off = 32; off > 0; off >>= 1) v[i] += __shfl_down(v[i], off, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][i] = v[i];
+  }
+  __syncthreads();
+  double s = 0.0;
+  if (threadIdx.x < N)
+    for (int w = 0; w < kT / 64; ++w) s += sh[w][threadIdx.x];
+  __syncthreads();
+  return s;
+}
+
+// The periodic axes of a box: cells, stride of the axis and of the columns across it in the
+// spectrum, the columns' counts, weight, and the basis.
+struct SpecSeam {
+  int n, ca, cb;
+  int64_t s, sa, sb;
+  int axis, ax_a, ax_b;
+  double a;
+  const double *Q;
+};
+struct SpecSeams {
+  int count;
+  SpecSeam s[3];
+};
+
+// How far no iterate passes the rule (see above).  blockIdx.y: four iterates, the first ones'
+// boundary part signed, the later ones' of moduli; blockIdx.z: a periodic axis, a thread taking columns
+// of modes along it.  The plain norms come with the first axis.  A mode that has decayed by e^60 is left
+// out, in f to the safe side, in B by less than 1e-24 of the base norm, which the test adds.
+// The last block sums and decides.  Bound: the exponentials of every mode and iterate, 260 us at 160^3 with
+// two periodic axes (393 with the logarithm of the decayed modes too); on small grids the
+// chain of one column and the decision, 18 us at 16^3 (eight iterates a block and the decision in one
+// thread: 39).
+__global__ void __launch_bounds__(kT) k_spec_clear(SpecGeo g, SpecSeams ss, const double *__restrict__ R,
+                                                   double *__restrict__ partials, const JacobiState *js,
+                                                   SpecState *st, int64_t base, int margin) {
+  constexpr int N = kSpecEach;
+  __shared__ double sh[kT / 64][2 * N];
+  __shared__ double sums[kSpecLook][4];              // f, then an axis each
   if (st->skip) return;
-  const double q = what ? st->steps : st->q1 - 1.0;
+  const SpecSeam m = ss.s[blockIdx.z];
+  const int first = (int)blockIdx.y * N;             // the block's iterates
+  const int nx[3] = {g.nx, g.ny, g.nz};
+  double q[N], acc[2 * N];                           // f, then B
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int j = first + i - kSpecFirst;
+    q[i] = j >= 0 ? st->look[j] - 1.0 : 0.0;
+    acc[i] = acc[N + i] = 0.0;
+  }
+  const double *es = g.eig[m.axis], *ea = g.eig[m.ax_a], *eb = g.eig[m.ax_b];
+  const int np = spec_cols(m.n);
+  const int64_t columns = (int64_t)m.ca * m.cb;
+  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < columns; t += (int64_t)gridDim.x * kT) {
+    const int ia = (int)(t % m.ca), ib = (int)(t / m.ca);
+    const double *r = R + ia * m.sa + ib * m.sb;
+    const double sab = ea[ia] + eb[ib], cab = ea[nx[m.ax_a] + ia] + eb[nx[m.ax_b] + ib];
+    if (first < kSpecFirst) {
+      // the two planes' sums of iterates first .. first + N, the rule's being one later
+      double v0[N + 1], vn[N + 1];
+#pragma unroll
+      for (int i = 0; i <= N; ++i) v0[i] = vn[i] = 0.0;
+      double next = r[0];
+      for (int k = 0; k < m.n; ++k) {
+        const double lam = 1.0 - (sab + es[k]);
+        double w = next;
+        if (k + 1 < m.n) next = r[(k + 1) * m.s];
+        for (int i = 0; i < first; ++i) w *= lam;
+        const double Q0 = m.Q[k], Qn = m.Q[(int64_t)(m.n - 1) * np + k];
+#pragma unroll
+        for (int i = 0; i <= N; ++i) {
+          v0[i] += Q0 * w;
+          vn[i] += Qn * w;
+          if (i) acc[i - 1] += w * w;
+          w *= lam;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        acc[N + i] += 2.0 * m.a * (v0[i + 1] * vn[i] + vn[i + 1] * v0[i]);
+    } else {
+      double S[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) S[i] = 0.0;
+      // a cosine and its sine (the same eigenvalue) together: their largest value on any plane
+      double r0 = r[0], r1 = 0.0;
+      for (int k = 0; k < m.n;) {
+        const bool pair = k > 0 && k + 1 < m.n;
+        const double p2 = r0 * r0 + r1 * r1;
+        const int up = k + (pair ? 2 : 1);
+        if (up < m.n) r0 = r[up * m.s];
+        r1 = up + 1 < m.n ? r[(up + 1) * m.s] : 0.0;
+        const double s = sab + es[k], c = cab + es[m.n + k];
+        k = up;
+        if (q[0] * fmin(s, c) > 60.0) continue;      // ln(1 - x) <= -x, at every iterate of the block
+        bool neg;
+        const double ln = spec_ln(s, c, &neg), lam = fabs(1.0 - s);
+        const double amp = sqrt(p2 * (pair ? 2.0 : 1.0) / (double)m.n);
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          if (q[i] * ln < -60.0) continue;
+          const double e = exp(q[i] * ln);
+          S[i] += amp * e;
+          acc[i] += p2 * ((e * lam) * (e * lam));
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) acc[N + i] += 4.0 * m.a * S[i] * S[i];
+    }
+  }
+  const double s = sum_each<2 * N>(acc, sh);
+  // entry: iterate, then f or the axis; the blocks of a group side by side
+  const unsigned nb = gridDim.x;
+  if (threadIdx.x < 2 * N) {
+    const int i = first + (int)(threadIdx.x % N);
+    const bool plain = threadIdx.x < N;
+    if (!plain || blockIdx.z == 0)
+      partials[((int64_t)i * 4 + (plain ? 0 : 1 + blockIdx.z)) * nb + blockIdx.x] = s;
+  }
+  __syncthreads();                       // before the fence of thread 0
+  if (!last_block(&st->arrive)) return;
+  static_assert(kSpecLook * 4 <= kT && kSpecLook < 64 && kSpecFirst % kSpecEach == 0, "one thread a sum, one lane an iterate");
+  if ((int)threadIdx.x < kSpecLook * 4) {
+    const int i = (int)threadIdx.x >> 2, w = (int)threadIdx.x & 3;
+    double v = 0.0;
+    if (w <= ss.count)
+      for (unsigned b = 0; b < nb; ++b) v += partials[((int64_t)i * 4 + w) * nb + b];
+    sums[i][w] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  // a lane an iterate: is it, or the stretch up to it from the one before, clear?
+  const int l = (int)threadIdx.x;
+  const double T = st->T + 1.0e-24 * st->f0;
+  const int from = l <= kSpecFirst ? l : l - 1;      // whose B
+  const bool ok = l < kSpecLook && (l == kSpecFirst ||
+                                    sums[l][0] - (sums[from][1] + sums[from][2] + sums[from][3]) > T);
+  const int cleared = (int)__builtin_ctzll(~__ballot(ok));     // lane 63 is none
+  if (l) return;
+  st->arrive = 0;
+  double clear = (double)cleared, f = 0.0, B = 0.0, left = 0.0;
+  if (cleared > kSpecFirst) {
+    const double *v = sums[cleared - 1];
+    f = v[0];
+    B = v[1] + v[2] + v[3];
+    const double at = st->look[cleared - 1 - kSpecFirst];
+    clear = at;
+    // ln f is convex: the chord from the nearest one before, continued, lies below it
+    int was = cleared - 2 - kSpecFirst;
+    while (was >= 0 && st->look[was] >= at) --was;
+    const double slope =
+        was >= 0 ? log(f / sums[kSpecFirst + was][0]) / (at - st->look[was]) : 0.0;
+    if (slope < 0.0 && clear < st->end) {
+      if (f - B > T) clear = fmin(st->end, clear + floor(log((T + B) / f) / slope));
+      // the boundary part is about 0.92 of B where one mode is left
+      left = fmax(0.0, at + ceil(log((T + 0.92 * B) / f) / slope) - clear);
+    }
+  }
+  spec_finish(js, st, base, margin, clear, f - B, left);
+}
+
+// The spectrum of the step's change of U, -af times the sum of its sweeps' residuals.
+__global__ void __launch_bounds__(kT) k_spec_scale(SpecGeo g, const double *__restrict__ R,
+                                                   double *__restrict__ out, const SpecState *st) {
+  if (st->skip) return;
+  const double q = st->steps;
   const bool odd = fmod(q, 2.0) != 0.0;
   for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < g.len; t += (int64_t)gridDim.x * kT) {
     const uint32_t row = (uint32_t)(t / g.PX), x = (uint32_t)(t % g.PX);
@@ -252,60 +487,12 @@ __global__ void __launch_bounds__(kT) k_spec_scale(SpecGeo g, const double *__re
       bool neg;
       const double ln = spec_ln(s, c, &neg);
       const double sg = neg && odd ? -1.0 : 1.0;
-      if (what == 0) {
-        v = q > 0.0 ? sg * exp(q * ln) : 1.0;
-      } else {
-        // (1 - lambda^q) / (1 - lambda)
-        v = s == 0.0 ? q : (neg ? 1.0 - sg * exp(q * ln) : -expm1(q * ln)) / s;
-        v = -g.af * v;
-      }
-      v = v * R[t];
+      // (1 - lambda^q) / (1 - lambda)
+      v = s == 0.0 ? q : (neg ? 1.0 - sg * exp(q * ln) : -expm1(q * ln)) / s;
+      v = -g.af * v * R[t];
     }
     out[t] = v;
   }
-}
-
-// Norm of J0 w (w = r_{q1-1}, zeros beyond every boundary): the stop rule's
-// residual of iterate base + q1.  The last block moves the crossing by the
-// slope and fixes the iterate the step ends on, `margin` before it.
-__global__ void __launch_bounds__(kT) k_spec_rule(SpecGeo g, const double *__restrict__ w,
-                                                  double *__restrict__ partials,
-                                                  const JacobiState *js, SpecState *st, int64_t base,
-                                                  int margin) {
-  __shared__ double sh[kT / 64];
-  if (st->skip) return;
-  double acc = 0.0;
-  const int64_t P = (int64_t)g.PX * g.ny;
-  for (int64_t t = (int64_t)blockIdx.x * kT + threadIdx.x; t < g.len; t += (int64_t)gridDim.x * kT) {
-    const uint32_t row = (uint32_t)(t / g.PX), x = (uint32_t)(t % g.PX);
-    if ((int)x >= g.nx) continue;
-    const uint32_t y = row % (uint32_t)g.ny, z = row / (uint32_t)g.ny;
-    const double e = (int)x + 1 < g.nx ? w[t + 1] : 0.0, ww = x > 0 ? w[t - 1] : 0.0;
-    const double n = (int)y + 1 < g.ny ? w[t + g.PX] : 0.0, s = y > 0 ? w[t - g.PX] : 0.0;
-    const double tp = (int)z + 1 < g.nz ? w[t + P] : 0.0, bt = z > 0 ? w[t - P] : 0.0;
-    const double r = g.ax * (e + ww) + g.ay * (n + s) + g.az * (tp + bt);
-    acc += r * r;
-  }
-  const double s = block_sum(acc, sh);
-  if (threadIdx.x == 0) partials[blockIdx.x] = s;
-  if (!last_block(&st->arrive)) return;
-  const double F = final_sum(partials, gridDim.x, sh);
-  if (threadIdx.x) return;
-  st->arrive = 0;
-  const int64_t last = js->last;
-  double q = st->q1;
-  if (st->fhi < 0.0) q = (double)(last - base);                  // not reached within the cap
-  else if (st->T > 0.0 && F > 0.0 && st->slope < 0.0) q = q + (log(st->T) - log(F)) / st->slope;
-  if (!(q < (double)(last - base))) q = (double)(last - base);
-  int64_t stop = base + (int64_t)ceil(q);
-  if (stop + 1 > (int64_t)js->maxit + 2) stop = last;            // the rule is not applied past maxit
-  const int64_t to = stop - margin;
-  if (to - base < kSpecFewest || to > 0x7fffff00) {
-    st->skip = kSpecFew;
-    return;
-  }
-  st->to = to;
-  st->steps = (double)(to - base);
 }
 
 // U_to = U_base + its change on interior nodes, into the sweeps' buffer of iterate `to`.
@@ -431,11 +618,13 @@ int spec_create(picard_ctx *c) {
   return PICARD_OK;
 }
 
-// From iterate `base` (in `u`, guard layout) to an iterate at least `margin`
-// before the one the stop rule will pick, left in the sweeps' buffers jb; *to is
-// that iterate, -1 if too few sweeps are left for a step, or -2 if the
-// residual has no finite norm.
-int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, bool apply, int64_t *to) {
+// From iterate `base` (in `u`, guard layout; `old`: the one before, if there is one) to an iterate at
+// least `margin` before the one the stop rule will pick, left in the sweeps' buffers jb.  *to: that
+// iterate, *ahead: sweeps to about the stop; or, with nothing done, kSpecFewLeft: too few sweeps are
+// left for a step, kSpecNoNorm: the residual has no finite norm, kSpecNotClear: early iterates may
+// pass the rule (few cells between periodic boundaries).
+int spec_step(picard_ctx *c, const double *u, const double *old, int64_t base, int margin, bool apply, int64_t *to,
+              int64_t *ahead) {
   const GridDims &g = c->gd;
   hipStream_t s = c->stream;
   SpecGeo sg;
@@ -481,18 +670,33 @@ int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, bool app
   if (nb > cap) nb = cap;
   const unsigned B = (unsigned)(nb < 1 ? 1 : nb);
   double *part = c->s.partials;
-  k_spec_residual<<<B, kT, 0, s>>>(sg, u, c->b, B0, part, c->js, st, base, c->spec_lnmax);
+  k_spec_residual<<<B, kT, 0, s>>>(sg, u, old, c->b, B0, part, c->js, st, base, c->spec_lnmax);
   axis(0, c->spec_fwd, B0, B1);
   axis(1, c->spec_fwd, B1, B2);
   axis(2, c->spec_fwd, B2, B0);
-  for (int p = 0; p < kSpecPasses; ++p) k_spec_search<<<B, kT, 0, s>>>(sg, B0, part, st, p);
-  k_spec_scale<<<B, kT, 0, s>>>(sg, B0, B1, st, 0);
-  axis(0, c->spec_inv, B1, B2);
-  axis(1, c->spec_inv, B2, B1);
-  axis(2, c->spec_inv, B1, B2);
-  k_spec_rule<<<B, kT, 0, s>>>(sg, B2, part, c->js, st, base, margin);
+  SpecSeams ss;
+  ss.count = 0;
+  const int n[3] = {g.nx, g.ny, g.nz};
+  const int64_t stride[3] = {1, sg.PX, P};
+  const double weight[3] = {sg.ax, sg.ay, sg.az};
+  int64_t columns = 0;
+  for (int d = 0; d < 3; ++d) {
+    if (g.flow[d]) continue;
+    const int a = d == 0 ? 1 : 0, b = d == 2 ? 1 : 2;
+    ss.s[ss.count++] = SpecSeam{n[d], n[a], n[b], stride[d], stride[a], stride[b], d, a, b, weight[d],
+                                c->spec_fwd[d]};
+    columns = std::max(columns, (int64_t)n[a] * n[b]);
+  }
+  for (int p = 0; p < kSpecPasses; ++p)
+    k_spec_search<<<B, kT, 0, s>>>(sg, B0, part, c->js, st, base, margin, ss.count, p);
+  if (ss.count) {
+    const int64_t room = 4 * c->s.partials_len / (4 * kSpecLook);
+    const int64_t nb = std::max<int64_t>(1, std::min((columns + kT - 1) / kT, room));
+    k_spec_clear<<<dim3((unsigned)nb, kSpecLook / kSpecEach, ss.count), kT, 0, s>>>(
+        sg, ss, B0, part, c->js, st, base, margin);
+  }
   if (apply) {
-    k_spec_scale<<<B, kT, 0, s>>>(sg, B0, B1, st, 1);
+    k_spec_scale<<<B, kT, 0, s>>>(sg, B0, B1, st);
     axis(0, c->spec_inv, B1, B2);
     axis(1, c->spec_inv, B2, B1);
     axis(2, c->spec_inv, B1, B2);
@@ -502,7 +706,9 @@ int spec_step(picard_ctx *c, const double *u, int64_t base, int margin, bool app
   PICARD_HIP(hipMemcpyAsync(c->spec_host, st, sizeof(SpecState), hipMemcpyDeviceToHost, s));
   PICARD_HIP(hipStreamSynchronize(s));
   const SpecState *h = c->spec_host;
-  *to = h->skip == kSpecBad ? -2 : (h->skip ? -1 : h->to);
+  *to = h->skip ? (h->skip == kSpecBad ? kSpecNoNorm : (h->skip == kSpecUnclear ? kSpecNotClear : kSpecFewLeft))
+                : h->to;
+  *ahead = h->skip ? 0 : h->ahead;
   return PICARD_OK;
 }
 
