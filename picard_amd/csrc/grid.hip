@@ -1241,11 +1241,12 @@ constexpr double kFix48Inv = 1.0 / 281474976710656.0;
 // its reads then lie four apart).
 constexpr int kFixSeg = 256;
 
-// (unsigned long long)llrint(F 2^48), 0 <= F <= 1 (NaN: 0): the sum with 2^52 rounds to
-// whole units, which are its low mantissa bits
+// (unsigned long long)llrint(F 2^48), NaN: 0.  -4 < F < 8: a particle up to a cell below the first
+// node has a remainder below zero (cic.h).  The sum with 3 2^51 rounds to whole units, which
+// are its low mantissa bits.
 __device__ __forceinline__ unsigned long long fix48(double F) {
-  const double v = fmin(fmax(F * kFix48, 0.0), 2.0 * kFix48) + 4503599627370496.0;
-  return (unsigned long long)__double_as_longlong(v) - 0x4330000000000000ull;
+  const double v = (F == F ? fmin(F * kFix48, 2251799813685247.0) : 0.0) + 6755399441055744.0;
+  return (unsigned long long)__double_as_longlong(v) - 0x4338000000000000ull;
 }
 
 __global__ void __launch_bounds__(kT) k_dep_fix64(ParticlesF64 p, GridDims g, int64_t nb,
