@@ -1295,6 +1295,28 @@ __global__ void __launch_bounds__(kT) k_dep_fix64(ParticlesF64 p, GridDims g, in
   }
 }
 
+// The same sums with one atomic in memory per corner and particle, for few particles.
+__global__ void __launch_bounds__(kT) k_dep_fix64_each(ParticlesF64 p, int64_t n, GridDims g,
+                                                       unsigned long long *__restrict__ Nfix,
+                                                       int32_t *__restrict__ errors) {
+  const int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x;
+  if (q >= n) return;
+  const CicLoc L = cic_locate(g, p.r[0][q], p.r[1][q], p.r[2][q]);
+  const int s0 = p.sp[q] - 1;
+  if (!cic_in_bounds(g, L) || s0 < 0 || s0 >= g.S) {
+    atomicAdd(errors, 1);
+    return;
+  }
+  const int64_t node = node_index(g, L.idx[0], L.idx[1], L.idx[2]);
+  const int64_t X = g.X, XY = (int64_t)g.X * g.Y;
+#pragma unroll
+  for (int o = 0; o < 8; ++o) {
+    const int64_t to = node + (o & 1) + X * ((o >> 1) & 1) + XY * (o >> 2);
+    atomicAdd(&Nfix[to * g.S + s0],
+              fix48(dep_weight(g, o & 1, o & 2, o & 4, L.rest[0], L.rest[1], L.rest[2])));
+  }
+}
+
 // Integer guard folds of the fixed-point sums, then N = W 2^-48 n2p and
 // C = sum_s N charge (ParticlesGridify.f90:129-293).
 __global__ void __launch_bounds__(kT) k_fold_fix64(GridDims g,
@@ -1325,9 +1347,14 @@ __global__ void __launch_bounds__(kT) k_fold_fix64(GridDims g,
   C[node] = cacc;
 }
 
-__global__ void k_zero_u64(unsigned long long *p, int64_t n) {
-  const int64_t q = (int64_t)blockIdx.x * kT + threadIdx.x;
-  if (q < n) p[q] = 0ull;
+// The deposits' counts, sums and errors cleared together: a launch of its own each, the two memsets and
+// the sums were 7 us of a small deposit.
+__global__ void __launch_bounds__(kT) k_dep_clear(int32_t *hist, int64_t nhist, unsigned long long *sums,
+                                                  int64_t nsums, int32_t *errors) {
+  const int64_t t0 = (int64_t)blockIdx.x * kT + threadIdx.x, step = (int64_t)gridDim.x * kT;
+  if (t0 == 0) *errors = 0;
+  for (int64_t t = t0; t < nhist; t += step) hist[t] = 0;
+  for (int64_t t = t0; t < nsums; t += step) sums[t] = 0;
 }
 
 __global__ void k_kstamp_reset(unsigned long long *ks, int n) {
@@ -1370,13 +1397,21 @@ int kstamp_collect(picard_ctx *c, int n) {
 
 // ---------------------------------------------------------------------------
 
-// Particles by (species, lower node): c->s.hist the buckets' starts, c->s.perm the
+// Clears the buckets' counts (if asked to), `nsums` fixed-point sums and the count of particles
+// outside the grid.
+static int clear_deposit(picard_ctx *c, bool counts, int64_t nsums) {
+  const int64_t nh = counts ? (int64_t)c->gd.S * c->K + 1 : 0;
+  const int nb = std::min(grid_blocks(std::max<int64_t>(std::max(nh, nsums), 1), kT), 8192);
+  k_dep_clear<<<nb, kT, 0, c->stream>>>(c->s.hist, nh, c->Nfix, nsums, c->s.counters);
+  PICARD_HIP(hipGetLastError());
+  return PICARD_OK;
+}
+
+// Particles by (species, lower node), from cleared counts: c->s.hist the buckets' starts, c->s.perm the
 // particles, those outside the grid counted.
 static int bucket_particles(picard_ctx *c) {
   const GridDims &g = c->gd;
   const int64_t n = c->n, nb = (int64_t)g.S * c->K;
-  PICARD_HIP(hipMemsetAsync(c->s.hist, 0, sizeof(int32_t) * (nb + 1), c->stream));
-  PICARD_HIP(hipMemsetAsync(c->s.counters, 0, sizeof(int32_t), c->stream));
   if (n > 0)
     k_dep_key<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, n, g, c->s.key, c->s.scan, c->s.hist,
                                                         c->s.counters);
@@ -1389,14 +1424,29 @@ static int bucket_particles(picard_ctx *c) {
   return PICARD_OK;
 }
 
+// Few particles, or few for the grid: one atomic per corner and particle, two launches, instead
+// of bucketing, seven, whose scan runs over all buckets.  The line where the two take the
+// same time with evenly spread particles, and below it where many meet on a node:
+// 8^3 2.2e4 (51 us), 12^3 6.0e4 (62), 24^3 1.0e5 (63), 48^3 1.4e5 (77), 72^3 3.0e5 (135), 96^3 5.9e5 (235),
+// 160^3 1.8e6 (700).  3e3 particles take 28 to 77 us where bucketed they take 35 to 141;
+// with particles in the grid's order the direct form is good for some 1.3 times more.
+static bool deposit_direct(const picard_ctx *c) {
+  const int64_t buckets = (int64_t)c->gd.S * c->K;
+  return c->n < 14 * buckets && c->n < 75000 + buckets / 4;
+}
+
 static int launch_gridify_fixed(picard_ctx *c) {
   const GridDims &g = c->gd;
   const int64_t n = c->n;
-  PICARD_TRY(bucket_particles(c));
-  k_zero_u64<<<grid_blocks((int64_t)g.S * g.G, kT), kT, 0, c->stream>>>(c->Nfix, (int64_t)g.S * g.G);
-  if (n > 0)
+  const bool direct = deposit_direct(c);
+  PICARD_TRY(clear_deposit(c, !direct, (int64_t)g.S * g.G));
+  if (!direct) {
+    PICARD_TRY(bucket_particles(c));
     k_dep_fix64<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, g, (int64_t)g.S * c->K, c->s.hist,
                                                               c->s.perm, c->Nfix);
+  } else if (n > 0) {
+    k_dep_fix64_each<<<grid_blocks(n, kT), kT, 0, c->stream>>>(c->p, n, g, c->Nfix, c->s.counters);
+  }
   k_fold_fix64<<<grid_blocks(g.G, kT), kT, 0, c->stream>>>(g, c->Nfix, c->N, c->C, c->consts);
   PICARD_HIP(hipGetLastError());
   PICARD_HIP(hipMemcpyAsync(c->host_counters, c->s.counters, sizeof(int32_t),
@@ -1415,6 +1465,7 @@ int launch_gridify(picard_ctx *c, bool flux) {
   const GridDims &g = c->gd;
   const int64_t n = c->n;
   const int64_t nb = (int64_t)g.S * c->K;
+  PICARD_TRY(clear_deposit(c, true, 0));
   PICARD_TRY(bucket_particles(c));
   // the outflow's scratch, free here: the sorted indices and, over pairs of
   // its int32 arrays, the in-cell offsets
