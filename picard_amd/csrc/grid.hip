@@ -96,9 +96,10 @@ __global__ void __launch_bounds__(kT) k_dep_order(ParticlesF64 p, GridDims g, in
 }
 
 // One thread per (node, species): 8-way merge by descending particle index.
-// With the number fluxes of ParticlesGridifyAll (ParticlesGridifyAll.f90:126-212), F(s, c,
-// node) += F_k n2p(s) v_c, in the same order; Fraw is laid out (s fastest, then c,
+// FLUX also accumulates the number fluxes of ParticlesGridifyAll (ParticlesGridifyAll.f90:126-212),
+// F(s, c, node) += F_k n2p(s) v_c, in the same order; Fraw is laid out (s fastest, then c,
 // then node).
+template <bool FLUX>
 __global__ void __launch_bounds__(kT) k_dep_gather(ParticlesF64 p, GridDims g, const double *n2p,
                                                     const int32_t *__restrict__ off,
                                                     const int32_t *__restrict__ sorted,
@@ -153,16 +154,19 @@ __global__ void __launch_bounds__(kT) k_dep_gather(ParticlesF64 p, GridDims g, c
     const double fz = (best & 4) ? L.rest[2] : L.drest[2];
     const double F = fx * fy * fz / g.dV;
     acc = acc + F * w;
-    const double Fw = F * w;
-    fl[0] = fl[0] + Fw * p.r[3][bestp];
-    fl[1] = fl[1] + Fw * p.r[4][bestp];
-    fl[2] = fl[2] + Fw * p.r[5][bestp];
+    if (FLUX) {
+      const double Fw = F * w;
+      fl[0] = fl[0] + Fw * p.r[3][bestp];
+      fl[1] = fl[1] + Fw * p.r[4][bestp];
+      fl[2] = fl[2] + Fw * p.r[5][bestp];
+    }
   }
   Nraw[node * g.S + s0] = acc;
-  for (int c = 0; c < 3; ++c) Fraw[(node * 3 + c) * g.S + s0] = fl[c];
+  if (FLUX)
+    for (int c = 0; c < 3; ++c) Fraw[(node * 3 + c) * g.S + s0] = fl[c];
 }
 
-// Without the fluxes a block takes one species' nodes i0.. of one row (j, k).  Their
+// Without the fluxes, unless particles are few (deposit_sparse), a block takes one species' nodes i0.. of one row (j, k).  Their
 // cells are four rows' (j - 1 | j, k - 1 | k), each row one contiguous stretch of the
 // sorted particles.  The four buckets of one x are a column; node n takes columns n and
 // n + 1.  A particle's place among its column's is its place in its own bucket plus
@@ -1460,6 +1464,13 @@ static int launch_gridify_fixed(picard_ctx *c) {
   return PICARD_OK;
 }
 
+// Few particles for the grid: a thread per node merges its buckets (k_dep_gather) instead of a block per row
+// (k_dep_rows), which pays its barriers for every row, empty or not.  Whole deposits, us, of evenly spread
+// particles, gather / rows: 3e3 on 24^3 54 / 68, on 96^3 88 / 147, on 160^3 214 / 407; about
+// the line 2e4 on 24^3 69 / 68, 8e4 on 48^3 75 / 78, 5e5 on 96^3 226 / 252, 2e6 on 160^3 891 / 946; beyond
+// 2e5 on 48^3 108 / 89, 1e6 on 96^3 430 / 333, 4e6 on 160^3 1898 / 1350.
+static bool deposit_sparse(const picard_ctx *c) { return 3 * c->n < (int64_t)c->gd.S * c->gd.G; }
+
 int launch_gridify(picard_ctx *c, bool flux) {
   if (!flux && c->order_free) return launch_gridify_fixed(c);
   const GridDims &g = c->gd;
@@ -1472,8 +1483,9 @@ int launch_gridify(picard_ctx *c, bool flux) {
   int32_t *sorted = c->s.flags;
   double *rest[3];
   for (int d = 0; d < 3; ++d) rest[d] = reinterpret_cast<double *>(c->s.work[2 * d]);
+  const bool rows = !flux && !deposit_sparse(c);
   if (n > 0) {
-    if (flux)
+    if (!rows)
       k_dep_order<false><<<grid_blocks(n, kT), kT, 0, c->stream>>>(
           c->p, g, nb, c->s.key, c->s.hist, c->s.perm, sorted, nullptr, nullptr, nullptr);
     else
@@ -1483,10 +1495,13 @@ int launch_gridify(picard_ctx *c, bool flux) {
   }
   if (flux) {
     PICARD_TRY(ensure_flux(c));
-    k_dep_gather<<<grid_blocks(g.G * g.S, kT), kT, 0, c->stream>>>(
+    k_dep_gather<true><<<grid_blocks(g.G * g.S, kT), kT, 0, c->stream>>>(
         c->p, g, c->consts, c->s.hist, sorted, c->Nraw, c->Fraw);
     PICARD_HIP(hipGetLastError());
     k_fold_flux<<<grid_blocks(g.G, kT), kT, 0, c->stream>>>(g, c->Fraw, c->F);
+  } else if (!rows) {
+    k_dep_gather<false><<<grid_blocks(g.G * g.S, kT), kT, 0, c->stream>>>(
+        c->p, g, c->consts, c->s.hist, sorted, c->Nraw, nullptr);
   } else {
     const int nseg = (g.X + kRowSeg - 1) / kRowSeg, seg = (g.X + nseg - 1) / nseg;
     const int64_t blocks = (int64_t)nseg * g.Y * g.Z * g.S;
