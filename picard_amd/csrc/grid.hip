@@ -775,28 +775,35 @@ struct JacobiCoef {
 // threshold and the first stop test.  Two launches in place of the norm's, the state's
 // upload and three copies, 20 us of a 16^3 step's 570; with the block that ends the sum in the
 // first launch every block's fence wrote its XCD's L2 back, 0.48 -> 0.04 ms at 160^3.
+// `images`: the copies' periodic guards are the interior's images, whatever U's are.
 template <bool COPY>
 __global__ void __launch_bounds__(kT) k_jacobi_begin(GridDims g, const double *__restrict__ C,
                                                       const double *__restrict__ U,
                                                       double *__restrict__ u0, double *__restrict__ u1,
                                                       double *__restrict__ u2,
                                                       double *__restrict__ b, double binv,
-                                                      double *__restrict__ partials) {
+                                                      double *__restrict__ partials, int images) {
   __shared__ double sh[kT / 64];
   double v2 = 0.0;
   for (int64_t node = (int64_t)blockIdx.x * kT + threadIdx.x; node < g.G;
        node += (int64_t)gridDim.x * kT) {
     const double bv = -C[node] * binv;               // CalcEpotential.f90:50
     b[node] = bv;
+    const uint32_t row = (uint32_t)node / (uint32_t)g.X;       // fewer than 2^32 nodes fit the memory
+    const int i = (int)((uint32_t)node - row * (uint32_t)g.X) + 1;
+    const int k = (int)(row / (uint32_t)g.Y) + 1, j = (int)(row % (uint32_t)g.Y) + 1;
     if (COPY) {
-      const double u = U[node];
+      int64_t from = node;
+      if (images) {
+        if (!g.flow[0] && (i == 1 || i == g.X)) from += i == 1 ? g.nx : -g.nx;
+        if (!g.flow[1] && (j == 1 || j == g.Y)) from += (int64_t)(j == 1 ? g.ny : -g.ny) * g.X;
+        if (!g.flow[2] && (k == 1 || k == g.Z)) from += (int64_t)(k == 1 ? g.nz : -g.nz) * g.X * g.Y;
+      }
+      const double u = U[from];
       u0[node] = u;
       u1[node] = u;
       u2[node] = u;
     }
-    const uint32_t row = (uint32_t)node / (uint32_t)g.X;       // fewer than 2^32 nodes fit the memory
-    const int i = (int)((uint32_t)node - row * (uint32_t)g.X) + 1;
-    const int k = (int)(row / (uint32_t)g.Y) + 1, j = (int)(row % (uint32_t)g.Y) + 1;
     if (i >= 2 && i <= g.nx + 1 && j >= 2 && j <= g.ny + 1 && k >= 2 && k <= g.nz + 1)
       v2 += bv * bv;
   }
@@ -1585,13 +1592,14 @@ int launch_bc_potentials(picard_ctx *c) {
 }
 
 // b = -C/(dV eps0), its interior norm, the threshold and the stop test of
-// loop iteration ss = 1 (CalcEpotential.f90:50-62); `copy`: jb = U.
+// loop iteration ss = 1 (CalcEpotential.f90:50-62); `copy`: jb = U (split form: with fresh images).
 int launch_begin(picard_ctx *c, const JacobiState &init, double maxerr, bool copy) {
   const GridDims &g = c->gd;
   const double binv = 1.0 / (g.dV * 8.854187817e-12);
   const int nb = std::min(grid_blocks(g.G, kT), 2048);
   auto *kf = copy ? k_jacobi_begin<true> : k_jacobi_begin<false>;
-  kf<<<nb, kT, 0, c->stream>>>(g, c->C, c->U, c->jb[0], c->jb[1], c->jb[2], c->b, binv, c->s.partials);
+  kf<<<nb, kT, 0, c->stream>>>(g, c->C, c->U, c->jb[0], c->jb[1], c->jb[2], c->b, binv, c->s.partials,
+                               c->split);
   k_jacobi_state<<<1, kT, 0, c->stream>>>(c->s.partials, nb, c->js, init, maxerr);
   PICARD_HIP(hipGetLastError());
   return PICARD_OK;
@@ -1684,8 +1692,9 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
                             (int32_t)first, ks);
   };
   StopSlot fin{};
-  // passes p, p + 1, ... to the end of the solve, the first of the sweeps being `first`
-  auto sweep = [&](int64_t p, int64_t first, int64_t batch) -> int {
+  // passes p, p + 1, ... to the end of the solve, the first of the sweeps being `first`, or until `most`
+  // are done
+  auto sweep = [&](int64_t p, int64_t first, int64_t batch, int64_t most) -> int {
     for (;;) {
       const int64_t todo = (last + 1 - (p - 1)) < batch ? (last + 1 - (p - 1)) : batch;
       // timing: one pass in kTimeEvery, with dispatch-packet events around it
@@ -1723,7 +1732,7 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
         PICARD_TRY(kstamp_collect(c, (int)timed));
       }
       fin = c->js_host->slot[(p - 1) & 1];
-      if (fin.done) return PICARD_OK;
+      if (fin.done || p > most) return PICARD_OK;
       if (p > last + 1) {
         set_error("CalcEpotential: pass accounting out of step");
         return PICARD_ERR_STATE;
@@ -1731,11 +1740,20 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
       batch = batch < 32 ? 16 : 64;
     }
   };
-  bool done = false, few = false;
+  const int64_t kNoLimit = last + 2;
+  bool done = false, few = false, begun = false;
   if (spec_eligible(c) && last > 64) {
-    // to a few iterates before the stop, no iterate before passing the test, then
+    // As few sweeps as the last solve took are tried first where that is less work than finding out
+    // (90 us; a solve of 16^3 to 0.1 takes 6 sweeps, 250).
+    const int64_t kQuick = 32;
+    if (c->last_sweeps > 0 && c->last_sweeps <= kQuick) {
+      PICARD_TRY(begin());
+      PICARD_TRY(sweep(1, 1, c->last_sweeps + 8, kQuick + 8));
+      done = fin.done != 0;
+    }
+    // Otherwise to a few iterates before the stop, no iterate before passing the test, then
     // the sweeps with it; a solve that passes one of its first two tests may have been taken past
-    // its stop by rounding and starts again with a wider margin
+    // its stop by rounding and starts again with a wider margin.
     const bool exact = !c->split && !c->order_free;
     for (int margin = 3; !done && margin <= 1024; margin *= 16) {
       PICARD_TRY(begin());
@@ -1746,8 +1764,8 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
       PICARD_TRY(spec_step(c, base ? c->jb[1] : c->U, base ? c->U : nullptr, base, margin, !exact, &to,
                            &ahead));
       if (to < 0) {
-        if (c->split) return kNoSpecStep;
-        few = to == kSpecFewLeft;
+        few = begun = to == kSpecFewLeft;      // iterates 0 and 1 are as they were: the sweeps follow
+        if (c->split && !few) return kNoSpecStep;
         break;
       }
       const int T = jacobi_block_sweeps(g);
@@ -1757,17 +1775,17 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
         to = base + T * launches;
         PICARD_TRY(launch_jacobi_block(c, base, launches));
       }
-      PICARD_TRY(sweep(to + 1, to + 1, ahead + 4));
+      PICARD_TRY(sweep(to + 1, to + 1, ahead + 4, kNoLimit));
       done = to >= maxit || fin.result > to + 2;
     }
   }
   if (!done) {
-    PICARD_TRY(begin());
+    if (!begun) PICARD_TRY(begin());
     // first batch from the previous solve's count (cold starts are alike from
     // step to step), then short batches: few no-op passes after convergence
     const int64_t kMaxBatch = int64_t(1) << 16;
     const int64_t batch = !few && c->last_sweeps > 64 ? (c->last_sweeps * 15) / 16 : 32;
-    PICARD_TRY(sweep(1, 1, batch < kMaxBatch ? batch : kMaxBatch));
+    PICARD_TRY(sweep(1, 1, batch < kMaxBatch ? batch : kMaxBatch, kNoLimit));
   }
   c->last_sweeps = fin.result;
   k_jacobi_finish<<<nbn, kT, 0, c->stream>>>(g, c->jb[0], c->jb[1], c->jb[2], c->U, fin.result);

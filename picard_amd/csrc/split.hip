@@ -10,9 +10,9 @@
 // Deposit: int64 fixed point (2^-40 units) with integer guard folds, so the
 // densities do not depend on particle order.  Field solve: the eigenbasis step
 // and FP64 sweeps of launch_calc_epotential; where that step is not taken (an
-// axis too long, a solve of few sweeps, a residual without a finite norm, or a
-// caller that asked for sweeps) iterative refinement -- FP32 Jacobi sweeps on the correction e of A e = r with an
-// FP64 outer residual r = b - A u and FP64 update u += e; the residual norm of
+// axis too long, maxit below 33, a residual without a finite norm, an early iterate that may pass the
+// rule, or a caller that asked for sweeps) iterative refinement -- FP32 Jacobi sweeps on the
+// correction e of A e = r with an FP64 outer residual r = b - A u and FP64 update u += e; the residual norm of
 // every sweep's iterate u + e_j (= r - A e_j) is accumulated in FP64, so the
 // stop rule of CalcEpotential.f90:60-62 is applied sweep by sweep.  E is
 // produced in FP32 for the gather; BCpotentials runs in FP64 (grid.hip).
