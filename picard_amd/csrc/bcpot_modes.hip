@@ -236,6 +236,7 @@ int bcpot_modes_prepare(picard_ctx *c, bool *even) {
 
 int launch_bcpot_modes(picard_ctx *c, double kfac) {
   const GridDims &g = c->gd;
+  if (!g.flow[0] && !g.flow[1] && !g.flow[2]) return PICARD_OK;      // no faces
   hipStream_t s = c->stream;
   const int px = (g.nx + 15) & ~15, lx = (2 * g.nx + 15) & ~15;
   const int64_t rows = (int64_t)g.ny * g.nz;
