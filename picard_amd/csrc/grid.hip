@@ -1737,7 +1737,7 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
         set_error("CalcEpotential: pass accounting out of step");
         return PICARD_ERR_STATE;
       }
-      batch = batch < 32 ? 16 : 64;
+      batch = batch < 32 ? 8 : 64;
     }
   };
   const int64_t kNoLimit = last + 2;
@@ -1775,7 +1775,7 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
         to = base + T * launches;
         PICARD_TRY(launch_jacobi_block(c, base, launches));
       }
-      PICARD_TRY(sweep(to + 1, to + 1, ahead + 4, kNoLimit));
+      PICARD_TRY(sweep(to + 1, to + 1, ahead + 2, kNoLimit));    // a stop is known two passes on
       done = to >= maxit || fin.result > to + 2;
     }
   }

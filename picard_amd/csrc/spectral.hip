@@ -22,8 +22,8 @@
 // B the part across the boundaries, 2 a (u_0 . v_n-1 + u_n-1 . v_0) of the first and last planes of
 // u = r_p and v = r_{p-1} for each periodic axis.  For the first iterates B is
 // formed as it stands; for the others every mode of a plane's sum enters with its modulus, which
-// falls with p, as f does, so that f(q) - B(p) > threshold^2 clears all iterates p to q.  Once the
-// slow modes are left that loses a few iterates at most (k_spec_clear).
+// falls with p, as f does, so that f(q) - B(p) > threshold^2 clears all iterates p to q.  What that
+// leaves open before the stop is looked at one by one again (k_spec_clear).
 //
 // Cost: six axis transforms of 2 n operations a cell, whatever the number of
 // sweeps (about 3 n^2 to 1e-6).  Measured, whole solve with its last sweeps
@@ -48,6 +48,7 @@ constexpr int kSpecFirst = 16;
 constexpr int kSpecLater = 40;
 constexpr int kSpecLook = kSpecFirst + kSpecLater;
 constexpr int kSpecEach = 4;        // of them in one block
+constexpr int kSpecNear = 32;       // and one by one again after the last of them that is clear
 
 // Device state of one search.  `skip`: no step is taken (0: go on).
 struct SpecState {
@@ -56,6 +57,9 @@ struct SpecState {
   double T, f0;                     // threshold^2, the base residual's norm^2
   double look[kSpecLater];          // the later iterates that are looked at, ascending
   double end;                       // the last of them: the crossing, or the last that is tested
+  double clear, above, left;        // iterates up to here do not pass, the bound there less B, sweeps left
+  double slope;                     // d ln f there
+  int32_t near;                     // more iterates are looked at one by one
   double steps;                     // sweeps the step covers
   int64_t to;                       // iterate the step ends on
   int64_t ahead;                    // sweeps from there to about the stop
@@ -197,7 +201,7 @@ __device__ __forceinline__ void spec_finish(const JacobiState *js, SpecState *st
     return;
   }
   st->to = to;
-  st->ahead = margin + (int64_t)(all ? 0.0 : fmin(left, 1024.0));
+  st->ahead = margin + (int64_t)(all ? 1.0 : fmax(1.0, fmin(left, 1024.0)));
   st->steps = (double)(to - base);
 }
 
@@ -339,24 +343,30 @@ struct SpecSeams {
 // boundary part signed, the later ones' of moduli; blockIdx.z: a periodic axis, a thread taking columns
 // of modes along it.  The plain norms come with the first axis.  A mode that has decayed by e^60 is left
 // out, in f to the safe side, in B by less than 1e-24 of the base norm, which the test adds.
-// The last block sums and decides.  Bound: the exponentials of every mode and iterate, 260 us at 160^3 with
+// The last block sums and decides.  NEAR, the second launch: the iterates that follow, one by one and signed
+// again, unless the first was sharp: 16 to 20 sweeps less for a solve to 1e-2 or 1e-3 (16^3 0.35 -> 0.26 ms,
+// 32^3 0.43 -> 0.29), where it is not needed one or two for 12 to 150 us.
+// Bound: the exponentials of every mode and iterate, 260 us at 160^3 with
 // two periodic axes (393 with the logarithm of the decayed modes too); on small grids the
 // chain of one column and the decision, 18 us at 16^3 (eight iterates a block and the decision in one
 // thread: 39).
+template <bool NEAR>
 __global__ void __launch_bounds__(kT) k_spec_clear(SpecGeo g, SpecSeams ss, const double *__restrict__ R,
                                                    double *__restrict__ partials, const JacobiState *js,
                                                    SpecState *st, int64_t base, int margin) {
   constexpr int N = kSpecEach;
+  constexpr int kLook = NEAR ? kSpecNear : kSpecLook, kFirst = NEAR ? kSpecNear : kSpecFirst;
   __shared__ double sh[kT / 64][2 * N];
-  __shared__ double sums[kSpecLook][4];              // f, then an axis each
-  if (st->skip) return;
+  __shared__ double sums[kLook][4];                  // f, then an axis each
+  if (st->skip || (NEAR && !st->near)) return;
   const SpecSeam m = ss.s[blockIdx.z];
   const int first = (int)blockIdx.y * N;             // the block's iterates
+  const double past = NEAR ? st->clear + (double)first : 0.0;
   const int nx[3] = {g.nx, g.ny, g.nz};
   double q[N], acc[2 * N];                           // f, then B
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    const int j = first + i - kSpecFirst;
+    const int j = first + i - kFirst;
     q[i] = j >= 0 ? st->look[j] - 1.0 : 0.0;
     acc[i] = acc[N + i] = 0.0;
   }
@@ -367,7 +377,7 @@ __global__ void __launch_bounds__(kT) k_spec_clear(SpecGeo g, SpecSeams ss, cons
     const int ia = (int)(t % m.ca), ib = (int)(t / m.ca);
     const double *r = R + ia * m.sa + ib * m.sb;
     const double sab = ea[ia] + eb[ib], cab = ea[nx[m.ax_a] + ia] + eb[nx[m.ax_b] + ib];
-    if (first < kSpecFirst) {
+    if (NEAR || first < kFirst) {
       // the two planes' sums of iterates first .. first + N, the rule's being one later
       double v0[N + 1], vn[N + 1];
 #pragma unroll
@@ -377,7 +387,15 @@ __global__ void __launch_bounds__(kT) k_spec_clear(SpecGeo g, SpecSeams ss, cons
         const double lam = 1.0 - (sab + es[k]);
         double w = next;
         if (k + 1 < m.n) next = r[(k + 1) * m.s];
-        for (int i = 0; i < first; ++i) w *= lam;
+        if (NEAR) {
+          bool neg;
+          const double s = sab + es[k], c = cab + es[m.n + k];
+          if (past * fmin(s, c) > 60.0) continue;
+          const double e = exp(past * spec_ln(s, c, &neg));
+          w = neg && fmod(past, 2.0) != 0.0 ? -w * e : w * e;
+        } else {
+          for (int i = 0; i < first; ++i) w *= lam;
+        }
         const double Q0 = m.Q[k], Qn = m.Q[(int64_t)(m.n - 1) * np + k];
 #pragma unroll
         for (int i = 0; i <= N; ++i) {
@@ -432,7 +450,7 @@ __global__ void __launch_bounds__(kT) k_spec_clear(SpecGeo g, SpecSeams ss, cons
   __syncthreads();                       // before the fence of thread 0
   if (!last_block(&st->arrive)) return;
   static_assert(kSpecLook * 4 <= kT && kSpecLook < 64 && kSpecFirst % kSpecEach == 0, "one thread a sum, one lane an iterate");
-  if ((int)threadIdx.x < kSpecLook * 4) {
+  if ((int)threadIdx.x < kLook * 4) {
     const int i = (int)threadIdx.x >> 2, w = (int)threadIdx.x & 3;
     double v = 0.0;
     if (w <= ss.count)
@@ -444,31 +462,61 @@ __global__ void __launch_bounds__(kT) k_spec_clear(SpecGeo g, SpecSeams ss, cons
   // a lane an iterate: is it, or the stretch up to it from the one before, clear?
   const int l = (int)threadIdx.x;
   const double T = st->T + 1.0e-24 * st->f0;
-  const int from = l <= kSpecFirst ? l : l - 1;      // whose B
-  const bool ok = l < kSpecLook && (l == kSpecFirst ||
-                                    sums[l][0] - (sums[from][1] + sums[from][2] + sums[from][3]) > T);
+  const int from = l <= kFirst ? l : l - 1;          // whose B
+  const bool ok = l < kLook && ((!NEAR && l == kFirst) ||
+                                sums[l][0] - (sums[from][1] + sums[from][2] + sums[from][3]) > T);
   const int cleared = (int)__builtin_ctzll(~__ballot(ok));     // lane 63 is none
   if (l) return;
   st->arrive = 0;
-  double clear = (double)cleared, f = 0.0, B = 0.0, left = 0.0;
-  if (cleared > kSpecFirst) {
+  double f = 0.0, B = 0.0;
+  if (cleared) {
     const double *v = sums[cleared - 1];
     f = v[0];
     B = v[1] + v[2] + v[3];
-    const double at = st->look[cleared - 1 - kSpecFirst];
+  }
+  // sweeps until the rule's norm meets the threshold, about: where one mode is left B falls as f does, and
+  // the square of the part across the boundaries, which B leaves out, is a / 2 of it, 1 / 12
+  auto until = [&](double slope) {
+    return slope < 0.0 && B < f ? fmax(0.0, log(T / (f - 0.917 * B)) / slope) : 0.0;
+  };
+  if (NEAR) {
+    const double clear = fmin(st->end, st->clear + (double)cleared);
+    double left = st->left;
+    if (cleared) {
+      if (clear > st->clear) st->above = f - B;
+      left = 1.0 + ceil(until(st->slope));
+    }
+    spec_finish(js, st, base, margin, clear, st->above, left);
+    return;
+  }
+  double clear = (double)cleared, left = 0.0;
+  if (cleared > kFirst) {
+    const double at = st->look[cleared - 1 - kFirst];
     clear = at;
     // ln f is convex: the chord from the nearest one before, continued, lies below it
-    int was = cleared - 2 - kSpecFirst;
+    int was = cleared - 2 - kFirst;
     while (was >= 0 && st->look[was] >= at) --was;
-    const double slope =
-        was >= 0 ? log(f / sums[kSpecFirst + was][0]) / (at - st->look[was]) : 0.0;
+    const double slope = was >= 0 ? log(f / sums[kFirst + was][0]) / (at - st->look[was]) : 0.0;
     if (slope < 0.0 && clear < st->end) {
       if (f - B > T) clear = fmin(st->end, clear + floor(log((T + B) / f) / slope));
-      // the boundary part is about 0.92 of B where one mode is left
-      left = fmax(0.0, at + ceil(log((T + 0.92 * B) / f) / slope) - clear);
+      left = fmax(0.0, 1.0 + ceil(at + until(slope) - clear));
     }
+    st->slope = slope;
+  } else {
+    st->slope = 0.0;
   }
-  spec_finish(js, st, base, margin, clear, f - B, left);
+  // Where the mode left is constant across the boundaries B is sharp, a few sweeps short of the stop;
+  // where more are left it is several times that.
+  double sharp = 0.0;
+  for (int d = 0; d < ss.count; ++d) sharp += 4.0 * ss.s[d].a / (double)ss.s[d].n;
+  st->near = B > 1.1 * sharp * f && clear < st->end ? 1 : 0;
+  if (!st->near) {
+    spec_finish(js, st, base, margin, clear, f - B, left);
+    return;
+  }
+  st->clear = clear;
+  st->above = f - B;
+  st->left = left;
 }
 
 // The spectrum of the step's change of U, -af times the sum of its sweeps' residuals.
@@ -692,7 +740,9 @@ int spec_step(picard_ctx *c, const double *u, const double *old, int64_t base, i
   if (ss.count) {
     const int64_t room = 4 * c->s.partials_len / (4 * kSpecLook);
     const int64_t nb = std::max<int64_t>(1, std::min((columns + kT - 1) / kT, room));
-    k_spec_clear<<<dim3((unsigned)nb, kSpecLook / kSpecEach, ss.count), kT, 0, s>>>(
+    k_spec_clear<false><<<dim3((unsigned)nb, kSpecLook / kSpecEach, ss.count), kT, 0, s>>>(
+        sg, ss, B0, part, c->js, st, base, margin);
+    k_spec_clear<true><<<dim3((unsigned)nb, kSpecNear / kSpecEach, ss.count), kT, 0, s>>>(
         sg, ss, B0, part, c->js, st, base, margin);
   }
   if (apply) {
