@@ -53,6 +53,14 @@ __device__ __forceinline__ void static_for(F &&f) {
   }
 }
 
+// Between lanes' stores to LDS and other lanes' reads of them, and between those reads and the next
+// stores there.  A block is one wave, whose LDS accesses the hardware keeps in order: this holds
+// the compiler to it and costs no instruction.
+__device__ __forceinline__ void staged() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // LDS of one block, in doubles: charge rows, then the ring or the rows of distances.
 template <int NC>
 constexpr int kFaceLds = kRB * 64 * NC + (64 * NC * kPitch > kRB * 64 * (NC + 1) ? 64 * NC * kPitch
@@ -154,6 +162,7 @@ __device__ __forceinline__ double face_chain(const FaceTask &t, const double *__
   int slot = 0;                                        // x faces: the row's newest column
   fetch();
   for (int k = 1; k <= nz; ++k) {
+    staged();                                          // the last plane's reads
     if (XF) {                                          // a new plane: the 63 older columns
       slot = 63;
       // below y = 0 there is no column, and no lane with a node uses one
@@ -173,6 +182,7 @@ __device__ __forceinline__ double face_chain(const FaceTask &t, const double *__
       }
     }
     for (int j = 1; j <= ny; j += kRB) {
+      staged();                                        // the last rows' reads
 #pragma unroll
       for (int b = 0; b < kRB; ++b) {
         const int sl = XF ? (slot + b >= kRing ? slot + b - kRing : slot + b) : b;
@@ -180,6 +190,7 @@ __device__ __forceinline__ double face_chain(const FaceTask &t, const double *__
 #pragma unroll
         for (int q = 0; q < NC; ++q) crow[b * NP + lane + 64 * q] = rc[b][q];
       }
+      staged();
       fetch();
       const int rows = ny + 1 - j < kRB ? ny + 1 - j : kRB;
       for (int b = 0; b < rows; ++b) {
