@@ -107,11 +107,25 @@ class _Lane:
         self.tuned = False
 
 
-# An idle lane that gets a job waits this long for others, so that jobs of one
-# burst start in the same launches: a small job's step (about 1 ms) costs as many
-# launches as a full batch's.  A lane with jobs on the device admits at every
-# step and never waits.
+# An idle lane starts jobs that arrive within this time of each other together, in the same launches:
+# a small job's step costs as many launches as a full batch's.  It waits for the next arrival only
+# where one is due in that time and fits beside those that are there; a job with no other behind it
+# starts at once, and so does every job that finds the lane at work.
 GATHER_S = 0.010
+
+
+def gather_until(pending, now: float, fits) -> float:
+    """When an idle lane should start the jobs at the head of `pending` (by arrival): `now`, or the next
+    arrival within GATHER_S of the first if fits(jobs) holds for the arrived ones and it."""
+    if not pending or pending[0].arrival > now:
+        return now
+    jobs = []
+    for j in pending:
+        jobs.append(j)
+        if j.arrival > now:
+            due = j.arrival <= pending[0].arrival + GATHER_S
+            return j.arrival if due and fits(jobs) else now
+    return now
 
 
 class Server:
@@ -157,6 +171,15 @@ class Server:
         errors: list[BaseException] = []
         t0 = time.perf_counter()
 
+        def fits_empty(q: int, batch: list[Job]) -> bool:
+            cap = self.lanes[q].spec
+            with self._lock:
+                held = sh["held"]
+            return (len(batch) <= cap.max_sims and
+                    sum(j.spec.cells for j in batch) <= cap.max_cells and
+                    sum(ensemble.footprint(j.spec)[1] for j in batch) <= cap.max_particles and
+                    held + sum(j.bytes for j in batch) <= self.budget)
+
         def serve(q: int):
             ln, pending = self.lanes[q], queues[q]
             ens, cap = ln.ens, ln.spec
@@ -166,9 +189,13 @@ class Server:
                 now = time.perf_counter() - t0
                 if time_limit is not None and now > time_limit:
                     break
-                if not running and pending and 0.0 <= now - pending[0].arrival < GATHER_S:
-                    time.sleep(GATHER_S - (now - pending[0].arrival))
-                    continue
+                if not running:
+                    until = gather_until(pending, now, lambda jobs: fits_empty(q, jobs))
+                    if time_limit is not None:
+                        until = min(until, time_limit)
+                    if until > now:
+                        time.sleep(until - now)
+                        continue
                 # admit, in arrival order, every job of this lane that has
                 # arrived and fits the lane and the shared budget
                 while pending and pending[0].arrival <= now:
