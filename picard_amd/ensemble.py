@@ -100,6 +100,15 @@ def footprint(spec: SimSpec) -> tuple[int, int]:
     return g.value, n.value
 
 
+# longest axis that the solve takes in closed form (picard_ensemble.h); beyond it is swept
+CLOSED_FORM_MAX_AXIS = 1024
+
+
+def swept(spec: SimSpec) -> bool:
+    """Whether the solve of a simulation runs the sweeps that the tile shape is about."""
+    return max(spec.nx, spec.ny, spec.nz) > CLOSED_FORM_MAX_AXIS
+
+
 # bytes per particle slot of the ensemble's arena: int16 cell x3, FP32 offset
 # x3, FP32 velocity x3, species, slot, id, sort rank; two arenas for the sort
 PARTICLE_BYTES = 2 * (6 + 12 + 12 + 1 + 2 + 4) + 4

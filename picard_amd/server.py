@@ -225,7 +225,9 @@ class Server:
                     wait = pending[0].arrival - now if pending else 0.0
                     time.sleep(min(max(wait, 0.001), 0.05))
                     continue
-                if self.tune_sweeps and not ln.tuned:
+                # inside the latency of the lane's first job that is swept, and of no other's
+                if (self.tune_sweeps and not ln.tuned and
+                        any(ensemble.swept(j.spec) for j in running.values())):
                     ens.tune(self.tune_sweeps)
                     ln.tuned = True
                 ts = time.perf_counter()

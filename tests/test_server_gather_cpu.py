@@ -83,3 +83,14 @@ def test_the_time_limit_ends_the_wait(monkeypatch):
 def test_gather_until(arrivals, now, want):
     assert server.gather_until(_jobs(*arrivals), now, lambda jobs: True) == want
     assert server.gather_until(_jobs(*arrivals), now, lambda jobs: False) == now
+
+
+@pytest.mark.parametrize("edge,tuned", [(16, 0), (1024, 0), (1025, 1)])
+def test_only_jobs_that_are_swept_are_tuned_for(monkeypatch, edge, tuned):
+    monkeypatch.setattr(ensemble, "Ensemble", _Ensemble)
+    jobs = _jobs(0.0, 0.05)
+    jobs[1].spec.nx, jobs[1].spec.ny, jobs[1].spec.nz = edge, 8, 8
+    srv = server.Server(tune_sweeps=32)
+    srv.run(jobs)
+    assert srv.lanes[0].ens.tuned == tuned
+    srv.close()
