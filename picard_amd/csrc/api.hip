@@ -231,12 +231,12 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   PICARD_TRY(dalloc(&c->D, DN));
   // the Jacobi iterates and b start one element into their allocations, so
   // that node pairs (i, i+1) with i even are 16-byte aligned when nx is even
-  for (int q = 0; q < 3; ++q) {
+  // (split form: with the eigenbasis step's arrays, below)
+  for (int q = 0; q < 3 && !c->split; ++q) {
     PICARD_TRY(dalloc(&c->jb_mem[q], g.G + 2));
     c->jb[q] = c->jb_mem[q] + 1;
   }
   PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->js_host), kHostState));
-  if (spec_eligible(c)) PICARD_TRY(spec_create(c));
   PICARD_TRY(dalloc(&c->b_mem, g.G + 2));
   c->b = c->b_mem + 1;
   PICARD_TRY(dalloc(&c->consts, 16));
@@ -277,6 +277,8 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   PICARD_HIP(hipMemsetAsync(c->C, 0, sizeof(double) * g.G, c->stream));
   PICARD_HIP(hipMemsetAsync(c->D, 0, sizeof(double) * DN, c->stream));
   PICARD_TRY(upload_species(c));
+  // last, as the domain can do without
+  PICARD_TRY(spec_create(c));
   return PICARD_OK;
 }
 
@@ -320,12 +322,21 @@ double *field_ptr(picard_ctx *c, int which) {
 int ensure_flux(picard_ctx *c) {
   const GridDims &g = c->gd;
   const int64_t len = 3 * (int64_t)g.S * g.G;
-  if (!c->F) PICARD_TRY(dalloc(&c->F, len));
-  if (c->split) {
-    if (!c->Ffix) PICARD_TRY(dalloc(&c->Ffix, len));
-  } else {
-    if (!c->Fraw) PICARD_TRY(dalloc(&c->Fraw, len));
+  auto later = [&](auto **p) { return *p ? PICARD_OK : alloc_later(c, reinterpret_cast<void **>(p), 8 * len); };
+  PICARD_TRY(later(&c->F));
+  return c->split ? later(&c->Ffix) : later(&c->Fraw);
+}
+
+int alloc_later(picard_ctx *c, void **p, int64_t bytes) {
+  *p = nullptr;
+  hipError_t rc = hipMalloc(p, (size_t)bytes);
+  if (rc == hipErrorOutOfMemory && c->spec_mem) {
+    (void)hipGetLastError();
+    PICARD_HIP(hipStreamSynchronize(c->stream));
+    spec_release(c);
+    rc = hipMalloc(p, (size_t)bytes);
   }
+  PICARD_HIP(rc);
   return PICARD_OK;
 }
 

@@ -235,13 +235,13 @@ int bcpot_fft_prepare(picard_ctx *c) {
     const int64_t plane = (int64_t)fg.M1 * fg.M2;
     for (int f = 0; f < 2; ++f) {
       if (!c->fft_K[d][f])
-        PICARD_HIP(hipMalloc(reinterpret_cast<void **>(&c->fft_K[d][f]),
-                             sizeof(double2) * plane * fg.nd));
+        PICARD_TRY(alloc_later(c, reinterpret_cast<void **>(&c->fft_K[d][f]),
+                               sizeof(double2) * plane * fg.nd));
     }
     for (int a = 0; a < 2; ++a) {
       const int L = a == 0 ? fg.M1 : fg.M2;
       if (!c->fft_tw[d][a])
-        PICARD_HIP(hipMalloc(reinterpret_cast<void **>(&c->fft_tw[d][a]), sizeof(double2) * 512));
+        PICARD_TRY(alloc_later(c, reinterpret_cast<void **>(&c->fft_tw[d][a]), sizeof(double2) * 512));
       k_twiddles<<<grid_blocks(L / 2, 256), 256, 0, c->stream>>>(c->fft_tw[d][a], L);
       PICARD_HIP(hipGetLastError());
     }
@@ -249,8 +249,9 @@ int bcpot_fft_prepare(picard_ctx *c) {
     if (c->fft_work_len < plane * (fg.nd + 2)) {
       if (c->fft_work) PICARD_HIP(hipFree(c->fft_work));
       c->fft_work = nullptr;
-      PICARD_HIP(hipMalloc(reinterpret_cast<void **>(&c->fft_work),
-                           sizeof(double2) * plane * (fg.nd + 2)));
+      c->fft_work_len = 0;
+      PICARD_TRY(alloc_later(c, reinterpret_cast<void **>(&c->fft_work),
+                             sizeof(double2) * plane * (fg.nd + 2)));
       c->fft_work_len = plane * (fg.nd + 2);
     }
     for (int f = 0; f < 2; ++f) {

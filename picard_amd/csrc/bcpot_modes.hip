@@ -212,18 +212,20 @@ int bcpot_modes_prepare(picard_ctx *c, bool *even) {
   PICARD_HIP(hipStreamSynchronize(s));
   *even = c->host_counters[0] == 0;
   if (!*even) return PICARD_OK;
-  if (!c->face_work) PICARD_HIP(hipMalloc(&c->face_work, sizeof(double) * work_len(g)));
+  auto later = [&](double **p, int64_t doubles) {
+    return *p ? PICARD_OK : alloc_later(c, reinterpret_cast<void **>(p), (int64_t)sizeof(double) * doubles);
+  };
+  PICARD_TRY(later(&c->face_work, work_len(g)));
   for (int d = 0; d < 3; ++d) {
-    if (!(g.flow[(d + 1) % 3] || g.flow[(d + 2) % 3]) || c->face_fwd[d]) continue;
-    PICARD_HIP(hipMalloc(&c->face_fwd[d], sizeof(double) * spec_mat_len(2 * n[d])));
-    PICARD_HIP(hipMalloc(&c->face_inv[d], sizeof(double) * spec_mat_len(2 * n[d])));
+    if (!(g.flow[(d + 1) % 3] || g.flow[(d + 2) % 3]) || (c->face_fwd[d] && c->face_inv[d])) continue;
+    PICARD_TRY(later(&c->face_fwd[d], spec_mat_len(2 * n[d])));
+    PICARD_TRY(later(&c->face_inv[d], spec_mat_len(2 * n[d])));
     PICARD_TRY(spec_axis_tables(s, 2 * n[d], false, 0.0, c->face_fwd[d], c->face_inv[d], nullptr));
   }
   for (int d = 0; d < 3; ++d) {
     if (!g.flow[d]) continue;
     const ModeGeo m = mode_geo(g, d);
-    if (!c->face_lam[d])
-      PICARD_HIP(hipMalloc(&c->face_lam[d], sizeof(double) * m.nd * (m.n1 + 1) * (m.n2 + 1)));
+    PICARD_TRY(later(&c->face_lam[d], (int64_t)m.nd * (m.n1 + 1) * (m.n2 + 1)));
     // A: nd n2 (n1 + 1) values of the work array's 7 nd n1 n2
     k_modes_eig<true><<<blocks_of((int64_t)m.nd * m.n2 * (m.n1 + 1)), kT, 0, s>>>(
         m, c->face_fwd[d == 0 ? 1 : 0], c->D, c->face_work, nullptr);

@@ -298,8 +298,9 @@ int ensure_stage(picard_ctx *c, int64_t want) {
   if (c->s.stage_sp) PICARD_HIP(hipFree(c->s.stage_sp));
   c->s.stage = nullptr;
   c->s.stage_sp = nullptr;
-  PICARD_HIP(hipMalloc(&c->s.stage, sizeof(double) * 8 * want));
-  PICARD_HIP(hipMalloc(&c->s.stage_sp, sizeof(int32_t) * want));
+  c->s.stage_cap = 0;
+  PICARD_TRY(alloc_later(c, reinterpret_cast<void **>(&c->s.stage), (int64_t)sizeof(double) * 8 * want));
+  PICARD_TRY(alloc_later(c, reinterpret_cast<void **>(&c->s.stage_sp), (int64_t)sizeof(int32_t) * want));
   c->s.stage_cap = want;
   return PICARD_OK;
 }

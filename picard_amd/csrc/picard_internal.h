@@ -276,6 +276,7 @@ int launch_bc_fields(picard_ctx *c);
 
 // ---- spectral.hip ----
 bool spec_eligible(const picard_ctx *c);
+// spec_create: no memory for its arrays is no error, the context then has none
 int spec_create(picard_ctx *c);
 void spec_release(picard_ctx *c);
 // apply = false: only finds the iterate
@@ -318,6 +319,9 @@ int sp_sort(picard_ctx *c, int wrap, int64_t npush = 0, double dt = 0.0);
 int sp_gridify(picard_ctx *c, bool flux = false);
 // allocates the flux arrays (F, and Fraw or Ffix) on first use
 int ensure_flux(picard_ctx *c);
+// device memory for a context that is at work: where there is none left, the eigenbasis step's
+// arrays are given up for it and solves sweep from then on
+int alloc_later(picard_ctx *c, void **p, int64_t bytes);
 int sp_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t *sweeps);
 int sp_efield(picard_ctx *c);
 int sp_widen_e(picard_ctx *c);

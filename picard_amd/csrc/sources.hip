@@ -325,7 +325,7 @@ int produce_haser(picard_ctx *c, const picard_plasma *pl, const picard_haser *hs
     if (c->haser_off) PICARD_HIP(hipFree(c->haser_off));
     c->haser_off = nullptr;
     c->haser_len = 0;
-    PICARD_HIP(hipMalloc(reinterpret_cast<void **>(&c->haser_off), sizeof(int32_t) * (ncs + 1)));
+    PICARD_TRY(alloc_later(c, reinterpret_cast<void **>(&c->haser_off), (int64_t)sizeof(int32_t) * (ncs + 1)));
     c->haser_len = ncs + 1;
   }
   if (c->s.scan_tmp_len < scan_tmp_required(ncs)) {

@@ -590,15 +590,16 @@ void launch_axis(hipStream_t s, const SpecTile &t, const SpecState *st) {
 
 // The forms that are held to the reference's rounding use it to find their
 // stop, where the sweeps up to it can do without the stop test.
-bool spec_eligible(const picard_ctx *c) {
-  const GridDims &g = c->gd;
-  const bool form = c->split ? !c->mx_forced : c->order_free || jacobi_block_eligible(g);
-  return form && g.nx <= kSpecMaxAxis && g.ny <= kSpecMaxAxis && g.nz <= kSpecMaxAxis;
-}
+bool spec_eligible(const picard_ctx *c) { return c->spec_mem && !(c->split && c->mx_forced); }
 
+// The split form's FP64 iterates go with them: its own sweeps do without.
 void spec_release(picard_ctx *c) {
   if (c->spec_mem) (void)hipFree(c->spec_mem);
   c->spec_mem = nullptr;
+  for (int q = 0; q < 3 && c->split; ++q) {
+    if (c->jb_mem[q]) (void)hipFree(c->jb_mem[q]);
+    c->jb_mem[q] = c->jb[q] = nullptr;
+  }
 }
 
 // Basis, transpose and eigenvalue parts of one axis; `a` is the Jacobi weight of its neighbours.
@@ -633,6 +634,9 @@ double spec_slowest(const int n[3], const int flow[3], const double a[3]) {
 int spec_create(picard_ctx *c) {
   const GridDims &g = c->gd;
   const int n[3] = {g.nx, g.ny, g.nz};
+  if (!(c->split || c->order_free || jacobi_block_eligible(g)) || n[0] > kSpecMaxAxis ||
+      n[1] > kSpecMaxAxis || n[2] > kSpecMaxAxis)
+    return PICARD_OK;
   const double d2[3] = {g.dxyz[0] * g.dxyz[0], g.dxyz[1] * g.dxyz[1], g.dxyz[2] * g.dxyz[2]};
   const double sum = 1.0 / d2[0] + 1.0 / d2[1] + 1.0 / d2[2];
   // one allocation, its parts at multiples of 256 bytes
@@ -641,7 +645,17 @@ int spec_create(picard_ctx *c) {
   const int64_t state = part((int64_t)(sizeof(SpecState) + sizeof(double) - 1) / (int64_t)sizeof(double));
   int64_t total = 3 * len + state;
   for (int d = 0; d < 3; ++d) total += 2 * spec_mat_len(n[d]) + part(2 * n[d]);
-  PICARD_HIP(hipMalloc(&c->spec_mem, sizeof(double) * total));
+  hipError_t rc = hipMalloc(&c->spec_mem, sizeof(double) * total);
+  for (int q = 0; q < 3 && c->split && rc == hipSuccess; ++q) {
+    rc = hipMalloc(&c->jb_mem[q], sizeof(double) * (g.G + 2));
+    c->jb[q] = c->jb_mem[q] + 1;
+  }
+  if (rc != hipSuccess) {
+    (void)hipGetLastError();
+    spec_release(c);
+    if (rc == hipErrorOutOfMemory) return PICARD_OK;
+    PICARD_HIP(rc);
+  }
   double *p = c->spec_mem;
   auto take = [&](int64_t doubles) {
     double *q = p;
