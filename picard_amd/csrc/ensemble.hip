@@ -48,6 +48,7 @@
 
 #include "../../include/picard_ensemble.h"
 #include "picard_internal.h"
+#include "grow.h"
 #include "readback.h"
 #include "split_particles.h"
 #include "reduce.h"
@@ -1990,21 +1991,20 @@ static void drop_axes(picard_ensemble *e, SlotHost &h) {
 }
 
 // Spectral work lists grow with what they hold (the graphs keep their
-// addresses, so they are captured again).
+// addresses, so they are captured again).  Without memory for more they stay as they are, and so
+// do the lists of the simulations that are there.
 static int grow_lists(picard_ensemble *e, const std::vector<Tile> &tiles, const std::vector<Tile> *axis) {
   auto grow = [&](auto **p, int64_t *cap, int64_t want, int64_t per) -> int {
-    if (want <= *cap) return PICARD_OK;
-    PICARD_HIP(hipStreamSynchronize(e->stream));
-    free_graphs(e);
-    if (*p) {
-      e->allocs.erase(std::find(e->allocs.begin(), e->allocs.end(), (void *)*p));
-      (void)hipFree(*p);
-      *p = nullptr;
-    }
-    *cap = 0;
-    PICARD_TRY(dalloc_n(e, p, per * (want + want / 2)));
-    *cap = want + want / 2;
-    return PICARD_OK;
+    return grow_array(
+        p, cap, want, per, [&](auto **q, int64_t n) { return dalloc_n(e, q, n); },
+        [&](void *old) -> int {
+          PICARD_HIP(hipStreamSynchronize(e->stream));
+          free_graphs(e);
+          if (!old) return PICARD_OK;
+          e->allocs.erase(std::find(e->allocs.begin(), e->allocs.end(), old));
+          (void)hipFree(old);
+          return PICARD_OK;
+        });
   };
   for (int d = 0; d < 3; ++d)
     PICARD_TRY(grow(&e->A.sp_axis[d], &e->cap_sp_axis[d], (int64_t)axis[d].size(), 1));

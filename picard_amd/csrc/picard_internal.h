@@ -20,6 +20,7 @@ void set_error(const std::string &msg);
     hipError_t e_ = (call);                                                         \
     if (e_ != hipSuccess) {                                                         \
       ::picard::set_error(std::string(#call) + ": " + hipGetErrorString(e_));       \
+      (void)hipGetLastError(); /* reported here, not by the next launch's check */  \
       return PICARD_ERR_HIP;                                                        \
     }                                                                               \
   } while (0)
