@@ -268,7 +268,7 @@ int create_impl(const picard_geometry *geo, const picard_species *sp, picard_ctx
   c->s.partials_len = pb;
   PICARD_TRY(dalloc(&c->s.partials, 4 * pb));     // two launches' worth (read + write) and scratch
   // allocating its chunks, 0.25 ms each pair, is worth it from a few MB on
-  c->readback = new Readback(int64_t(4) << 20);
+  c->readback = new Readback(int64_t(4) << 20, int64_t(4) << 20);
   PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->host_counters), 16 * sizeof(int32_t)));
   // the reference zeroes U, N, E and the particle arrays at start (picard.f90:434-439)
   PICARD_HIP(hipMemsetAsync(c->U, 0, sizeof(double) * g.G, c->stream));

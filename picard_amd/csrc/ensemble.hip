@@ -1734,8 +1734,10 @@ struct picard_ensemble {
   int device = 0;
   int cus = 256;
   hipStream_t stream = nullptr;
-  // the simulations share its chunks; 0.05 MB takes the runtime 14 us, and 27 through one
-  Readback readback{int64_t(1) << 16};
+  // The simulations share its chunks.  A copy takes the runtime 15, 25, 39 and 63 us at 0.08, 0.3, 0.6 and 1.0
+  // MB where the chunks take 23, 33, 46 and 67, and 165 and 140 at 2.2; E, which the runtime's way
+  // widens into an array of its own first, is faster through them from 0.1 MB on.
+  Readback readback{int64_t(1) << 20, int64_t(1) << 16};
   Arenas A{};
   PartArena P[2]{};
   int cur = 0;                       // arena holding the sorted particles

@@ -9,8 +9,8 @@ namespace picard {
 
 class Readback {
  public:
-  // arrays of fewer than `direct` bytes go the runtime's way
-  explicit Readback(int64_t direct) : direct_(direct) {}
+  // copies of fewer than `copy` bytes and E of fewer than `widen` go the runtime's way
+  Readback(int64_t copy, int64_t widen) : direct_copy_(copy), direct_widen_(widen) {}
   ~Readback();
   // host[0 .. bytes) = dev, in the stream's order; returns when it is there
   int copy(int device, hipStream_t stream, void *host, const void *dev, int64_t bytes);
@@ -29,7 +29,7 @@ class Readback {
   template <typename OUT>
   hipError_t work(Worker &w, int device, hipStream_t stream, const char *dev, int64_t bytes,
                   int64_t chunk, int first, int step, const OUT &out);
-  const int64_t direct_;
+  const int64_t direct_copy_, direct_widen_;
   std::mutex mu_;
   Worker w_[kMaxWorkers];
 };

@@ -98,7 +98,7 @@ int Readback::run(int device, hipStream_t stream, const char *dev, int64_t bytes
 }
 
 int Readback::copy(int device, hipStream_t stream, void *host, const void *dev, int64_t bytes) {
-  if (bytes < direct_ || !pageable(host)) {
+  if (bytes < direct_copy_ || !pageable(host)) {
     PICARD_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream));
     PICARD_HIP(hipStreamSynchronize(stream));
     return PICARD_OK;
@@ -111,7 +111,7 @@ int Readback::copy(int device, hipStream_t stream, void *host, const void *dev, 
 
 int Readback::widen(int device, hipStream_t stream, double *host, const float4 *E, int64_t n,
                     bool *taken) {
-  *taken = n * (int64_t)sizeof(float4) >= direct_ && pageable(host);
+  *taken = n * (int64_t)sizeof(float4) >= direct_widen_ && pageable(host);
   if (!*taken) return PICARD_OK;
   return run(device, stream, reinterpret_cast<const char *>(E), n * (int64_t)sizeof(float4),
              [host](const char *pin, int64_t at, int64_t m) {
