@@ -67,12 +67,19 @@ int Readback::run(int device, hipStream_t stream, const char *dev, int64_t bytes
   const int64_t chunk = bytes < kBig ? kPin / 2 : kPin;
   const int cpus = std::max(1, (int)std::thread::hardware_concurrency());
   int workers = (int)std::min<int64_t>(std::min(kMaxWorkers, cpus), std::max<int64_t>(1, bytes / kPin));
-  for (int t = 0; t < workers; ++t)
+  // as many as there is pinned memory for
+  auto ready = [](Worker &w) {
     for (int b = 0; b < 2; ++b) {
-      if (!w_[t].pin[b])
-        PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&w_[t].pin[b]), kPin));
-      if (!w_[t].ev[b]) PICARD_HIP(hipEventCreateWithFlags(&w_[t].ev[b], hipEventDisableTiming));
+      if (!w.pin[b] && hipHostMalloc(reinterpret_cast<void **>(&w.pin[b]), kPin) != hipSuccess) return false;
+      if (!w.ev[b] && hipEventCreateWithFlags(&w.ev[b], hipEventDisableTiming) != hipSuccess) return false;
     }
+    return true;
+  };
+  int have = 0;
+  while (have < workers && ready(w_[have])) ++have;
+  if (have < workers) (void)hipGetLastError();
+  if (!have) return kNoChunks;
+  workers = have;
   hipError_t rc[kMaxWorkers] = {};
   std::thread threads[kMaxWorkers];
   int started = 1;
@@ -98,28 +105,31 @@ int Readback::run(int device, hipStream_t stream, const char *dev, int64_t bytes
 }
 
 int Readback::copy(int device, hipStream_t stream, void *host, const void *dev, int64_t bytes) {
-  if (bytes < direct_copy_ || !pageable(host)) {
-    PICARD_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream));
-    PICARD_HIP(hipStreamSynchronize(stream));
-    return PICARD_OK;
+  if (bytes >= direct_copy_ && pageable(host)) {
+    const int rc = run(device, stream, static_cast<const char *>(dev), bytes,
+                       [host](const char *pin, int64_t at, int64_t m) {
+                         std::memcpy(static_cast<char *>(host) + at, pin, m);
+                       });
+    if (rc != kNoChunks) return rc;
   }
-  return run(device, stream, static_cast<const char *>(dev), bytes,
-             [host](const char *pin, int64_t at, int64_t m) {
-               std::memcpy(static_cast<char *>(host) + at, pin, m);
-             });
+  PICARD_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream));
+  PICARD_HIP(hipStreamSynchronize(stream));
+  return PICARD_OK;
 }
 
 int Readback::widen(int device, hipStream_t stream, double *host, const float4 *E, int64_t n,
                     bool *taken) {
   *taken = n * (int64_t)sizeof(float4) >= direct_widen_ && pageable(host);
   if (!*taken) return PICARD_OK;
-  return run(device, stream, reinterpret_cast<const char *>(E), n * (int64_t)sizeof(float4),
+  const int rc = run(device, stream, reinterpret_cast<const char *>(E), n * (int64_t)sizeof(float4),
              [host](const char *pin, int64_t at, int64_t m) {
                const float *e = reinterpret_cast<const float *>(pin);
                double *o = host + 3 * (at / (int64_t)sizeof(float4));
                for (int64_t q = 0; q < m / (int64_t)sizeof(float4); ++q)
                  for (int d = 0; d < 3; ++d) o[3 * q + d] = e[4 * q + d];
              });
+  *taken = rc != kNoChunks;
+  return *taken ? rc : PICARD_OK;
 }
 
 }  // namespace picard
