@@ -802,7 +802,7 @@ __global__ void __launch_bounds__(kT) k_sp_residual(Arenas A) {
     const Tile tl = A.sp_tiles[t];
     const SimDev &sd = A.sims[tl.slot];
     const double *u = A.u[0] + sd.gbase, *Cs = A.C + sd.gbase;
-    double *out = A.sp[0] + sd.sbase;
+    double *out = sd.sp_ok ? A.sp[0] + sd.sbase : nullptr;     // the sums are every slot's
     const int64_t X = sd.X, XY = (int64_t)sd.X * sd.Y;
     const double i2 = sd.i2, dVeps0 = sd.dVeps0;
     const uint32_t nx = (uint32_t)sd.nx, ny = (uint32_t)sd.ny, nz = (uint32_t)sd.nz;
@@ -824,7 +824,7 @@ __global__ void __launch_bounds__(kT) k_sp_residual(Arenas A) {
         bb += b * b;
         rr += r * r;
       }
-      out[el] = r;
+      if (out) out[el] = r;
     }
     const double s0 = block_sum(bb, sh[0]), s1 = block_sum(rr, sh[1]);
     if (threadIdx.x == 0) {
@@ -1057,6 +1057,7 @@ __global__ void __launch_bounds__(kT) k_sp_charge(Arenas A) {
   for (int t = blockIdx.x; t < nt; t += gridDim.x) {
     const Tile tl = A.sp_tiles[t];
     const SimDev &sd = A.sims[tl.slot];
+    if (!sd.sp_ok) continue;
     for (int q = 0; q < kSpecTile / kT; ++q) {
       const uint32_t el = (uint32_t)tl.a + q * kT + threadIdx.x;
       if (el >= (uint32_t)sd.slen) break;
@@ -1957,7 +1958,7 @@ constexpr int64_t kAxesKept = int64_t(256) << 20;
 
 static int hold_axes(picard_ensemble *e, SlotHost &h) {
   const int n[3] = {h.p.nx, h.p.ny, h.p.nz}, flow[3] = {1, 0, 0};
-  if (n[0] > kSpecMaxAxis || n[1] > kSpecMaxAxis || n[2] > kSpecMaxAxis) return PICARD_OK;
+  if (!e->A.sp[0] || n[0] > kSpecMaxAxis || n[1] > kSpecMaxAxis || n[2] > kSpecMaxAxis) return PICARD_OK;
   for (int d = 0; d < 3; ++d) {
     auto &t = e->axes[{n[d], flow[d]}];
     if (!t.mem) {
@@ -2369,7 +2370,6 @@ int picard_ensemble_create(const picard_ensemble_config *cfg, picard_ensemble **
   PICARD_TRY(dalloc_n(e, &A.fscr, e->max_face));
   PICARD_TRY(dalloc_n(e, &A.r32, e->max_cells));
   for (int q = 0; q < kEBufs; ++q) PICARD_TRY(dalloc_n(e, &A.e32[q], e->max_cells));
-  for (int q = 0; q < 3; ++q) PICARD_TRY(dalloc_n(e, &A.sp[q], 2 * e->max_cells));
   PICARD_TRY(dalloc_n(e, &A.hist, kcap + 1));
   PICARD_TRY(dalloc_n(e, &A.rank, e->cap));
   e->scan_tmp_len = scan_tmp_required(kcap);
@@ -2393,6 +2393,21 @@ int picard_ensemble_create(const picard_ensemble_config *cfg, picard_ensemble **
                            hipHostMallocMapped | hipHostMallocCoherent));
   PICARD_HIP(hipHostMalloc(reinterpret_cast<void **>(&e->host_err), sizeof(int32_t),
                            hipHostMallocMapped | hipHostMallocCoherent));
+  // last, as the simulations can do without: with no room for them their solves sweep
+  for (int q = 0; q < 3; ++q) {
+    const hipError_t rc = hipMalloc(reinterpret_cast<void **>(&A.sp[q]), sizeof(double) * 2 * e->max_cells);
+    if (rc == hipSuccess) continue;
+    (void)hipGetLastError();
+    A.sp[q] = nullptr;
+    while (q > 0) {
+      (void)hipFree(A.sp[--q]);
+      A.sp[q] = nullptr;
+    }
+    if (rc == hipErrorOutOfMemory) break;
+    PICARD_HIP(rc);
+  }
+  for (double *b : A.sp)
+    if (b) e->allocs.push_back(b);
   for (auto &ev : e->chunk_ev) PICARD_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
   std::memset(e->host_status, 0, sizeof(picard_sim_status) * S);
   *e->host_n = 0;
