@@ -1173,7 +1173,6 @@ __global__ void __launch_bounds__(kT) k_jacobi_finish(GridDims g, double *b0, do
                                                        double *b2, double *U, int64_t q) {
   const int64_t node = (int64_t)blockIdx.x * kT + threadIdx.x;
   if (node >= g.G) return;
-  if (q == 0) return;
   const double *src_buf = q % 3 == 0 ? b0 : (q % 3 == 1 ? b1 : b2);
   const int i = (int)(node % g.X) + 1;
   const int j = (int)((node / g.X) % g.Y) + 1;
@@ -1788,7 +1787,9 @@ int launch_calc_epotential(picard_ctx *c, double maxerr, int32_t maxit, int64_t 
     PICARD_TRY(sweep(1, 1, batch < kMaxBatch ? batch : kMaxBatch, kNoLimit));
   }
   c->last_sweeps = fin.result;
-  k_jacobi_finish<<<nbn, kT, 0, c->stream>>>(g, c->jb[0], c->jb[1], c->jb[2], c->U, fin.result);
+  // without a sweep U stays as it came in; the split form's halo is the images all the same
+  if (fin.result > 0 || c->split)
+    k_jacobi_finish<<<nbn, kT, 0, c->stream>>>(g, c->jb[0], c->jb[1], c->jb[2], c->U, fin.result);
   PICARD_HIP(hipGetLastError());
   *sweeps = fin.result;
   // Running all 2*maxit+1 sweeps means every stop test failed; the reference

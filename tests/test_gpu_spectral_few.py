@@ -69,3 +69,17 @@ def test_caps_about_the_shortest_step(maxit, form):
     for _ in range(2):
         _compare(form, cfg, dom, C, _images(U, cfg.flow), 1e-8, maxit, fp32=maxit <= 32)
     dom.close()
+
+
+@pytest.mark.parametrize("form", list(FORMS))
+@pytest.mark.parametrize("flow", [(True, False, False), (False, False, False), (False, True, True)])
+def test_no_sweep_at_all(flow, form):
+    """Without charge the first test passes: the potential stays, and the split form's halo is its images."""
+    cfg, C, U = _setup((7, 5, 6), flow)
+    dom = host.Domain(cfg, max_particles=64, **FORMS[form])
+    for _ in range(2):
+        dom.set_field(_lib.FIELD_C, np.zeros_like(C))
+        dom.set_field(_lib.FIELD_U, U)
+        assert dom.calc_epotential(maxerr=1e-6, maxit=1000) == 0
+        assert np.array_equal(dom.field(_lib.FIELD_U), _images(U, flow) if form == "split" else U)
+    dom.close()
