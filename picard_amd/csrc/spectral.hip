@@ -195,13 +195,16 @@ __global__ void __launch_bounds__(kT) k_spec_residual(SpecGeo g, const double *_
 __device__ __forceinline__ void spec_finish(const JacobiState *js, SpecState *st, int64_t base, int margin,
                                             double clear, double above, double left) {
   const bool all = clear >= (double)((int64_t)js->maxit - 1 - base) && above > 1.02 * st->T;
-  const int64_t to = (all ? js->last : base + (int64_t)clear) - margin;
+  // of `left` sweeps that are expected after the last clear iterate, three are kept for the estimate
+  const int64_t on = all ? 1 : (int64_t)fmax(1.0, fmin(left, 1024.0));
+  const int64_t in = on > 3 ? (on - 3 < 3 ? on - 3 : 3) : 0;
+  const int64_t to = (all ? js->last : base + (int64_t)clear) - margin + in;
   if (to - base < kSpecFewest || to > 0x7fffff00) {
     st->skip = st->end > 4.0 * kSpecFewest ? kSpecUnclear : kSpecFew;
     return;
   }
   st->to = to;
-  st->ahead = margin + (int64_t)(all ? 1.0 : fmax(1.0, fmin(left, 1024.0)));
+  st->ahead = margin - in + on;
   st->steps = (double)(to - base);
 }
 
