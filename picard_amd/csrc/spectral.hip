@@ -27,8 +27,8 @@
 //
 // Cost: six axis transforms of 2 n operations a cell, whatever the number of
 // sweeps (about 3 n^2 to 1e-6).  Measured, whole solve with its last sweeps
-// against sweeping: 16^3 0.19 ms (FP32 sweeps 7.3), 64^3 0.37 ms (FP64 sweeps 280),
-// 128^3 to 1e-10 0.74 ms (FP32 sweeps 620), 160^3 1.1 ms (FP32 sweeps 880).
+// against sweeping: 16^3 0.19 ms (FP32 sweeps 7.3), 64^3 0.38 ms (FP64 sweeps 280),
+// 128^3 all open to 1e-10 0.60 ms (FP32 sweeps 620), 160^3 1.3 ms (FP32 sweeps 880), 256^3 4.3 ms (3900).
 // Against the FP64 form that sweeps all the way U differs by 2e-15 to 3e-13
 // (the FP32 sweeps differed by 5e-7 to 5e-6) and the sweep counts are equal.
 #include <algorithm>
@@ -349,7 +349,7 @@ struct SpecSeams {
 // The last block sums and decides.  NEAR, the second launch: the iterates that follow, one by one and signed
 // again, unless the first was sharp: 16 to 20 sweeps less for a solve to 1e-2 or 1e-3 (16^3 0.35 -> 0.26 ms,
 // 32^3 0.43 -> 0.29), where it is not needed one or two for 12 to 150 us.
-// Bound: the exponentials of every mode and iterate, 260 us at 160^3 with
+// Bound: the exponentials of every mode and iterate, 250 us at 160^3 with
 // two periodic axes (393 with the logarithm of the decayed modes too); on small grids the
 // chain of one column and the decision, 18 us at 16^3 (eight iterates a block and the decision in one
 // thread: 39).

@@ -172,7 +172,7 @@ constexpr double kFluxFixInv = 1.0 / 16777216.0;
 // A thread loads its chunk whole, 16 bytes at a time, so that a wave's loads cover one
 // contiguous stretch of each array: read a particle at a time, lanes 16 particles
 // apart, the kernel fetched 300 bytes a particle where 19 are needed (5.58 ms
-// at 1.4e8 particles; now 0.63, 4.2 TB/s).
+// at 1.4e8 particles; now 0.63, 4.0 TB/s).
 // Without the fluxes the adds are staged in LDS per block: the block's ROUNDS x 256 x
 // CHUNK sorted particles cover a short stretch of lower nodes from the first one's, b0, so
 // their corners fall in four node segments b0 + {0, X, XY, XY + X} + [0,
